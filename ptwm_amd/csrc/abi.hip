@@ -184,8 +184,9 @@ int64_t ilv_decode_payload(DevCtx& ctx, uint64_t in_dev, size_t in_len, uint64_t
   X.planes[0].len = in_len;
   X.planes[0].coded = 1;
   X.family = family;
-  X.crc_first = kIlvNoCrc;
-  int64_t rc = ilv_decode_tensors(ctx, std::vector<IlvTensor>{X});
+  X.crc_ix = kIlvNoCrc;
+  std::vector<uint32_t> sums, flagged;
+  int64_t rc = ilv_decode_tensors(ctx, std::vector<IlvTensor>{X}, 0, sums, flagged);
   if (rc != kOk) return rc;
   if (realign) {
     PTWM_HIP_TRY(hipMemcpyAsync(reinterpret_cast<void*>(out_dev), ctx.stage_out.ptr, expected,

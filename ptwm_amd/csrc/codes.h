@@ -48,4 +48,10 @@ enum ChainKind : uint32_t {
   kChainPassthrough = 6,
 };
 
+// Whether the chain's planes hold nibbles: its merge takes the low four bits
+// of every plane byte.
+constexpr bool chain_nibbles(uint32_t chain) {
+  return chain == kChainE4m3Nibble || chain == kChainE5m2Nibble || chain == kChainNibbleSplit;
+}
+
 }  // namespace ptwm

@@ -11,7 +11,6 @@ constexpr uint32_t kIlvLanes = 64;
 constexpr uint32_t kIlvGroup = 16;      // symbols per lane per round
 constexpr uint32_t kIlvRounds = kIlvBlock / (kIlvLanes * kIlvGroup);  // 16
 constexpr uint32_t kIlvBlocksPerTile = 4;   // blocks per tile (one per wavefront)
-constexpr uint32_t kIlvStageSpare = 96;     // spare LDS words after the staging area
 constexpr uint32_t kIlvMaxLds = 81920;      // LDS budget of one decode workgroup (2 per CU)
 constexpr uint32_t kMaxGridY = 65535;       // launches with one plane or job per gridDim.y slot are sliced
 
@@ -24,6 +23,10 @@ constexpr uint32_t kIlvErrLane = 4;     // a lane's word count disagrees with it
 // the stored nor the packed length) and the tensor is decoded again with a
 // slot for every plane.
 constexpr uint32_t kIlvRetrySlots = 16;
+// Not an input error either: a nibble chain's plane whose CRC is checked may
+// hold symbols above 15, which the merge masks but the CRC covers; the
+// tensor is decoded again through plane scratch.
+constexpr uint32_t kIlvRetryPlanes = 32;
 
 // Payload bytes read per native plane at a tensor's start (tag, n, weights
 // header: at most 135), kept in the staging area.
@@ -49,14 +52,14 @@ struct IlvTensor {
   uint32_t n_planes;
   IlvPlane planes[4];
   uint32_t family;  // IlvFamily
-  // huff_ilv family, chains with CRC-able planes (crc_chain_supported): the
-  // zero-init CRC-32 of every whole 16 KiB block of each plane, relative to
-  // the block's end, goes to crc_part[4 * (crc_first + block) + plane];
-  // kIlvNoCrc: none
-  uint32_t crc_first;
+  // the tensor's plane CRCs go to the accumulators crc_ix .. crc_ix +
+  // n_planes - 1 (kIlvNoCrc: none); crc_last: 16 KiB blocks of the planes
+  // after this tensor's block 0 (a chunk of a plane is a tensor of its own)
+  uint32_t crc_ix;
+  uint32_t crc_last;
+  uint32_t pad;
 };
 constexpr uint32_t kIlvNoCrc = 0xFFFFFFFFu;
-constexpr uint32_t kIlvCrcWords = 2048;  // LDS words of the fused CRC's tables (T0..T3, 1 KiB advance)
 
 struct IlvEncPlane {
   uint64_t src;        // plane bytes (16-byte aligned)
@@ -85,8 +88,8 @@ struct IlvPackJob {
 };
 
 // Launch chain code of the two-chain decode kernel: tensors of chains `a`
-// and `b` (huff_ilv family, no fused CRC) in one launch, e.g. MXFP4 weights
-// (nibble split) with their E8M0 scales (passthrough).
+// and `b` (huff_ilv family) in one launch, e.g. MXFP4 weights (nibble split)
+// with their E8M0 scales (passthrough).
 constexpr uint32_t ilv_chain_pair(uint32_t a, uint32_t b) { return 0x100u | a << 4 | b; }
 constexpr bool ilv_is_pair(uint32_t code) { return code >= 0x100u; }
 constexpr uint32_t ilv_pair_a(uint32_t code) { return (code >> 4) & 15u; }
@@ -113,18 +116,20 @@ struct IlvInline {
 // chain `chain`); tensor tix[j] owns the 4-block tiles tpre[j] ..
 // tpre[j+1] - 1 (or the same from `inl` when inl.m is nonzero).  grid:
 // persistent workgroups, each taking an equal range of tiles.  n_slots: LDS
-// table slots per workgroup (>= the coded planes of any tensor);
-// stage_words: LDS staging words per wavefront (multiple of 4); blocks
-// needing more are decoded from global memory.  status: one word per tensor
+// table slots a tensor may take; pool: LDS bytes (of kIlvPoolAlign) that a
+// tensor's table slots and, in what they leave, its blocks' staging share;
+// blocks that do not fit are decoded from global memory.  status: one word per tensor
 // index, zero before the launch, in host-coherent memory (the kernel ORs
-// its error bits in at system scope).  crc_tab: the CRC tables
-// (crc_device.h layout) when some tensor has crc_first set, else null; the
-// kernel then also writes the CRC block partials to crc_part.
+// its error bits in at system scope).  crc: the CRC arguments (crc_device.h)
+// when some tensor of the launch has crc_ix set, else null.
+struct CrcArgs;
+constexpr uint32_t kIlvPoolAlign = 128;  // the 64-entry tables that follow the pool are indexed by OR
 hipError_t launch_ilv_decode(uint32_t chain, const IlvTensor* tensors, const uint32_t* tix, const uint32_t* tpre,
                              uint32_t m, const IlvInline& inl, uint32_t grid, uint32_t* status, uint32_t n_slots,
-                             uint32_t stage_words, const uint32_t* crc_tab, uint32_t* crc_part, hipStream_t stream);
-size_t ilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc);
-hipError_t ilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc, int* wg_per_cu);
+                             uint32_t pool, const CrcArgs* crc, hipStream_t stream);
+uint32_t ilv_slot_bytes(uint32_t chain);
+size_t ilv_decode_lds_bytes(uint32_t chain, uint32_t pool, bool crc);
+hipError_t ilv_decode_occupancy(uint32_t chain, uint32_t pool, bool crc, int* wg_per_cu);
 hipError_t launch_ilv_pack(const IlvPackJob* jobs, uint32_t n_jobs, uint64_t max_n, hipStream_t stream);
 
 // Stored and Identity payload bodies: n plane bytes from src to dst + shift;

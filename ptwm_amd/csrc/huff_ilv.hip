@@ -33,7 +33,6 @@
 // from the code lengths), a host prefix sum for block offsets, and an encode
 // pass that writes each lane's words at its prefix-summed offset.
 #include "huff_ilv.h"
-#include "crc_device.h"
 #include "ilv_common.h"
 
 #include <cstring>
@@ -81,6 +80,7 @@ struct BuildScratch {
   uint32_t base[12];               // per length: first canonical index minus first code
   uint32_t lim[12];                // per length: end of the codes of length <= l, left-aligned to 11 bits
   uint32_t err, hdr_len, pair, max_bits;
+  uint32_t wide;  // the header lists symbols above 15
 };
 
 struct alignas(16) DecodeCtl {
@@ -96,9 +96,13 @@ struct alignas(16) DecodeCtl {
   uint64_t pbase[4], plen[4];  // the tensor's plane descriptors (IlvPlane)
   uint32_t pcoded[4];
   uint32_t bad;
-  uint32_t pad[3];
+  uint32_t flag;  // crc_finish
+  uint32_t used;  // table slots of the current tensor
+  uint32_t pad;
+  uint32_t sums[4];  // the workgroup's plane CRCs of the current tensor
 };
-static_assert(sizeof(DecodeCtl) % 16 == 0, "DecodeCtl keeps the staging area 16-byte aligned");
+static_assert(sizeof(DecodeCtl) % 16 == 0 && offsetof(DecodeCtl, t64) == 0 && kIlvPoolAlign == 2 * 64,
+              "DecodeCtl follows the pool: each 64-entry table on a boundary of its size");
 
 // Layout of a huff_ilv coded payload (tag 1): tag, n (4 bytes), the
 // weights header (0x80 | count, or 0x80 then count; then the 4-bit weights),
@@ -208,6 +212,7 @@ __device__ __forceinline__ void build_tables(uint16_t* tab, uint16_t* t64, bool 
     bs.max_bits = max_bits;
     bs.hdr_len = hb + (n + 1) / 2;
     bs.pair = pair_ok && n <= 16 && max_bits <= 6 ? 1u : 0u;
+    bs.wide = n > 16 ? 1u : 0u;
   }
   __syncthreads();
   err = bs.err;
@@ -470,6 +475,9 @@ __host__ __device__ constexpr uint32_t chain_slot_bytes(uint32_t chain) {
                                                                         : kIlvPairLutBytes;
 }
 
+// Whether a launch's CRCs take the nibble form (crc_round).
+__host__ __device__ constexpr bool ilv_crc_nib(uint32_t code) { return !ilv_is_pair(code) && chain_nibbles(code); }
+
 template <uint32_t C>
 struct ChainTag {
   static constexpr uint32_t value = C;
@@ -518,23 +526,26 @@ __device__ __forceinline__ void load_raw(const BlockState<ChainInfo<kChain>::np>
 // table lookups), merge and store.  luts: LDS address of the first table
 // slot; plane p uses the table at st.lut[p].  out: output tensor address.
 //
-// kCrc (crc_on uniform, whole blocks only): acc[p] becomes the zero-init
-// CRC-32 of the lane's 16 pieces of plane p (pieces 1 KiB apart), relative
-// to the end of its last piece: acc' = acc x^(8 * 1024) xor crc0(piece).
-// crc0 by slicing-by-4 (Kounavis & Berry) and the advance by four
-// byte-sliced lookups, from tables at LDS address 0 (crc_round_lds0); a
-// plane whose symbols are held rotated is rotated back first.
-template <uint32_t kChain, bool kTail, bool kStaged, bool kCrc = false, uint32_t kFix = 0>
+// kCrc: the planes' CRCs of the block go to crc->val (CrcLane), a group of
+// rounds at a time, or a round at a time where registers count more (kTail);
+// a plane whose symbols are held transformed is taken back first.  kNib:
+// crc_round's nibble form.  hi (nibble chains with kCrc): high nibbles seen
+// in stored planes.
+template <uint32_t kChain, bool kTail, bool kStaged, bool kCrc = false, uint32_t kFix = 0, bool kNib = false>
 __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& st, uint32_t luts, uint64_t out,
                                              uint64_t n, uint64_t bstart, uint32_t lane,
-                                             uint32_t* acc = nullptr) {
+                                             CrcLane* crc = nullptr, uint32_t* hi = nullptr) {
   constexpr uint32_t NP = ChainInfo<kChain>::np;
   constexpr uint32_t RATIO = ChainInfo<kChain>::ratio;
   static_assert(kFix == 0 || (!kTail && kStaged), "fixed plane forms: fast staged path only");
   const uint32_t coded_mask = kFix ? kFix - 1 : st.coded_mask;
   const uint32_t pair_mask = kFix ? 0u : st.pair_mask;
   const uint32_t packed_mask = kFix ? 0u : st.packed_mask;
-  static_assert(kIlvCrcWords == kCrcLdsWords, "LDS copy of the CRC tables");
+  static_assert(kIlvBlock == kCrcBlock, "the CRC's block weights");
+  constexpr bool kHigh = kCrc && chain_nibbles(kChain);
+  // a partial block's rounds end with the plane
+  const uint32_t rounds =
+      !kTail || n - bstart >= kIlvBlock ? kIlvRounds : (uint32_t)((n - bstart + 1023) / 1024);
   // the fixed-form fast path reads the coded planes' staged streams through
   // registers (elsewhere the readers' extra registers cost more occupancy
   // than the shorter lookup chain gains)
@@ -551,7 +562,8 @@ __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& 
 #pragma unroll
     for (uint32_t k = 0; k < RATIO; ++k) vmem_nop(out, k);
   }
-  for (uint32_t r = 0; r < kIlvRounds; ++r) {
+  f32x16 cm[kTail ? 1 : NP];
+  const auto round = [&](uint32_t r, uint32_t rr) {
     const uint64_t pos = bstart + (uint64_t)kIlvGroup * (r * 64u + lane);
     const uint32_t count = group_count<kTail>(pos, n);
     uint32_t v[NP][4];
@@ -591,6 +603,7 @@ __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& 
     for (uint32_t p = 0; p < NP; ++p) {
       if constexpr (kTail) {
         if (coded_mask & (1u << p)) continue;
+        if constexpr (kHigh) *hi |= (nxt[p][0] | nxt[p][1] | nxt[p][2] | nxt[p][3]) & 0xF0F0F0F0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[p][k] = xform_word(ChainInfo<kChain>::xf[p], nxt[p][k]);
       } else {
@@ -600,24 +613,19 @@ __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& 
         if (kFix && !raw) continue;
         uint32_t x[4];
         expand_group((packed_mask >> p) & 1u, nxt[p], x);
+        if constexpr (kHigh) *hi |= raw ? (x[0] | x[1] | x[2] | x[3]) & 0xF0F0F0F0u : 0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[p][k] = raw ? xform_word(ChainInfo<kChain>::xf[p], x[k]) : v[p][k];
       }
     }
     if constexpr (kTail) {
-      if (r + 1 < kIlvRounds) load_raw<kChain, kTail, kFix != 0>(st, coded_mask, packed_mask, pos + (uint64_t)kIlvGroup * 64u, n, nxt);
+      if (r + 1 < rounds) load_raw<kChain, kTail, kFix != 0>(st, coded_mask, packed_mask, pos + (uint64_t)kIlvGroup * 64u, n, nxt);
     } else {
       load_raw<kChain, kTail, kFix != 0>(st, coded_mask, packed_mask, pos + (uint64_t)kIlvGroup * 64u, n, nxt, r + 1 < kIlvRounds);
     }
-    if constexpr (kCrc) {
-#pragma unroll
-      for (uint32_t p = 0; p < NP; ++p) {
-        const uint32_t xf = ChainInfo<kChain>::xf[p];
-        acc[p] = crc_round_lds0(acc[p], u32x4_make(unxform_word(xf, v[p][0]), unxform_word(xf, v[p][1]),
-                                                   unxform_word(xf, v[p][2]), unxform_word(xf, v[p][3])));
-      }
-    }
-    if (kTail && count == 0) continue;
+    if constexpr (kCrc && kTail) crc_round_alone<kChain, kNib>(*crc, r, lane, v, count);
+    else if constexpr (kCrc) crc_round<kChain, kNib>(cm, *crc, rr, lane, v);
+    if (kTail && count == 0) return;
     uint32_t o[4 * RATIO];
     merge_group<kChain>(v, o);
     const uint64_t dst = out + RATIO * pos;
@@ -630,6 +638,19 @@ __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& 
     } else {
       for (uint32_t k = 0; k < RATIO * count; ++k) gstore_u8(dst + k, o[k >> 2] >> (8 * (k & 3)));
     }
+  };
+  if constexpr (kCrc && !kTail) {
+#pragma unroll 1
+    for (uint32_t g = 0; g < kIlvRounds / 4; ++g) {
+#pragma unroll
+      for (uint32_t p = 0; p < NP; ++p) cm[p] = crc_mma_open();
+#pragma unroll 1
+      for (uint32_t rr = 0; rr < 4; ++rr) round(4 * g + rr, rr);
+      crc_group_end<NP>(cm, *crc, 4 * g + 3, lane);
+    }
+  } else {
+#pragma unroll 1
+    for (uint32_t r = 0; r < rounds; ++r) round(r, 0);
   }
   if constexpr (kReg) {
 #pragma unroll
@@ -642,17 +663,17 @@ __device__ __forceinline__ void decode_block(BlockState<ChainInfo<kChain>::np>& 
 // entry, whose 4-block tiles are tpre[j] .. tpre[j+1] - 1 (m entries,
 // n_tiles = tpre[m]).  Workgroup g takes tiles [g n_tiles / G, (g+1) n_tiles / G).
 // Four wavefronts per SIMD (four workgroups per CU, the LDS budget of the
-// one- and two-coded-plane chains) need at most 128 VGPRs per lane; the
-// four-plane IEEE-32 chain runs at two workgroups per CU (256 VGPRs).  The
-// fused-CRC variants get no cap: held to 128 VGPRs they spill, and their
-// headline launch ran 7.98 ms against 7.2 ms uncapped.
+// one- and two-coded-plane chains) need at most 128 VGPRs per lane, with the
+// fused CRC's two accumulators too (8 registers spill, once per tile; at
+// three workgroups per CU four bf16 layers, 1.74 GB, took 805 us against
+// 750); the four-plane IEEE-32 chain runs at two workgroups per CU (256
+// VGPRs), with CRCs uncapped.
 template <uint32_t kChain, bool kCrc>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(kCrc ? 1 : kChain == kChainIeee32Split4 ? 2 : 4)))
+    __attribute__((amdgpu_waves_per_eu(kChain == kChainIeee32Split4 ? (kCrc ? 1 : 2) : 4)))
 ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, const uint32_t* __restrict__ tix_mem,
                   const uint32_t* __restrict__ tpre_mem, uint32_t m_mem, uint32_t* __restrict__ status,
-                  uint32_t n_slots, uint32_t stage_words, const uint32_t* __restrict__ crc_tab,
-                  uint32_t* __restrict__ crc_part) {
+                  uint32_t n_slots, uint32_t pool, CrcArgs crc_args) {
   // Descriptors from the kernel arguments or from device memory, both read
   // through constant-address-space pointers (uniform: scalar loads).  The
   // inline ones are read in place (the first argument: offset 0 of the
@@ -668,16 +689,21 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
   // The kernel has no static LDS, so the dynamic area starts at LDS address
   // 0 and every table sits on a SLOT boundary (entry address =
   // (window & mask) | table base).  Layout:
-  //   [kCrc: CRC tables, 8 KiB at address 0 (crc_round_lds0)]
-  //   [n_slots tables (coded planes from the last one down)][DecodeCtl]
-  //   [4 wavefronts x stage_words][96 spare words]
-  extern __shared__ __align__(16) uint8_t lds[];
-  uint8_t* const smem = lds + (kCrc ? 4u * kIlvCrcWords : 0u);
-  DecodeCtl& ctl = *reinterpret_cast<DecodeCtl*>(smem + n_slots * SLOT);
-  uint32_t* const stage = reinterpret_cast<uint32_t*>(smem + n_slots * SLOT + sizeof(DecodeCtl));
-  // while a tensor's tables are built, the staging area holds the payload
-  // heads (the host sizes it for NP x kIlvHeadWords words at least)
-  uint32_t (*const head)[kIlvHeadWords] = reinterpret_cast<uint32_t (*)[kIlvHeadWords]>(stage);
+  //   [the pool: the tensor's tables (coded planes from the last one down),
+  //    then the four wavefronts' staging]
+  //   [DecodeCtl][kCrc: the CRC's weights and constant operand]
+  // The tables and the staging share the pool because a launch holds tensors
+  // of both kinds: small ones with more coded planes (norm weights) and large
+  // ones with longer blocks; room for the larger of each would cost a
+  // workgroup per CU.  (A lane reads up to 90 words past its stream: inside
+  // the dynamic area, as DecodeCtl follows.)
+  extern __shared__ __align__(16) uint8_t smem[];
+  DecodeCtl& ctl = *reinterpret_cast<DecodeCtl*>(smem + pool);
+  static_assert(sizeof(DecodeCtl) >= 4 * 96, "reads past the staging stay in LDS");
+  // while a tensor's tables are built, the end of the pool holds the payload
+  // heads (the host sizes it for n_slots tables and them at least)
+  uint32_t (*const head)[kIlvHeadWords] =
+      reinterpret_cast<uint32_t (*)[kIlvHeadWords]>(smem + pool - 16u * kIlvHeadWords);
   const uint32_t luts = lds_addr(smem);
   BuildScratch& bs = ctl.bs;
   uint64_t* const s_table = ctl.table;
@@ -687,7 +713,10 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
   uint32_t* const s_coded = ctl.coded;
   uint32_t* const s_pair = ctl.pair;
   uint32_t& s_bad = ctl.bad;
-  const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63u;
+  // (uniform where registers are short; the MXFP4 launch is 0.5 us of 32
+  // slower with the block geometry on the scalar unit)
+  const uint32_t wave = kCrc ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+  uint32_t t = threadIdx.x, lane = t & 63u;
   if (luts & (SLOT - 1)) {
     // not reachable with the layout above; refuse rather than mis-decode
     if (t == 0 && blockIdx.x == 0) status_or(&status[tix[0]], kIlvErrHeader);
@@ -696,7 +725,6 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
   const uint32_t n_tiles = tpre[m];
   const uint32_t tile0 = (uint32_t)((uint64_t)blockIdx.x * n_tiles / gridDim.x);
   const uint32_t tile1 = (uint32_t)((uint64_t)(blockIdx.x + 1) * n_tiles / gridDim.x);
-  if (tile0 >= tile1) return;
   // entry holding tile0: the last j with tpre[j] <= tile0
   uint32_t lo = 0, hi = m;
   while (hi - lo > 1) {
@@ -705,25 +733,24 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
     else hi = mid;
   }
   uint32_t j = lo, cur = 0xFFFFFFFFu, bad = 0;
-  uint32_t* const sw = stage + wave * stage_words;
-  // CRC nibble tables N, NR, NA (visible after the first tile's barriers)
-  if constexpr (kCrc) {
-    // T0..T3 and the byte-sliced advance over 1 KiB
-    uint32_t* const crcT = reinterpret_cast<uint32_t*>(lds);
-    if (lds_addr(crcT) != 0) {  // not reachable: the kernel has no static LDS
-      if (t == 0 && blockIdx.x == 0) status_or(&status[tix[0]], kIlvErrHeader);
-      return;
-    }
-    for (uint32_t i = t; i < kIlvCrcWords; i += 256) crcT[i] = crc_tab[i < 1024 ? i : i - 1024 + kCrcTabS1024];
-  }
+  constexpr bool kNib = kCrc && ilv_crc_nib(kChain);
+  CrcLane cl;
+  CrcOpen co;
+  uint32_t crc_ix = kIlvNoCrc;  // the current tensor's accumulators
+  if constexpr (kCrc) co = crc_lane_open<kNib>(cl, crc_args.tab, lds_addr(smem) + pool + (uint32_t)sizeof(DecodeCtl));
   // At a tensor's first tile each wavefront requests its block's offsets
   // as soon as the payload heads are in LDS (while thread 0 parses them),
   // then its lane counts, and touches every 128-byte line of the block
   // before the tables are built (loads into one discarded register), so that
   // the copy into LDS after the build reads from the L2 cache: the parse and
   // the build hide the memory latency.
+  if constexpr (kCrc) crc_lane_ready<kNib>(cl, co, ctl.sums);
   for (uint32_t tile = tile0; tile < tile1; ++tile) {
     while (tile >= tpre[j + 1]) ++j;
+    // (opaque: addresses of every form of the decode that depend on the lane
+    // would otherwise be computed before the loop and held through it, which
+    // took the fused-CRC kernels past 128 VGPRs: 40 spilled, 148 bytes a lane)
+    asm volatile("" : "+v"(lane), "+v"(t));
     const uint32_t ti = tix[j];
     const KConst IlvTensor& T = inl_on ? inl.t[j] : *(const KConst IlvTensor*)(tensors + ti);
     // the tile, decoded by the code of its tensor's chain (a two-chain
@@ -842,7 +869,12 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
         if (bad && lane == 0) status_or(&status[cur], bad);
         bad = 0;
         cur = ti;
+        if constexpr (kCrc) crc_sum_up(cl, ctl.sums, lane);
         __syncthreads();  // every wavefront is done with the previous tables
+        if constexpr (kCrc) {
+          if (crc_ix != kIlvNoCrc) crc_sum_out(ctl.sums, crc_args.acc, crc_ix);
+          crc_ix = T.crc_ix;
+        }
         // the payload heads (tag, n, weights header) and last bytes, loaded
         // by all threads at once (coded payloads start 4-byte aligned)
         for (uint32_t k = t; k < NP * (kIlvHeadWords + 1); k += 256) {
@@ -930,6 +962,7 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
               s_bad |= kIlvRetrySlots;
             }
           }
+          ctl.used = k;
         }
         __syncthreads();
         // (the build's barriers do not wait for global loads)
@@ -946,6 +979,7 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
           if (t == 0) {
             s_pair[p] = bs.pair;
             if (bs.err) s_bad |= kIlvErrHeader;
+            if (kCrc && chain_nibbles(C) && T.crc_ix != kIlvNoCrc && bs.wide) s_bad |= kIlvRetryPlanes;
           }
           __syncthreads();
         }
@@ -977,10 +1011,15 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
       }
       const uint64_t out = T.out;
       uint32_t q0[NP];
-      const bool crc_on = kCrc && T.crc_first != kIlvNoCrc && bstart + kIlvBlock <= n;
-      uint32_t acc[NP];
-#pragma unroll
-      for (uint32_t p = 0; p < NP; ++p) acc[p] = 0;
+      uint32_t hi = 0;
+      if constexpr (kCrc) {
+        cl.val = 0;
+        cl.last = T.crc_last;
+      }
+      // the wavefront's staging: a quarter of what the tables leave
+      const uint32_t tables = st.coded_mask ? __builtin_amdgcn_readfirstlane(ctl.used) * SLOT : 0u;
+      const uint32_t stage_words = ((pool - tables) / 16u) & ~3u;
+      uint32_t* const sw = reinterpret_cast<uint32_t*>(smem + tables) + wave * stage_words;
       // skew uniform planes only when the staging budget has room for it
       if (need + need_skew > stage_words) uni_mask = 0;
       if (need <= stage_words) {
@@ -1046,16 +1085,11 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
         // the bf16 exponent-coded plane forms get a branch-free round body
         const bool fix = C == kChainIeee16Split2 && st.coded_mask == 2u && st.pair_mask == 0u &&
                          st.packed_mask == 0u;
-        if (full && crc_on) {
-          if (fix) decode_block<C, false, true, kCrc, 3>(st, luts, out, n, bstart, lane, acc);
-          else decode_block<C, false, true, kCrc>(st, luts, out, n, bstart, lane, acc);
-        } else if (full) {
-          if (fix) decode_block<C, false, true, false, 3>(st, luts, out, n, bstart, lane);
-          else decode_block<C, false, true, false>(st, luts, out, n, bstart, lane);
-        } else if (crc_on) {
-          decode_block<C, true, true, kCrc>(st, luts, out, n, bstart, lane, acc);
+        if (full) {
+          if (fix) decode_block<C, false, true, kCrc, 3, kNib>(st, luts, out, n, bstart, lane, &cl, &hi);
+          else decode_block<C, false, true, kCrc, 0, kNib>(st, luts, out, n, bstart, lane, &cl, &hi);
         } else {
-          decode_block<C, true, true, false>(st, luts, out, n, bstart, lane);
+          decode_block<C, true, true, kCrc, 0, kNib>(st, luts, out, n, bstart, lane, &cl, &hi);
         }
         __builtin_amdgcn_wave_barrier();
       } else {
@@ -1065,20 +1099,13 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
           st.nw[p] = lane_c[p];
           q0[p] = 0;
         }
-        if (crc_on) decode_block<C, true, false, kCrc>(st, luts, out, n, bstart, lane, acc);
-        else decode_block<C, true, false, false>(st, luts, out, n, bstart, lane);
+        decode_block<C, true, false, kCrc, 0, kNib>(st, luts, out, n, bstart, lane, &cl, &hi);
       }
       if constexpr (kCrc) {
-        if (crc_on) {
-          // lane l's last piece ends 16 (63 - l) bytes before the block's end
-          const uint32_t K = crc_tab[kCrcTabK64 + lane];
-#pragma unroll
-          for (uint32_t p = 0; p < NP; ++p) {
-            uint32_t a = gf2_mulmod_seq(acc[p], K);
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) a ^= __shfl_xor(a, d, 64);
-            if (lane == 0) g_st<uint32_t>(reinterpret_cast<uint64_t>(crc_part + 4ull * (T.crc_first + bi) + p), a);
-          }
+        // (a launch's tensors without plane CRCs compute and drop them)
+        if (T.crc_ix != kIlvNoCrc) {
+          crc_block_add(cl, bi, crc_args.tab, lane);
+          if (chain_nibbles(C) && hi) bad |= kIlvRetryPlanes;
         }
       }
       // acceptance: every lane's words hold exactly its codes
@@ -1098,6 +1125,14 @@ ilv_decode_kernel(IlvInline inl_arg, const IlvTensor* __restrict__ tensors, cons
   }
   bad = wave_or_status(bad);
   if (bad && lane == 0) status_or(&status[cur], bad);
+  if constexpr (kCrc) {
+    if (crc_ix != kIlvNoCrc) {
+      crc_sum_up(cl, ctl.sums, lane);
+      __syncthreads();
+      crc_sum_out(ctl.sums, crc_args.acc, crc_ix);
+    }
+    if (crc_args.n) crc_finish(crc_args, &ctl.flag);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1255,15 +1290,10 @@ __global__ void __launch_bounds__(64) ilv_encode_kernel(const IlvEncPlane* __res
   }
 }
 
-size_t ilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc) {
-  return (size_t)n_slots * chain_slot_bytes(chain) + sizeof(DecodeCtl) +
-         (4ull * stage_words + kIlvStageSpare + (crc ? kIlvCrcWords : 0u)) * 4ull;
-}
+uint32_t ilv_slot_bytes(uint32_t chain) { return chain_slot_bytes(chain); }
 
-// the fused plane CRC exists for the chains whose plane bytes are the
-// decoded symbols up to a byte rotation (crc_chain_supported)
-static bool ilv_crc_chain(uint32_t chain) {
-  return chain == kChainIeee16Split2 || chain == kChainIeee32Split4 || chain == kChainPassthrough;
+size_t ilv_decode_lds_bytes(uint32_t chain, uint32_t pool, bool crc) {
+  return (size_t)pool + sizeof(DecodeCtl) + (crc ? crc_lds_bytes(ilv_crc_nib(chain)) : 0u);
 }
 
 static const void* ilv_decode_fn(uint32_t chain, bool crc) {
@@ -1271,7 +1301,11 @@ static const void* ilv_decode_fn(uint32_t chain, bool crc) {
     switch (chain) {
       case kChainIeee16Split2: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainIeee16Split2, true>);
       case kChainIeee32Split4: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainIeee32Split4, true>);
+      case kChainE4m3Nibble: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainE4m3Nibble, true>);
+      case kChainE5m2Nibble: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainE5m2Nibble, true>);
+      case kChainNibbleSplit: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainNibbleSplit, true>);
       case kChainPassthrough: return reinterpret_cast<const void*>(&ilv_decode_kernel<kChainPassthrough, true>);
+      case kIlvPairNibblePass: return reinterpret_cast<const void*>(&ilv_decode_kernel<kIlvPairNibblePass, true>);
       default: return nullptr;
     }
   }
@@ -1287,26 +1321,26 @@ static const void* ilv_decode_fn(uint32_t chain, bool crc) {
   }
 }
 
-hipError_t ilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc, int* wg_per_cu) {
+hipError_t ilv_decode_occupancy(uint32_t chain, uint32_t pool, bool crc, int* wg_per_cu) {
   const void* fn = ilv_decode_fn(chain, crc);
   if (!fn) return hipErrorInvalidValue;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, fn, 256,
-                                                      ilv_decode_lds_bytes(chain, n_slots, stage_words, crc));
+                                                      ilv_decode_lds_bytes(chain, pool, crc));
 }
 
 hipError_t launch_ilv_decode(uint32_t chain, const IlvTensor* tensors, const uint32_t* tix, const uint32_t* tpre,
                              uint32_t m, const IlvInline& inl_in, uint32_t grid, uint32_t* status, uint32_t n_slots,
-                             uint32_t stage_words, const uint32_t* crc_tab, uint32_t* crc_part, hipStream_t stream) {
+                             uint32_t pool, const CrcArgs* crc_args, hipStream_t stream) {
   if (!grid || !(inl_in.m ? inl_in.m : m)) return hipSuccess;
   if (inl_in.m > kIlvInlineTensors) return hipErrorInvalidValue;
   IlvInline inl = inl_in;
-  if (stage_words % 4 != 0 || stage_words < 8) return hipErrorInvalidValue;
-  const bool crc = crc_tab != nullptr;
-  if (crc && (!crc_part || !ilv_crc_chain(chain))) return hipErrorInvalidValue;
-  const size_t lds = ilv_decode_lds_bytes(chain, n_slots, stage_words, crc);
+  if (pool % kIlvPoolAlign != 0 || pool < n_slots * chain_slot_bytes(chain) + 16u * kIlvHeadWords) return hipErrorInvalidValue;
+  const bool crc = crc_args != nullptr;
+  CrcArgs ca = crc ? *crc_args : CrcArgs{};
+  const size_t lds = ilv_decode_lds_bytes(chain, pool, crc);
   const void* fn = ilv_decode_fn(chain, crc);
   if (!fn) return hipErrorInvalidValue;
-  void* args[] = {&inl, &tensors, &tix, &tpre, &m, &status, &n_slots, &stage_words, &crc_tab, &crc_part};
+  void* args[] = {&inl, &tensors, &tix, &tpre, &m, &status, &n_slots, &pool, &ca};
   const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, lds, stream);
   return e != hipSuccess ? e : hipGetLastError();
 }

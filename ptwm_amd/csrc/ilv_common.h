@@ -4,6 +4,7 @@
 #pragma once
 
 #include "chain_ops.h"
+#include "crc_device.h"
 #include "huff_ilv.h"
 #include "ptwm_common.h"
 
@@ -97,16 +98,22 @@ __device__ __forceinline__ uint32_t xform_word(uint32_t x, uint32_t v) {
   }
 }
 
+// Plane symbols back from xform_word's output (symbols of a nibble chain are
+// below 16 there), for the fused decodes' plane CRCs.
+__device__ __forceinline__ uint32_t unxform_word(uint32_t x, uint32_t v) {
+  switch (x) {
+    case kXRot1: return ((v << 1) & 0xFEFEFEFEu) | ((v >> 7) & 0x01010101u);
+    case kXHi3: return v >> 3;
+    case kXE4m3Lo: return ((v >> 4) & 0x08080808u) | (v & 0x07070707u);
+    case kXE5m2Lo: return ((v & 0x04040404u) << 1) | ((v >> 5) & 0x04040404u) | (v & 0x03030303u);
+    case kXHi4: return v >> 4;
+    default: return v;
+  }
+}
+
 // Planes, output bytes per plane byte and the symbol transform of each plane
 // (applied by the decode table for coded planes, by xform_word for raw
 // ones) per chain.
-// Plane bytes back from xform_word's output, for the transforms of the
-// chains whose fused decode also computes plane CRCs (kXNone, kXRot1: the
-// inverse rotates each byte left by one).
-__device__ __forceinline__ uint32_t unxform_word(uint32_t x, uint32_t v) {
-  return x == kXRot1 ? ((v << 1) & 0xFEFEFEFEu) | ((v >> 7) & 0x01010101u) : v;
-}
-
 template <uint32_t kChain>
 struct ChainInfo;
 template <> struct ChainInfo<kChainIeee16Split2> {
@@ -178,6 +185,90 @@ __device__ __forceinline__ void merge_group(const uint32_t (&v)[ChainInfo<kChain
 #pragma unroll
     for (int k = 0; k < 4; ++k) o[k] = v[0][k] | v[1][k];
   }
+}
+
+// The data words of a lane's 16 symbols for the CRC: v[k] = plane p's
+// transformed bytes 4k..4k+3; with kNib two words of symbols to a word.
+template <bool kNib>
+constexpr uint32_t kCrcSteps = kNib ? 2 : 4;
+template <bool kNib>
+__device__ __forceinline__ uint32_t crc_data(uint32_t xf, const uint32_t (&v)[4], uint32_t k) {
+  return kNib ? unxform_word(xf, v[2 * k]) | (unxform_word(xf, v[2 * k + 1]) << 4) : unxform_word(xf, v[k]);
+}
+
+// Add round rr of the group (rounds 4 g .. 4 g + 3) to the planes' CRC
+// accumulators.
+template <uint32_t kChain, bool kNib>
+__device__ __forceinline__ void crc_round(f32x16 (&cm)[ChainInfo<kChain>::np], const CrcLane& cl, uint32_t rr,
+                                          uint32_t lane, const uint32_t (&v)[ChainInfo<kChain>::np][4]) {
+  const uint32_t at = cl.mma + 256u * kCrcSteps<kNib> * rr + 4u * lane;
+#pragma unroll
+  for (uint32_t k = 0; k < kCrcSteps<kNib>; ++k) {
+    const i32x8 b = crc_mma_const(lds_ld32(at + 256u * k));
+#pragma unroll
+    for (uint32_t p = 0; p < ChainInfo<kChain>::np; ++p)
+      crc_mma_word(cm[p], crc_data<kNib>(ChainInfo<kChain>::xf[p], v[p], k), b);
+  }
+}
+
+// The planes' CRCs up to the end of round r into lanes 4 r + p of cl.val.
+template <uint32_t NP>
+__device__ __forceinline__ void crc_group_end(const f32x16 (&cm)[NP], CrcLane& cl, uint32_t r, uint32_t lane) {
+  uint32_t x[NP];
+  crc_mma_close<NP>(cm, cl.row, lane, x);
+#pragma unroll
+  for (uint32_t p = 0; p < NP; ++p) cl.val = lane == 4 * r + p ? x[p] : cl.val;
+}
+
+// Round r by itself, a plane at a time: a sixteenth of the registers and four
+// times the reductions.  Bytes past `count` are not in the plane (the CRC
+// covers whole blocks, padded with zeros).
+template <uint32_t kChain, bool kNib>
+__device__ __forceinline__ void crc_round_alone(CrcLane& cl, uint32_t r, uint32_t lane,
+                                                const uint32_t (&v)[ChainInfo<kChain>::np][4], uint32_t count) {
+  const uint32_t at = cl.mma + 256u * kCrcSteps<kNib> * 3 + 4u * lane;
+#pragma unroll
+  for (uint32_t p = 0; p < ChainInfo<kChain>::np; ++p) {
+    uint32_t u[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+      u[k] = v[p][k] & (count >= 4 * k + 4 ? 0xFFFFFFFFu : count <= 4 * k ? 0u : (1u << (8 * (count - 4 * k))) - 1u);
+    f32x16 cm[1] = {crc_mma_open()};
+#pragma unroll
+    for (uint32_t k = 0; k < kCrcSteps<kNib>; ++k)
+      crc_mma_word(cm[0], crc_data<kNib>(ChainInfo<kChain>::xf[p], u, k), crc_mma_const(lds_ld32(at + 256u * k)));
+    uint32_t x[1];
+    crc_mma_close<1>(cm, cl.row, lane, x);
+    cl.val = lane == 4 * r + p ? x[0] : cl.val;
+  }
+}
+
+// The wavefront's CRC state at the start of a launch: the accumulator weights
+// and the constant operand go to LDS at address `at` (crc_lds_bytes).  Every
+// thread loads its two 16-byte pieces here and stores them later
+// (crc_lane_ready, before a barrier), while it looks for its tiles.
+struct CrcOpen {
+  u32x4 row, mma;
+};
+template <bool kNib>
+__device__ __forceinline__ CrcOpen crc_lane_open(CrcLane& cl, const uint32_t* tab, uint32_t at) {
+  static_assert(kCrcRowWords == 1024 && kCrcMmaWordsB == 1024, "a 16-byte piece per thread");
+  const uint32_t t = threadIdx.x;
+  cl.row = at;
+  cl.mma = at + 4u * kCrcRowWords;
+  cl.val = cl.sum = 0;
+  CrcOpen o;
+  o.row = g_ld<u32x4>(reinterpret_cast<uint64_t>(tab + kCrcTabRow) + 16u * t);
+  o.mma = g_ld<u32x4>(reinterpret_cast<uint64_t>(tab + (kNib ? kCrcTabMmaN : kCrcTabMmaB)) +
+                      16u * (kNib ? t & (kCrcMmaWordsN / 4 - 1) : t));
+  return o;
+}
+template <bool kNib>
+__device__ __forceinline__ void crc_lane_ready(const CrcLane& cl, const CrcOpen& o, uint32_t* sums) {
+  const uint32_t t = threadIdx.x;
+  *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(cl.row + 16u * t) = o.row;
+  if (!kNib || t < kCrcMmaWordsN / 4) *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(cl.mma + 16u * t) = o.mma;
+  if (t < 4) sums[t] = 0;
 }
 
 // Symbols of plane positions [pos, pos + 16) clipped to n.

@@ -53,7 +53,11 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
                            uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed);
 
 // Decode and merge the given tensors (fused path; each tensor's coded planes
-// are of its codec family).  Returns kOk or kInvalidInput.
-int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors, bool all_slots = false);
+// are of its codec family).  crc: the sums of the n_acc plane-CRC
+// accumulators that the tensors name (IlvTensor::crc_ix).  flagged: tensors
+// (indexes) whose planes have to be decoded through scratch for their CRCs
+// (kIlvRetryPlanes).  Returns kOk or kInvalidInput.
+int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors, uint32_t n_acc,
+                           std::vector<uint32_t>& crc, std::vector<uint32_t>& flagged, bool all_slots = false);
 
 }  // namespace ptwm

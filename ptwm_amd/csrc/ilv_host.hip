@@ -270,7 +270,8 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
   return (int64_t)total;
 }
 
-int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in, bool all_slots) {
+int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in, uint32_t n_acc,
+                           std::vector<uint32_t>& crc, std::vector<uint32_t>& flagged, bool all_slots) {
   hipStream_t s = ctx.stream;
   if (tensors_in.empty()) return kOk;
   std::vector<IlvTensor> tensors = tensors_in;
@@ -311,29 +312,29 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
   }
   // One persistent launch per chain present.  Per launch: the tensor list,
   // its 4-block tile prefix sums, the LDS table slots (most coded planes of
-  // any tensor) and the staging words per wavefront: the largest estimated
-  // block of any tensor (coded payload words per block, +2%, rounded up),
-  // capped by the workgroup LDS budget.  Blocks above it take the kernel's
-  // global-memory path.
+  // any tensor) and the room for blocks' streams: estimated block sizes
+  // (coded payload words per block, +2%, rounded up), capped by the workgroup
+  // LDS budget.  rans_ilv: staging words per wavefront, the largest of any
+  // tensor; huff_ilv: the pool's bytes, the most that any tensor's tables and
+  // staging take together.  Blocks above it take the kernel's global-memory
+  // path.
   struct Launch {
-    uint32_t family, chain, first, m, slots, stage_words, grid;
-    bool crc;  // some tensor of the launch has fused CRC partials (huff_ilv family)
+    uint32_t family, chain, first, m, slots, room, grid;
+    bool crc;  // some tensor of the launch has plane CRCs
   };
   std::vector<Launch> launches;
   // The launch chain codes of a family: one per chain present, except that
   // huff_ilv nibble-split and passthrough tensors (MXFP4 weights and their
-  // scales) share one two-chain launch when none of them has fused CRC
-  // partials (the two-chain kernel has no CRC variant).
+  // scales) share one two-chain launch.
   bool pair_ok = false;
   {
-    bool has5 = false, has6 = false, crc56 = false;
+    bool has5 = false, has6 = false;
     for (const IlvTensor& T : tensors) {
       if (T.family != kFamilyHuff || T.n == 0) continue;
       has5 |= T.chain == kChainNibbleSplit;
       has6 |= T.chain == kChainPassthrough;
-      crc56 |= (T.chain == kChainNibbleSplit || T.chain == kChainPassthrough) && T.crc_first != kIlvNoCrc;
     }
-    pair_ok = has5 && has6 && !crc56;
+    pair_ok = has5 && has6;
   }
   auto launch_codes = [&](uint32_t fam) {
     std::vector<uint32_t> codes{kChainIeee16Split2, kChainIeee32Split4, kChainE4m3Nibble, kChainE5m2Nibble};
@@ -367,15 +368,12 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
   for (uint32_t chain : launch_codes(fam)) {
     std::vector<uint32_t> tix, tpre{0};
     uint32_t slots = 0;
-    uint64_t est = 0;
-    bool crc = false;
+    uint64_t est = 0, pool = 0, pool_skew = 0;
+    bool with_crc = false;
     for (const uint32_t ti : order) {
       const IlvTensor& T = tensors[ti];
       if (T.family != fam || !ilv_code_has(chain, T.chain) || T.n == 0) continue;
-      if (T.crc_first != kIlvNoCrc) {
-        if (fam != kFamilyHuff) return kInternal;
-        crc = true;
-      }
+      with_crc |= T.crc_ix != kIlvNoCrc;
       const uint64_t nb = (T.n + kIlvBlock - 1) / kIlvBlock;
       // LDS table slots and staging for the planes that may be coded: a
       // native payload of the stored (n + 1) or packed (8 + ceil(n / 2))
@@ -383,49 +381,71 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
       // slot, and its tensor is decoded again with a slot for every plane
       // (kIlvRetrySlots); its blocks may take the kernel's global-memory path.
       uint32_t need_slots = 0;
-      uint64_t words = fam == kFamilyHuff ? 4 : 0;
+      // (skew: huff_ilv nibble chains may carry fixed-length codes, whose
+      // equal-length lane streams the kernel skews by up to two words a lane)
+      uint64_t words = fam == kFamilyHuff ? 4 : 0, skew = 0;
       for (uint32_t p = 0; p < T.n_planes; ++p) {
         const IlvPlane& P = T.planes[p];
         if (!P.coded) continue;
         if (!all_slots && (P.len == T.n + 1 || P.len == kPackedHeadBytes + (T.n + 1) / 2)) continue;
         ++need_slots;
         const uint64_t per_block = (T.planes[p].len + 4 * nb - 1) / (4 * nb);
-        // huff_ilv nibble chains may carry fixed-length codes: room for the
-        // kernel's per-lane skew of equal-length lane streams (two words per lane)
-        const uint64_t skew =
-            fam == kFamilyRans || T.chain == kChainIeee16Split2 || T.chain == kChainIeee32Split4 ? 0 : 128;
-        words += align_up(per_block + per_block / 50 + skew + 4, 4);
+        words += align_up(per_block + per_block / 50 + 4, 4);
+        skew += fam == kFamilyRans || T.chain == kChainIeee16Split2 || T.chain == kChainIeee32Split4 ? 0 : 128;
       }
       slots = std::max(slots, need_slots);
       est = std::max(est, words);
+      if (fam == kFamilyHuff) {
+        const uint64_t tables = (uint64_t)need_slots * ilv_slot_bytes(chain);
+        pool = std::max(pool, tables + 16 * words);
+        pool_skew = std::max(pool_skew, tables + 16 * (words + skew));
+      }
       tix.push_back(ti);
       tpre.push_back(tpre.back() + (uint32_t)((nb + kIlvBlocksPerTile - 1) / kIlvBlocksPerTile));
     }
     if (tix.empty()) continue;
-    const uint64_t max_lds = fam == kFamilyHuff ? kIlvMaxLds : kRilvMaxLds;
-    const uint64_t fixed =
-        fam == kFamilyHuff ? ilv_decode_lds_bytes(chain, slots, 0, crc) : rilv_decode_lds_bytes(chain, slots, 0);
-    uint64_t cap_words = ((max_lds - std::min<uint64_t>(fixed, max_lds)) / 16) & ~3ull;
-    // the staging area also holds the payload heads at a tensor's start
-    const uint64_t head_min = fam == kFamilyHuff ? kIlvHeadWords : kRilvHeadWords;  // 4 planes over 4 wavefronts
-    uint64_t stage = align_up(std::max<uint64_t>(std::max<uint64_t>(est, 8), head_min), 4);
-    if (stage > cap_words) stage = cap_words;
-    if (stage < head_min) return kInternal;
+    // workgroups per CU with `room` (Launch::room) for the blocks
+    const auto occupancy = [&](uint64_t room, int& per_cu) -> int64_t {
+      const uint64_t key =
+          (uint64_t)chain | ((uint64_t)slots << 12) | (room << 20) | ((uint64_t)with_crc << 61) | ((uint64_t)fam << 62);
+      auto it = ctx.ilv_occupancy.find(key);
+      if (it != ctx.ilv_occupancy.end()) {
+        per_cu = it->second;
+        return kOk;
+      }
+      if (fam == kFamilyHuff) PTWM_HIP_TRY(ilv_decode_occupancy(chain, (uint32_t)room, with_crc, &per_cu));
+      else PTWM_HIP_TRY(rilv_decode_occupancy(chain, slots, (uint32_t)room, with_crc, &per_cu));
+      ctx.ilv_occupancy[key] = per_cu;
+      return kOk;
+    };
     int per_cu = 0;
-    const uint64_t occ_key =
-        (uint64_t)chain | ((uint64_t)slots << 12) | (stage << 20) | ((uint64_t)crc << 61) | ((uint64_t)fam << 62);
-    auto it = ctx.ilv_occupancy.find(occ_key);
-    if (it != ctx.ilv_occupancy.end()) {
-      per_cu = it->second;
+    uint64_t room = 0;
+    // The LDS budgets hold without what plane CRCs take on top (blocks that
+    // are not staged decode from global memory, several times slower).  The
+    // room also holds the payload heads at a tensor's start.
+    if (fam == kFamilyHuff) {
+      const uint64_t least = (uint64_t)slots * ilv_slot_bytes(chain) + 16 * kIlvHeadWords;
+      const uint64_t most = (kIlvMaxLds - ilv_decode_lds_bytes(chain, 0, false)) / kIlvPoolAlign * kIlvPoolAlign;
+      if (least > most) return kInternal;
+      room = std::min(align_up(std::max(pool, least), kIlvPoolAlign), most);
+      if (int64_t rc = occupancy(room, per_cu); rc != kOk) return rc;
+      // room for the skew where it does not cost a workgroup per CU
+      const uint64_t with_skew = std::min(align_up(std::max(pool_skew, least), kIlvPoolAlign), most);
+      int n = 0;
+      if (with_skew != room)
+        if (int64_t rc = occupancy(with_skew, n); rc != kOk) return rc;
+      if (n >= per_cu) room = with_skew;
     } else {
-      if (fam == kFamilyHuff) PTWM_HIP_TRY(ilv_decode_occupancy(chain, slots, (uint32_t)stage, crc, &per_cu));
-      else PTWM_HIP_TRY(rilv_decode_occupancy(chain, slots, (uint32_t)stage, &per_cu));
-      ctx.ilv_occupancy[occ_key] = per_cu;
+      const uint64_t fixed = rilv_decode_lds_bytes(chain, slots, 0, false);
+      const uint64_t cap_words = ((kRilvMaxLds - std::min<uint64_t>(fixed, kRilvMaxLds)) / 16) & ~3ull;
+      room = std::min(align_up(std::max<uint64_t>({est, 8, kRilvHeadWords}), 4), cap_words);
+      if (room < kRilvHeadWords) return kInternal;
+      if (int64_t rc = occupancy(room, per_cu); rc != kOk) return rc;
     }
     if (per_cu < 1) per_cu = 1;
     const uint64_t n_tiles = tpre.back();
     const uint32_t grid = (uint32_t)std::min<uint64_t>(n_tiles, (uint64_t)per_cu * ctx.cu_count);
-    launches.push_back(Launch{fam, chain, (uint32_t)idx.size(), (uint32_t)tix.size(), slots, (uint32_t)stage, grid, crc});
+    launches.push_back(Launch{fam, chain, (uint32_t)idx.size(), (uint32_t)tix.size(), slots, (uint32_t)room, grid, with_crc});
     idx.insert(idx.end(), tpre.begin(), tpre.end());
     idx.insert(idx.end(), tix.begin(), tix.end());
   }
@@ -456,11 +476,18 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
     PTWM_HIP_TRY(ctx.ensure_events());
     PTWM_HIP_TRY(hipEventRecord(ctx.ev[3], s));
   }
-  const uint32_t* crc_tab = nullptr;
-  for (const Launch& L : launches)
-    if (L.crc && !crc_tab)
-      if (int64_t rc = crc_tables(ctx, &crc_tab); rc != kOk) return rc;
-  for (const Launch& L : launches) {
+  // the call's last launch with plane CRCs hands their sums over
+  CrcArgs crc_args{};
+  size_t last_crc = launches.size();
+  for (size_t i = 0; i < launches.size(); ++i)
+    if (launches[i].crc) last_crc = i;
+  if (last_crc < launches.size())
+    if (int64_t rc = crc_begin(ctx, n_acc, crc_args); rc != kOk) return rc;
+  for (size_t li = 0; li < launches.size(); ++li) {
+    const Launch& L = launches[li];
+    CrcArgs ca = crc_args;
+    if (li != last_crc) ca.n = 0;
+    const CrcArgs* const cp = L.crc ? &ca : nullptr;
     const uint32_t* hidx = idx.data() + L.first;  // [m + 1 prefix][m tensor indexes]
     if (inline_ok(L)) {
       IlvInline inl{};
@@ -471,19 +498,17 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
         inl.t[j] = tensors[inl.tix[j]];
       }
       PTWM_HIP_TRY(launch_ilv_decode(L.chain, nullptr, nullptr, nullptr, 0, inl, L.grid, hs, L.slots,
-                                     L.stage_words, L.crc ? crc_tab : nullptr,
-                                     static_cast<uint32_t*>(ctx.crc_part.ptr), s));
+                                     L.room, cp, s));
       continue;
     }
     const uint32_t* base = reinterpret_cast<const uint32_t*>(d + off_idx) + L.first;
     const IlvTensor* td = reinterpret_cast<const IlvTensor*>(d);
     if (L.family == kFamilyHuff)
       PTWM_HIP_TRY(launch_ilv_decode(L.chain, td, base + L.m + 1, base, L.m, IlvInline{}, L.grid, hs, L.slots,
-                                     L.stage_words, L.crc ? crc_tab : nullptr,
-                                     static_cast<uint32_t*>(ctx.crc_part.ptr), s));
+                                     L.room, cp, s));
     else
       PTWM_HIP_TRY(launch_rilv_decode(L.chain, td, base + L.m + 1, base, L.m, L.grid, hs, L.slots,
-                                      L.stage_words, s));
+                                      L.room, cp, s));
   }
   if (ctx.profile) PTWM_HIP_TRY(hipEventRecord(ctx.ev[2], s));
   PTWM_HIP_TRY(hipStreamSynchronize(s));
@@ -493,15 +518,35 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
     ctx.last_ms[0] += ms;
     ctx.last_ms[2] += ms;
   }
-  std::vector<IlvTensor> again;
+  if (last_crc < launches.size())
+    if (int64_t rc = crc_take(ctx, crc_args, crc); rc != kOk) return rc;
+  std::vector<char> retry(nt, 0);
+  bool any_retry = false;
   for (size_t i = 0; i < nt; ++i) {
-    if (hs[i] & ~kIlvRetrySlots) return kInvalidInput;
-    if (hs[i]) again.push_back(tensors[i]);
+    if (hs[i] & ~(kIlvRetrySlots | kIlvRetryPlanes)) return kInvalidInput;
+    if (hs[i] & kIlvRetryPlanes) flagged.push_back((uint32_t)i);
+    else if (hs[i]) any_retry = retry[i] = 1;
   }
-  if (!again.empty()) {
-    if (all_slots) return kInternal;
-    return ilv_decode_tensors(ctx, again, true);
-  }
+  if (!any_retry) return kOk;
+  if (all_slots) return kInternal;
+  // a tensor without its sums again, and with it the chunks that share them
+  for (size_t i = 0; i < nt; ++i)
+    if (retry[i] && tensors[i].crc_ix != kIlvNoCrc)
+      for (size_t k = 0; k < nt; ++k)
+        if (tensors[k].crc_ix == tensors[i].crc_ix) retry[k] = 1;
+  std::vector<IlvTensor> again;
+  std::vector<uint32_t> again_ix;
+  for (size_t i = 0; i < nt; ++i)
+    if (retry[i]) {
+      again.push_back(tensors[i]);
+      again_ix.push_back((uint32_t)i);
+    }
+  std::vector<uint32_t> sums, flags;
+  if (int64_t rc = ilv_decode_tensors(ctx, again, n_acc, sums, flags, true); rc != kOk) return rc;
+  for (const uint32_t f : flags) flagged.push_back(again_ix[f]);
+  for (const IlvTensor& T : again)
+    if (T.crc_ix != kIlvNoCrc)
+      for (uint32_t p = 0; p < T.n_planes; ++p) crc[T.crc_ix + p] = sums[T.crc_ix + p];
   return kOk;
 }
 

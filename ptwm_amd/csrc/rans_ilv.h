@@ -34,9 +34,9 @@ struct RilvEncBlock {
 // memory.
 hipError_t launch_rilv_decode(uint32_t chain, const IlvTensor* tensors, const uint32_t* tix, const uint32_t* tpre,
                               uint32_t m, uint32_t grid, uint32_t* status, uint32_t n_slots, uint32_t stage_words,
-                              hipStream_t stream);
-size_t rilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words);
-hipError_t rilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, int* wg_per_cu);
+                              const CrcArgs* crc, hipStream_t stream);
+size_t rilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc);
+hipError_t rilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc, int* wg_per_cu);
 
 // Encoder passes over blocks: word counts (block_words[i]), then the blocks.
 hipError_t launch_rilv_size(const IlvEncPlane* planes, const RilvEncBlock* blocks, uint32_t n_blocks,

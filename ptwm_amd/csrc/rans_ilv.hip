@@ -50,7 +50,9 @@ struct alignas(16) RilvCtl {
   uint32_t bad;
   uint32_t wsum[4];     // table build scratch: per-wavefront frequency sums
   uint32_t last[4];     // last byte of each native payload
-  uint32_t pad[3];
+  uint32_t flag;        // crc_finish
+  uint32_t pad[2];
+  uint32_t sums[4];     // the workgroup's plane CRCs of the current tensor
   uint16_t cum[264];    // table build scratch: cumulative frequencies
   uint16_t f[256];
 };
@@ -100,9 +102,12 @@ struct RilvBlock {
   uint32_t packed_mask;
 };
 
-template <uint32_t kChain, bool kTail, bool kStaged>
+// kCrc, crc, hi: as decode_block of huff_ilv.hip.
+template <uint32_t kChain, bool kTail, bool kStaged, bool kCrc = false>
 __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, uint64_t out, uint64_t n,
-                                                  uint64_t bstart, uint32_t lane) {
+                                                  uint64_t bstart, uint32_t lane, CrcLane* crc = nullptr,
+                                                  uint32_t* hi = nullptr) {
+  constexpr bool kNib = chain_nibbles(kChain);
   constexpr uint32_t NP = ChainInfo<kChain>::np;
   constexpr uint32_t RATIO = ChainInfo<kChain>::ratio;
   // full blocks: the raw planes' next group is loaded a round ahead, one
@@ -117,7 +122,11 @@ __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, 
 #pragma unroll
     for (uint32_t k = 0; k < RATIO; ++k) vmem_nop(out, k);
   }
-  for (uint32_t r = 0; r < kIlvRounds; ++r) {
+  // a partial block's rounds end with the plane
+  const uint32_t rounds =
+      !kTail || n - bstart >= kIlvBlock ? kIlvRounds : (uint32_t)((n - bstart + 1023) / 1024);
+  f32x16 cm[kTail ? 1 : NP];
+  const auto round = [&](uint32_t r, uint32_t rr) {
     const uint64_t pos = bstart + (uint64_t)kIlvGroup * (r * 64u + lane);
     const uint32_t count = group_count<kTail>(pos, n);
     uint32_t v[NP][4];
@@ -128,6 +137,7 @@ __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, 
         if (st.coded_mask & (1u << p)) continue;
         // stored plane: the group's 16 bytes (or 8 bytes of packed nibbles)
         load_group(st.raw[p], (st.packed_mask >> p) & 1u, pos, count, v[p]);
+        if constexpr (kCrc && kNib) *hi |= (v[p][0] | v[p][1] | v[p][2] | v[p][3]) & 0xF0F0F0F0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[p][k] = xform_word(ChainInfo<kChain>::xf[p], v[p][k]);
       } else {
@@ -135,6 +145,7 @@ __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, 
         uint32_t x[4];
         expand_group((st.packed_mask >> p) & 1u, nxt[p], x);
         const bool raw = !(st.coded_mask & (1u << p));
+        if constexpr (kCrc && kNib) *hi |= raw ? (x[0] | x[1] | x[2] | x[3]) & 0xF0F0F0F0u : 0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[p][k] = raw ? xform_word(ChainInfo<kChain>::xf[p], x[k]) : 0u;
       }
@@ -156,7 +167,9 @@ __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, 
         v[p][t >> 2] |= sym << (8 * (t & 3));
       }
     }
-    if (kTail && count == 0) continue;
+    if constexpr (kCrc && kTail) crc_round_alone<kChain, kNib>(*crc, r, lane, v, count);
+    else if constexpr (kCrc) crc_round<kChain, kNib>(cm, *crc, rr, lane, v);
+    if (kTail && count == 0) return;
     uint32_t o[4 * RATIO];
     merge_group<kChain>(v, o);
     const uint64_t dst = out + RATIO * pos;
@@ -169,6 +182,19 @@ __device__ __forceinline__ void rilv_decode_block(RilvBlock& st, uint32_t luts, 
     } else {
       for (uint32_t k = 0; k < RATIO * count; ++k) gstore_u8(dst + k, o[k >> 2] >> (8 * (k & 3)));
     }
+  };
+  if constexpr (kCrc && !kTail) {
+#pragma unroll 1
+    for (uint32_t g = 0; g < kIlvRounds / 4; ++g) {
+#pragma unroll
+      for (uint32_t p = 0; p < NP; ++p) cm[p] = crc_mma_open();
+#pragma unroll 1
+      for (uint32_t rr = 0; rr < 4; ++rr) round(4 * g + rr, rr);
+      crc_group_end<NP>(cm, *crc, 4 * g + 3, lane);
+    }
+  } else {
+#pragma unroll 1
+    for (uint32_t r = 0; r < rounds; ++r) round(r, 0);
   }
 }
 
@@ -188,26 +214,33 @@ __device__ __forceinline__ void rilv_build_table(uint32_t* tab, const RilvCtl& c
   }
 }
 
-template <uint32_t kChain>
+template <uint32_t kChain, bool kCrc>
 __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __restrict__ tensors,
                                                           const uint32_t* __restrict__ tix,
                                                           const uint32_t* __restrict__ tpre, uint32_t m,
                                                           uint32_t* __restrict__ status, uint32_t n_slots,
-                                                          uint32_t stage_words) {
+                                                          uint32_t stage_words, CrcArgs crc_args) {
   constexpr uint32_t NP = ChainInfo<kChain>::np;
-  // LDS: [n_slots tables (coded planes from the last one down)][RilvCtl][4 x stage_words]
-  extern __shared__ __align__(16) uint8_t smem[];
+  // LDS: [kCrc: the CRC's weights and constant operand][n_slots tables (coded
+  // planes from the last one down)][RilvCtl][4 x stage_words]
+  extern __shared__ __align__(16) uint8_t lds_mem[];
+  uint8_t* const smem = lds_mem + (kCrc ? crc_lds_bytes(chain_nibbles(kChain)) : 0u);
+  constexpr bool kNib = chain_nibbles(kChain);
+  CrcLane cl;
+  CrcOpen co;
+  uint32_t crc_ix = kIlvNoCrc;  // the current tensor's accumulators
+  if constexpr (kCrc) co = crc_lane_open<kNib>(cl, crc_args.tab, lds_addr(lds_mem));
   RilvCtl& ctl = *reinterpret_cast<RilvCtl*>(smem + n_slots * kRilvTableBytes);
   uint32_t* const stage = reinterpret_cast<uint32_t*>(smem + n_slots * kRilvTableBytes + sizeof(RilvCtl));
   // while a tensor's tables are built, the staging area holds the payload
   // heads (the host sizes it for NP x kRilvHeadWords words at least)
   uint32_t (*const head)[kRilvHeadWords] = reinterpret_cast<uint32_t (*)[kRilvHeadWords]>(stage);
   const uint32_t luts = lds_addr(smem);
-  const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t t = threadIdx.x, lane = t & 63u;
   const uint32_t n_tiles = tpre[m];
   const uint32_t tile0 = (uint32_t)((uint64_t)blockIdx.x * n_tiles / gridDim.x);
   const uint32_t tile1 = (uint32_t)((uint64_t)(blockIdx.x + 1) * n_tiles / gridDim.x);
-  if (tile0 >= tile1) return;
   uint32_t lo = 0, hi = m;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) / 2;
@@ -216,8 +249,10 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
   }
   uint32_t j = lo, cur = 0xFFFFFFFFu, bad = 0;
   uint32_t* const sw = stage + wave * stage_words;
+  if constexpr (kCrc) crc_lane_ready<kNib>(cl, co, ctl.sums);
   for (uint32_t tile = tile0; tile < tile1; ++tile) {
     while (tile >= tpre[j + 1]) ++j;
+    asm volatile("" : "+v"(lane), "+v"(t));  // as in ilv_decode_kernel
     const uint32_t ti = tix[j];
     const IlvTensor& T = tensors[ti];
     const uint64_t n = T.n;
@@ -228,7 +263,12 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
       if (bad && lane == 0) status_or(&status[cur], bad);
       bad = 0;
       cur = ti;
+      if constexpr (kCrc) crc_sum_up(cl, ctl.sums, lane);
       __syncthreads();
+      if constexpr (kCrc) {
+        if (crc_ix != kIlvNoCrc) crc_sum_out(ctl.sums, crc_args.acc, crc_ix);
+        crc_ix = T.crc_ix;
+      }
       // the payload heads and last bytes, loaded by all threads at once
       // (native payloads start 4-byte aligned)
       for (uint32_t k = t; k < NP * (kRilvHeadWords + 1); k += 256) {
@@ -306,6 +346,7 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
           ctl.cum[256] = 2048;
           const uint32_t total = ctl.wsum[0] + ctl.wsum[1] + ctl.wsum[2] + ctl.wsum[3];
           bool ok = hok && total == 2048u;
+          if (kCrc && chain_nibbles(kChain) && T.crc_ix != kIlvNoCrc && ms > 15) ctl.bad |= kIlvRetryPlanes;
           const uint64_t head = (hl + 3) & ~3ull;
           const uint64_t data0 = head + 4ull * (nb + 1);
           ok = ok && data0 <= P.len;
@@ -382,6 +423,11 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
       if (!(st.coded_mask & (1u << p)) && !raw_aligned(st.raw[p], packed)) full = false;
     }
     const uint64_t out = T.out;
+    uint32_t high = 0;
+    if constexpr (kCrc) {
+      cl.val = 0;
+      cl.last = T.crc_last;
+    }
     if (need <= stage_words) {
       // coalesced copy of each coded plane's words into this wavefront's LDS
       __builtin_amdgcn_wave_barrier();
@@ -397,11 +443,17 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (full) rilv_decode_block<kChain, false, true>(st, luts, out, n, bstart, lane);
-      else rilv_decode_block<kChain, true, true>(st, luts, out, n, bstart, lane);
+      if (full) rilv_decode_block<kChain, false, true, kCrc>(st, luts, out, n, bstart, lane, &cl, &high);
+      else rilv_decode_block<kChain, true, true, kCrc>(st, luts, out, n, bstart, lane, &cl, &high);
       __builtin_amdgcn_wave_barrier();
     } else {
-      rilv_decode_block<kChain, true, false>(st, luts, out, n, bstart, lane);
+      rilv_decode_block<kChain, true, false, kCrc>(st, luts, out, n, bstart, lane, &cl, &high);
+    }
+    if constexpr (kCrc) {
+      if (T.crc_ix != kIlvNoCrc) {  // (a launch's other tensors compute and drop them)
+        crc_block_add(cl, bi, crc_args.tab, lane);
+        if (chain_nibbles(kChain) && high) bad |= kIlvRetryPlanes;
+      }
     }
     // acceptance: every word taken, every lane back at 2^16
 #pragma unroll
@@ -412,6 +464,14 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
   }
   bad = wave_or_status(bad);
   if (bad && lane == 0) status_or(&status[cur], bad);
+  if constexpr (kCrc) {
+    if (crc_ix != kIlvNoCrc) {
+      crc_sum_up(cl, ctl.sums, lane);
+      __syncthreads();
+      crc_sum_out(ctl.sums, crc_args.acc, crc_ix);
+    }
+    if (crc_args.n) crc_finish(crc_args, &ctl.flag);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -553,43 +613,12 @@ __global__ void __launch_bounds__(64) rilv_encode_kernel(const IlvEncPlane* __re
 // launchers
 // ---------------------------------------------------------------------------
 
-static const void* rilv_decode_fn(uint32_t chain) {
+static const void* rilv_decode_fn(uint32_t chain, bool crc) {
   switch (chain) {
-    case kChainIeee16Split2: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainIeee16Split2>);
-    case kChainIeee32Split4: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainIeee32Split4>);
-    case kChainE4m3Nibble: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainE4m3Nibble>);
-    case kChainE5m2Nibble: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainE5m2Nibble>);
-    case kChainNibbleSplit: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainNibbleSplit>);
-    case kChainPassthrough: return reinterpret_cast<const void*>(&rilv_decode_kernel<kChainPassthrough>);
-    default: return nullptr;
-  }
-}
-
-size_t rilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words) {
-  (void)chain;
-  return (size_t)n_slots * kRilvTableBytes + sizeof(RilvCtl) + 4ull * stage_words * 4ull;
-}
-
-hipError_t rilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, int* wg_per_cu) {
-  const void* fn = rilv_decode_fn(chain);
-  if (!fn) return hipErrorInvalidValue;
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, fn, 256,
-                                                      rilv_decode_lds_bytes(chain, n_slots, stage_words));
-}
-
-hipError_t launch_rilv_decode(uint32_t chain, const IlvTensor* tensors, const uint32_t* tix, const uint32_t* tpre,
-                              uint32_t m, uint32_t grid, uint32_t* status, uint32_t n_slots, uint32_t stage_words,
-                              hipStream_t stream) {
-  if (m == 0 || grid == 0) return hipSuccess;
-  if (stage_words % 4 != 0 || n_slots > 4) return hipErrorInvalidValue;
-  const size_t lds = rilv_decode_lds_bytes(chain, n_slots, stage_words);
-  if (lds > kRilvMaxLds) return hipErrorInvalidValue;
-  switch (chain) {
-#define PTWM_RILV_CASE(C)                                                                                      \
-  case C:                                                                                                      \
-    hipLaunchKernelGGL(rilv_decode_kernel<C>, dim3(grid), dim3(256), lds, stream, tensors, tix, tpre, m, status, \
-                       n_slots, stage_words);                                                                  \
-    break;
+#define PTWM_RILV_CASE(C) \
+  case C:                 \
+    return crc ? reinterpret_cast<const void*>(&rilv_decode_kernel<C, true>) \
+               : reinterpret_cast<const void*>(&rilv_decode_kernel<C, false>);
     PTWM_RILV_CASE(kChainIeee16Split2)
     PTWM_RILV_CASE(kChainIeee32Split4)
     PTWM_RILV_CASE(kChainE4m3Nibble)
@@ -597,10 +626,35 @@ hipError_t launch_rilv_decode(uint32_t chain, const IlvTensor* tensors, const ui
     PTWM_RILV_CASE(kChainNibbleSplit)
     PTWM_RILV_CASE(kChainPassthrough)
 #undef PTWM_RILV_CASE
-    default:
-      return hipErrorInvalidValue;
+    default: return nullptr;
   }
-  return hipGetLastError();
+}
+
+size_t rilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc) {
+  return (size_t)n_slots * kRilvTableBytes + sizeof(RilvCtl) + 4ull * stage_words * 4ull +
+         (crc ? crc_lds_bytes(chain_nibbles(chain)) : 0u);
+}
+
+hipError_t rilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc, int* wg_per_cu) {
+  const void* fn = rilv_decode_fn(chain, crc);
+  if (!fn) return hipErrorInvalidValue;
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(wg_per_cu, fn, 256,
+                                                      rilv_decode_lds_bytes(chain, n_slots, stage_words, crc));
+}
+
+hipError_t launch_rilv_decode(uint32_t chain, const IlvTensor* tensors, const uint32_t* tix, const uint32_t* tpre,
+                              uint32_t m, uint32_t grid, uint32_t* status, uint32_t n_slots, uint32_t stage_words,
+                              const CrcArgs* crc_args, hipStream_t stream) {
+  if (m == 0 || grid == 0) return hipSuccess;
+  if (stage_words % 4 != 0 || n_slots > 4) return hipErrorInvalidValue;
+  const bool crc = crc_args != nullptr;
+  CrcArgs ca = crc ? *crc_args : CrcArgs{};
+  const size_t lds = rilv_decode_lds_bytes(chain, n_slots, stage_words, crc);
+  const void* fn = rilv_decode_fn(chain, crc);
+  if (lds > kRilvMaxLds + (crc ? crc_lds_bytes(chain_nibbles(chain)) : 0u) || !fn) return hipErrorInvalidValue;
+  void* args[] = {&tensors, &tix, &tpre, &m, &status, &n_slots, &stage_words, &ca};
+  const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(256), args, lds, stream);
+  return e != hipSuccess ? e : hipGetLastError();
 }
 
 hipError_t launch_rilv_size(const IlvEncPlane* planes, const RilvEncBlock* blocks, uint32_t n_blocks,

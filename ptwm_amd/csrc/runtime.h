@@ -36,24 +36,24 @@ struct PinnedBuffer {
 
 // The allocation-free decode (ptwm_mi355x_dispatch_decode_noalloc_cuda):
 // all its device scratch lives in one fixed array per device (runtime.hip),
-// laid out as [CRC tables][tensor descriptors, launch indexes, status]
-// [CRC range arguments][CRC combine arguments][exact-route stubs][CRC block
-// partials], and its host staging in a fixed per-device host area.
+// laid out as [CRC accumulators][tensor descriptors, launch indexes][CRC
+// tables][exact-route stubs], and its host staging in a fixed per-device host
+// area.
 constexpr uint64_t kNoAllocScratchBytes = 16ull << 20;
-constexpr uint64_t kNoAllocTabOff = 0, kNoAllocTabBytes = 16ull << 10;
-constexpr uint64_t kNoAllocArgsOff = kNoAllocTabOff + kNoAllocTabBytes, kNoAllocArgsBytes = 1ull << 20;
-constexpr uint64_t kNoAllocCrcArgsOff = kNoAllocArgsOff + kNoAllocArgsBytes, kNoAllocCrcArgsBytes = 1ull << 20;
-constexpr uint64_t kNoAllocCombOff = kNoAllocCrcArgsOff + kNoAllocCrcArgsBytes, kNoAllocCombBytes = 512ull << 10;
-constexpr uint64_t kNoAllocStubOff = kNoAllocCombOff + kNoAllocCombBytes, kNoAllocStubBytes = 4096;
-constexpr uint64_t kNoAllocPartOff = kNoAllocStubOff + kNoAllocStubBytes;
-constexpr uint64_t kNoAllocPartBytes = kNoAllocScratchBytes - kNoAllocPartOff;
+constexpr uint64_t kNoAllocAccOff = 0, kNoAllocAccBytes = 128ull << 10;
+constexpr uint64_t kNoAllocArgsOff = kNoAllocAccOff + kNoAllocAccBytes, kNoAllocArgsBytes = 1ull << 20;
+constexpr uint64_t kNoAllocTabOff = kNoAllocArgsOff + kNoAllocArgsBytes, kNoAllocTabBytes = 128ull << 10;
+constexpr uint64_t kNoAllocStubOff = kNoAllocTabOff + kNoAllocTabBytes, kNoAllocStubBytes = 4096;
+static_assert(kNoAllocStubOff + kNoAllocStubBytes <= kNoAllocScratchBytes, "allocation-free scratch layout");
 constexpr uint64_t kNoAllocHostBytes = 1ull << 20;
-// host-coherent status words of the fused decode (one per tensor)
+// host-coherent words of the fused decode: a status word per tensor, then
+// its plane CRC sums
 constexpr uint64_t kNoAllocStatusBytes = 16ull << 10;
+constexpr uint64_t kNoAllocCrcOutBytes = (64ull << 10) + 256;
 static_assert(kNoAllocStatusBytes >= 4ull * 4096, "a status word for every tensor the allocation-free decode takes");
 // limits of a plan the allocation-free decode accepts
 constexpr uint32_t kNoAllocMaxTensors = 4096;
-constexpr uint64_t kNoAllocMaxCrcBlocks = kNoAllocPartBytes / 16;
+constexpr uint64_t kNoAllocMaxCrcBlocks = 883456;
 
 // One host hashing worker (hash_host.hip): its stream, two pinned chunk
 // buffers and their copy-done events.
@@ -85,7 +85,6 @@ struct DevCtx {
   PinnedBuffer h_small;
   // huff_ilv encoder / decoder scratch
   DeviceBuffer enc_planes, enc_hist, enc_codes, enc_blocks, enc_lane_words, enc_block_bytes, enc_pack;
-  DeviceBuffer crc_comb, crc_part;  // CRC combine arguments; fused-decode CRC block partials
   DeviceBuffer ilv_args, ilv_realign, realign_jobs;
   PinnedBuffer h_realign;
   // reference-format (Huffman / rANS) encoder scratch
@@ -112,6 +111,10 @@ struct DevCtx {
   PinnedBuffer h_chunk;
   // integrity (CRC-32 / XXH64) tables and arguments
   DeviceBuffer crc_tab, crc_args;
+  DeviceBuffer crc_acc;       // workgroup counter and plane accumulators, zero between calls
+  PinnedBuffer h_crc;         // their sums, written by the kernels (host-coherent)
+  PinnedBuffer h_crc_args;
+  bool crc_dirty = false;     // a call began to add to them and has not taken them
   std::vector<HashWorker> hash_workers;  // XXH64 on host cores (hash_host.hip)
   hipEvent_t hash_ready = nullptr;       // the restore is complete before the copies
   bool crc_tab_ready = false;
@@ -136,8 +139,8 @@ struct DevCtx {
   // in the scratch yet
   uint8_t* noalloc_dev = nullptr;
   std::unique_ptr<uint8_t[]> noalloc_host;
-  void* noalloc_status = nullptr;  // kNoAllocStatusBytes of host-coherent memory
-  bool noalloc_tab_ready = false;
+  void* noalloc_status = nullptr;  // kNoAllocStatusBytes + kNoAllocCrcOutBytes of host-coherent memory
+  bool noalloc_tab_ready = false, noalloc_crc_dirty = false;
 };
 
 // Returns nullptr if the ordinal is invalid or HIP initialisation fails.

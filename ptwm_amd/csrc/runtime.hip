@@ -124,13 +124,14 @@ DevCtx* get_ctx(uint32_t ord) {
   ctx->stream = ctx->own_stream;
   ctx->h_ilv_status.flags = hipHostMallocCoherent;
   ctx->h_job_status.flags = hipHostMallocCoherent;
+  ctx->h_crc.flags = hipHostMallocCoherent;
   // the allocation-free decode's scratch on this device (the device is
   // current): its address, or null, and the entry point then reports
   // MissingCapability
   void* sp = nullptr;
   note_alloc();
   if (hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)) == hipSuccess && sp &&
-      hipHostMalloc(&ctx->noalloc_status, kNoAllocStatusBytes, hipHostMallocCoherent) == hipSuccess) {
+      hipHostMalloc(&ctx->noalloc_status, kNoAllocStatusBytes + kNoAllocCrcOutBytes, hipHostMallocCoherent) == hipSuccess) {
     ctx->noalloc_dev = static_cast<uint8_t*>(sp);
     ctx->noalloc_host.reset(new uint8_t[kNoAllocHostBytes]);
   } else {
@@ -152,10 +153,8 @@ bool fused_eligible(const PlanTensor& T, uint64_t out_dev) {
     else if (P.codec == kCodecRansIlv) any_rans = true;
     else if (P.codec != kCodecIdentity || P.payload_len != P.plane_len) ok = false;
   }
-  // one codec family per fused tensor; a plane CRC is checked on the
-  // restored tensor where the chain is a bijection on plane bytes (other
-  // chains keep their planes in scratch)
-  return ok && any_huff != any_rans && (!T.has_crc || crc_chain_supported(T.chain));
+  // one codec family per fused tensor
+  return ok && any_huff != any_rans;
 }
 
 namespace {
@@ -164,27 +163,26 @@ namespace {
 // buffers for the length of one allocation-free call; the context's own
 // buffers come back when it ends.
 struct Borrow {
-  DeviceBuffer* dst[9];
-  DeviceBuffer saved[9];
-  PinnedBuffer* hdst[4];
-  PinnedBuffer hsaved[4];
-  bool tab_ready;
+  DeviceBuffer* dst[8];
+  DeviceBuffer saved[8];
+  PinnedBuffer* hdst[5];
+  PinnedBuffer hsaved[5];
+  bool tab_ready, crc_dirty;
   DevCtx& ctx;
   explicit Borrow(DevCtx& c) : ctx(c) {
     uint8_t* d = c.noalloc_dev;
     struct View {
       DeviceBuffer* b;
       uint64_t off, len;
-    } v[9] = {{&c.crc_tab, kNoAllocTabOff, kNoAllocTabBytes},
+    } v[8] = {{&c.crc_tab, kNoAllocTabOff, kNoAllocTabBytes},
+              {&c.crc_acc, kNoAllocAccOff, kNoAllocAccBytes},
               {&c.ilv_args, kNoAllocArgsOff, kNoAllocArgsBytes},
-              {&c.crc_args, kNoAllocCrcArgsOff, kNoAllocCrcArgsBytes},
-              {&c.crc_comb, kNoAllocCombOff, kNoAllocCombBytes},
+              {&c.crc_args, 0, 0},
               {&c.planes, kNoAllocStubOff, 1024},
               {&c.jobs, kNoAllocStubOff + 1024, 1024},
               {&c.status, kNoAllocStubOff + 2048, 1024},
-              {&c.crc_part, kNoAllocPartOff, kNoAllocPartBytes},
               {&c.ilv_realign, 0, 0}};
-    for (int i = 0; i < 9; ++i) {
+    for (int i = 0; i < 8; ++i) {
       dst[i] = v[i].b;
       saved[i] = *v[i].b;
       v[i].b->ptr = v[i].len ? d + v[i].off : nullptr;
@@ -192,11 +190,12 @@ struct Borrow {
       v[i].b->borrowed = true;
     }
     uint8_t* h = c.noalloc_host.get();
-    PinnedBuffer* hb[4] = {&c.h_ilv, &c.h_jobs, &c.h_status, &c.h_ilv_status};
-    uint8_t* const hbase[4] = {h, h, h, static_cast<uint8_t*>(c.noalloc_status)};
-    const uint64_t hoff[4] = {0, kNoAllocHostBytes - 2048, kNoAllocHostBytes - 1024, 0};
-    const uint64_t hlen[4] = {kNoAllocHostBytes - 2048, 1024, 1024, kNoAllocStatusBytes};
-    for (int i = 0; i < 4; ++i) {
+    uint8_t* st = static_cast<uint8_t*>(c.noalloc_status);
+    PinnedBuffer* hb[5] = {&c.h_ilv, &c.h_jobs, &c.h_status, &c.h_ilv_status, &c.h_crc};
+    uint8_t* const hbase[5] = {h, h, h, st, st};
+    const uint64_t hoff[5] = {0, kNoAllocHostBytes - 2048, kNoAllocHostBytes - 1024, 0, kNoAllocStatusBytes};
+    const uint64_t hlen[5] = {kNoAllocHostBytes - 2048, 1024, 1024, kNoAllocStatusBytes, kNoAllocCrcOutBytes};
+    for (int i = 0; i < 5; ++i) {
       hdst[i] = hb[i];
       hsaved[i] = *hb[i];
       hb[i]->ptr = hbase[i] + hoff[i];
@@ -205,12 +204,16 @@ struct Borrow {
     }
     tab_ready = c.crc_tab_ready;
     c.crc_tab_ready = c.noalloc_tab_ready;
+    crc_dirty = c.crc_dirty;
+    c.crc_dirty = c.noalloc_crc_dirty;
   }
   ~Borrow() {
     ctx.noalloc_tab_ready = ctx.crc_tab_ready;
     ctx.crc_tab_ready = tab_ready;
-    for (int i = 0; i < 9; ++i) *dst[i] = saved[i];
-    for (int i = 0; i < 4; ++i) *hdst[i] = hsaved[i];
+    ctx.noalloc_crc_dirty = ctx.crc_dirty;
+    ctx.crc_dirty = crc_dirty;
+    for (int i = 0; i < 8; ++i) *dst[i] = saved[i];
+    for (int i = 0; i < 5; ++i) *hdst[i] = hsaved[i];
   }
 };
 
@@ -222,6 +225,8 @@ int64_t execute_plan_noalloc(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uin
   uint64_t crc_blocks = 0;
   for (const PlanTensor& T : plan.tensors) {
     if (T.has_hash || !fused_eligible(T, out_dev)) return kUnsupported;
+    // (its fused CRC may have to be taken again through plane scratch)
+    if (T.has_crc && chain_nibbles(T.chain)) return kUnsupported;
     bool rans = false;
     for (const PlanPlane& P : T.planes) {
       rans |= P.codec == kCodecRansIlv;
@@ -344,12 +349,12 @@ bool chunked_fused_eligible(const PlanTensor& T, uint64_t out_dev, const ChunkRa
       if (P.codec == kCodecIdentity && rg.second != P.chunks[k].decoded_size) return false;
     }
   }
-  return any_huff != any_rans && (!T.has_crc || crc_chain_supported(T.chain));
+  return any_huff != any_rans;
 }
 
-}  // namespace
-
-int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t out_dev) {
+// execute_plan; with scratch_nibbles, nibble-chain tensors with plane CRCs
+// take the exact route (the fused one found symbols above 15 in them).
+int64_t execute_plan_on(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t out_dev, bool scratch_nibbles) {
   // Route 1 (fused): a tensor whose planes are all unchunked Identity or
   // GPU-native payloads of one codec family (huff_ilv or rans_ilv), with at
   // least one coded plane, is decoded and merged in one pass by that
@@ -368,10 +373,12 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
     }
   std::vector<IlvTensor> ilv;
   std::vector<char> fused(nt, 0);
-  // huff_ilv tensors with plane CRCs: the decode kernel also writes the CRC
-  // partials of their whole blocks (tensor t's from block crc_first[t])
-  std::vector<uint32_t> crc_first(nt, kIlvNoCrc);
-  uint64_t crc_blocks = 0;
+  std::vector<uint32_t> ilv_of;  // the plan tensor of each of them (or kNone)
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  // fused tensors with plane CRCs: the decode kernels sum tensor t's into the
+  // accumulators from crc_ix[t] on
+  std::vector<uint32_t> crc_ix(nt, kIlvNoCrc);
+  uint32_t n_acc = 0;
   ChunkRanges cr;
   {
     const int64_t rc = chunk_ranges(ctx, plan, in_dev, cr);
@@ -379,17 +386,18 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
   }
   for (size_t t = 0; t < nt; ++t) {
     const PlanTensor& T = plan.tensors[t];
+    if (scratch_nibbles && T.has_crc && chain_nibbles(T.chain)) continue;
     if (!fused_eligible(T, out_dev)) {
       if (!chunked_fused_eligible(T, out_dev, cr, t)) continue;
       // one sub-tensor per chunk (chunked_fused_eligible)
       bool any_rans = false;
       for (const PlanPlane& P : T.planes) any_rans |= P.codec == kCodecRansIlv;
       fused[t] = 1;
-      const uint64_t n = T.planes[0].plane_len;
-      if (T.has_crc && !any_rans && n > 0) {
-        crc_first[t] = (uint32_t)crc_blocks;
-        crc_blocks += (n + kIlvBlock - 1) / kIlvBlock;
-        if (crc_blocks > 0xFFFFFFFEull) return kInvalidInput;
+      const uint64_t nb = (T.planes[0].plane_len + kIlvBlock - 1) / kIlvBlock;
+      if (nb > 0xFFFFFFFEull) return kInvalidInput;
+      if (T.has_crc && nb) {
+        crc_ix[t] = n_acc;
+        n_acc += (uint32_t)T.planes.size();
       }
       const uint32_t coded_codec = any_rans ? kCodecRansIlv : kCodecHuffIlv;
       const uint64_t ratio = (uint64_t)chain_ratio(T.chain);
@@ -401,14 +409,18 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
         X.chain = T.chain;
         X.n_planes = (uint32_t)T.planes.size();
         X.family = any_rans ? kFamilyRans : kFamilyHuff;
-        X.crc_first = crc_first[t] == kIlvNoCrc ? kIlvNoCrc : crc_first[t] + (uint32_t)(a / kIlvBlock);
+        X.crc_ix = crc_ix[t];
+        X.crc_last = (uint32_t)(nb - 1 - a / kIlvBlock);
         for (size_t p = 0; p < T.planes.size(); ++p) {
           X.planes[p].base = cr.r[t][p][k].first;
           X.planes[p].len = cr.r[t][p][k].second;
           X.planes[p].coded = T.planes[p].codec == coded_codec ? 1 : 0;
           X.planes[p].lut = (uint32_t)p;
         }
-        if (X.n > 0) ilv.push_back(X);
+        if (X.n > 0) {
+          ilv.push_back(X);
+          ilv_of.push_back((uint32_t)t);
+        }
         a += X.n;
       }
       continue;
@@ -422,11 +434,13 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
     X.chain = T.chain;
     X.n_planes = (uint32_t)T.planes.size();
     X.family = any_rans ? kFamilyRans : kFamilyHuff;
-    X.crc_first = kIlvNoCrc;
-    if (T.has_crc && !any_rans && X.n > 0) {
-      X.crc_first = crc_first[t] = (uint32_t)crc_blocks;
-      crc_blocks += (X.n + kIlvBlock - 1) / kIlvBlock;
-      if (crc_blocks > 0xFFFFFFFEull) return kInvalidInput;
+    X.crc_ix = kIlvNoCrc;
+    const uint64_t nb = (X.n + kIlvBlock - 1) / kIlvBlock;
+    if (nb > 0xFFFFFFFEull) return kInvalidInput;
+    if (T.has_crc && nb) {
+      X.crc_ix = crc_ix[t] = n_acc;
+      X.crc_last = (uint32_t)(nb - 1);
+      n_acc += (uint32_t)T.planes.size();
     }
     const uint32_t coded_codec = any_rans ? kCodecRansIlv : kCodecHuffIlv;
     for (size_t p = 0; p < T.planes.size(); ++p) {
@@ -436,6 +450,7 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
       X.planes[p].lut = (uint32_t)p;
     }
     ilv.push_back(X);
+    ilv_of.push_back((uint32_t)t);
   }
   // Pass 1 (exact route): lay out plane scratch and count jobs.  A plane
   // needs scratch unless it is a single unchunked Identity payload whose
@@ -518,8 +533,11 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
           X.planes[0].len = cr.r[t][p][k].second;
           X.planes[0].coded = 1;
           X.family = P.codec == kCodecRansIlv ? kFamilyRans : kFamilyHuff;
-          X.crc_first = kIlvNoCrc;
-          if (X.n > 0) ilv.push_back(X);
+          X.crc_ix = kIlvNoCrc;
+          if (X.n > 0) {
+            ilv.push_back(X);
+            ilv_of.push_back(kNone);
+          }
           off += P.chunks[k].decoded_size;
         }
         continue;
@@ -535,8 +553,9 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
         X.planes[0].len = P.payload_len;
         X.planes[0].coded = 1;
         X.family = P.codec == kCodecRansIlv ? kFamilyRans : kFamilyHuff;
-        X.crc_first = kIlvNoCrc;
+        X.crc_ix = kIlvNoCrc;
         ilv.push_back(X);
+        ilv_of.push_back(kNone);
         continue;
       }
       if (!P.chunked) {
@@ -581,10 +600,21 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
     ctx.last_ms[0] = ctx.last_ms[1] = ctx.last_ms[2] = 0;
   }
   // huff_ilv first: fused tensors straight to the output, passthrough planes to scratch
+  std::vector<uint32_t> fused_crc;  // the accumulators' sums
+  std::vector<char> through_scratch(nt, 0);
+  Plan again;  // tensors to be decoded again through plane scratch
   if (!ilv.empty()) {
-    if (crc_blocks) PTWM_HIP_TRY(ctx.crc_part.ensure(16ull * crc_blocks));
-    int64_t rc = ilv_decode_tensors(ctx, ilv);
+    std::vector<uint32_t> flagged;
+    int64_t rc = ilv_decode_tensors(ctx, ilv, n_acc, fused_crc, flagged);
     if (rc != kOk) return rc;
+    for (const uint32_t i : flagged) {
+      const uint32_t t = ilv_of[i];
+      if (t == kNone) return kInternal;
+      if (through_scratch[t]) continue;
+      through_scratch[t] = 1;
+      again.tensors.push_back(plan.tensors[t]);
+    }
+    if (scratch_nibbles && !again.tensors.empty()) return kInternal;
   }
   if (ctx.profile) PTWM_HIP_TRY(hipEventRecord(ctx.ev[0], s));
   // Reference-format payloads: parallel Huffman path where it applies, exact
@@ -632,6 +662,15 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
     const int64_t rc = run_plane_ops(ctx, ops);
     if (rc != kOk) return rc;
   }
+  // The exact route's plane CRCs (container.rs:2154-2159: of each decoded
+  // plane, before its op), queued with the merges.
+  std::vector<CrcTask> crc_tasks;
+  for (size_t t = 0; t < nt; ++t)
+    if (!fused[t] && plan.tensors[t].has_crc)
+      for (size_t p = 0; p < plan.tensors[t].planes.size(); ++p)
+        crc_tasks.push_back(CrcTask{plane_addr[t][p], plan.tensors[t].planes[p].plane_len, kChainPassthrough});
+  CrcRun crc_run;
+  bool queued = false;  // work on the stream that nothing has waited for
   if (ctx.profile) PTWM_HIP_TRY(hipEventRecord(ctx.ev[1], s));
   const auto launch_merges = [&]() -> int64_t {
     for (size_t t = 0; t < nt; ++t) {
@@ -641,6 +680,7 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
       for (size_t p = 0; p < T.planes.size(); ++p) pp[p] = reinterpret_cast<const uint8_t*>(merge_addr[t][p]);
       uint8_t* out = reinterpret_cast<uint8_t*>(out_dev + T.out_offset);
       if (T.planes[0].plane_len == 0) continue;
+      queued = true;
       if (merge_tmp[t] == kDirect) {
         PTWM_HIP_TRY(launch_merge(T.chain, pp, T.planes[0].plane_len, out, s));
       } else {
@@ -654,18 +694,25 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
   {
     int64_t rc = launch_merges();
     if (rc != kOk) return rc;
+    if (ctx.profile) PTWM_HIP_TRY(hipEventRecord(ctx.ev[2], s));
+    rc = crc_launch(ctx, crc_tasks, crc_run);
+    if (rc != kOk) return rc;
+    queued |= crc_run.any;
     if (n_jobs && !any_op) {
       bool rewritten = false;
       rc = complete_jobs(rewritten);
       if (rc != kOk) return rc;
+      queued = false;
       if (rewritten) {
         rc = launch_merges();
         if (rc != kOk) return rc;
+        rc = crc_launch(ctx, crc_tasks, crc_run);
+        if (rc != kOk) return rc;
+        queued = true;
       }
     }
   }
-  if (ctx.profile) PTWM_HIP_TRY(hipEventRecord(ctx.ev[2], s));
-  PTWM_HIP_TRY(hipStreamSynchronize(s));
+  if (queued || ctx.profile) PTWM_HIP_TRY(hipStreamSynchronize(s));
   if (ctx.profile) {
     float a = 0, b = 0;
     PTWM_HIP_TRY(hipEventElapsedTime(&a, ctx.ev[0], ctx.ev[1]));
@@ -677,46 +724,38 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
   // Integrity, after every tensor is restored: CRC-32 of each decoded plane
   // (container.rs:2154-2159) and XXH64 of each restored tensor
   // (container.rs:2185-2194); a mismatch is InvalidContainer there.
-  std::vector<CrcTask> crc_tasks;
-  std::vector<uint32_t> crc_want;
-  std::vector<FusedCrc> crc_fused;
-  std::vector<uint32_t> crc_fused_want;
+  std::vector<uint32_t> exact_crc;
+  {
+    const int64_t rc = crc_values(ctx, crc_run, exact_crc);
+    if (rc != kOk) return rc;
+  }
   std::vector<HashTask> hash_tasks;
   std::vector<uint64_t> hash_want;
+  size_t next_exact = 0;
   for (size_t t = 0; t < nt; ++t) {
     const PlanTensor& T = plan.tensors[t];
-    if (T.has_crc && crc_first[t] != kIlvNoCrc) {
-      crc_fused.push_back(FusedCrc{out_dev + T.out_offset, T.planes[0].plane_len, T.chain, crc_first[t]});
-      for (const PlanPlane& P : T.planes) crc_fused_want.push_back(P.crc32);
-    } else if (T.has_crc) {
-      if (fused[t]) {
-        crc_tasks.push_back(CrcTask{out_dev + T.out_offset, T.planes[0].plane_len, T.chain});
-      } else {
-        for (size_t p = 0; p < T.planes.size(); ++p)
-          crc_tasks.push_back(CrcTask{plane_addr[t][p], T.planes[p].plane_len, kChainPassthrough});
+    if (T.has_crc && !through_scratch[t])
+      for (size_t p = 0; p < T.planes.size(); ++p) {
+        const PlanPlane& P = T.planes[p];
+        uint32_t got = 0, want = P.crc32;  // an empty plane's CRC is 0
+        if (crc_ix[t] != kIlvNoCrc) {
+          got = fused_crc[crc_ix[t] + p];
+          want = crc_expected(P.crc32, P.plane_len, kIlvBlock);
+        } else if (!fused[t]) {
+          got = exact_crc[next_exact++];
+          if (P.plane_len) want = crc_expected(P.crc32, P.plane_len, 1);
+        }
+        if (got != want) return kInvalidInput;
       }
-      for (const PlanPlane& P : T.planes) crc_want.push_back(P.crc32);
-    }
-    if (T.has_hash) {
+    if (T.has_hash && !through_scratch[t]) {
       hash_tasks.push_back(HashTask{out_dev + T.out_offset, T.out_len});
       hash_want.push_back(T.xxh64);
     }
   }
-  if (!crc_tasks.empty()) {
-    std::vector<uint32_t> got;
-    const int64_t rc = crc32_planes(ctx, crc_tasks, got);
+  // (the scratch and the job list are free again here)
+  if (!again.tensors.empty()) {
+    const int64_t rc = execute_plan_on(ctx, again, in_dev, out_dev, true);
     if (rc != kOk) return rc;
-    if (got.size() != crc_want.size()) return kInternal;
-    for (size_t k = 0; k < got.size(); ++k)
-      if (got[k] != crc_want[k]) return kInvalidInput;
-  }
-  if (!crc_fused.empty()) {
-    std::vector<uint32_t> got;
-    const int64_t rc = crc32_fused(ctx, crc_fused, static_cast<uint32_t*>(ctx.crc_part.ptr), got);
-    if (rc != kOk) return rc;
-    if (got.size() != crc_fused_want.size()) return kInternal;
-    for (size_t k = 0; k < got.size(); ++k)
-      if (got[k] != crc_fused_want[k]) return kInvalidInput;
   }
   if (!hash_tasks.empty()) {
     std::vector<uint64_t> got;
@@ -726,6 +765,12 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
       if (got[k] != hash_want[k]) return kInvalidInput;
   }
   return kOk;
+}
+
+}  // namespace
+
+int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t out_dev) {
+  return execute_plan_on(ctx, plan, in_dev, out_dev, false);
 }
 
 }  // namespace ptwm
