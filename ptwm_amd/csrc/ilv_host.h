@@ -3,6 +3,7 @@
 
 #include <vector>
 
+#include "code_tables.h"
 #include "huff_ilv.h"
 #include "runtime.h"
 
@@ -25,13 +26,6 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
 // Payload forms of both GPU-native codecs.
 enum IlvForm : uint32_t { kFormStored = 0, kFormCoded = 1, kFormPacked = 2, kFormIdentity = 3 };
 
-// True when the 256-bin histogram has no symbol >= 16.
-inline bool all_nibbles(const uint32_t* hist) {
-  for (int s = 16; s < 256; ++s)
-    if (hist[s]) return false;
-  return true;
-}
-
 // The encoders' choice of payload form (the format specification's rule):
 // coded (tag 1) when strictly smaller than both other forms; else packed
 // nibbles (tag 2) when every symbol is < 16 and that beats storing; else
@@ -47,6 +41,12 @@ uint32_t ilv_choose_form(uint64_t n, bool nibbles, bool codable, uint64_t coded_
 // plane copies and one pack launch.  Returns kOk or an error status.
 int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
                          const IlvEncResult* res, const uint32_t* form, std::vector<uint8_t>& keep);
+
+// Histograms and entropy tables (TableKind `kind`) of the planes: the planes
+// to ctx.enc_planes, the tables to ctx.enc_codes; *info: what the host needs
+// of them, valid until the next table build.  Blocks until done.
+int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, uint64_t max_n, uint32_t kind,
+                         const TableInfo** info);
 
 // The same for the rans_ilv codec (rans_host.hip).
 int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,

@@ -1,7 +1,7 @@
 // ilv_host.hip -- host orchestration of the huff_ilv encoder and decoder.
 //
-// Encode (per call, any number of planes): histogram kernel -> host code
-// tables (huffman_host.cpp) -> size kernel -> host prefix sums and payload
+// Encode (per call, any number of planes): histogram kernel -> code tables
+// (code_tables.hip) -> size kernel -> host prefix sums and payload
 // layout -> encode kernel plus header / offset-table uploads.  Each plane
 // takes the smallest payload form (ilv_choose_form): coded, packed nibbles
 // or stored.
@@ -13,11 +13,9 @@
 
 #include <algorithm>
 #include <cstring>
-#include <thread>
 #include <vector>
 
 #include "huff_ilv.h"
-#include "huffman_host.h"
 #include "ilv_host.h"
 #include "integrity.h"
 #include "rans_ilv.h"
@@ -89,71 +87,60 @@ int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, ui
   return kOk;
 }
 
+int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, uint64_t max_n, uint32_t kind,
+                         const TableInfo** info) {
+  hipStream_t s = ctx.stream;
+  const uint32_t np = (uint32_t)planes.size();
+  const size_t b_pl = np * sizeof(IlvEncPlane), b_tj = np * sizeof(TableJob);
+  PTWM_HIP_TRY(ctx.enc_planes.ensure(b_pl + b_tj));
+  PTWM_HIP_TRY(ctx.enc_hist.ensure(np * 256 * sizeof(uint32_t)));
+  PTWM_HIP_TRY(ctx.enc_codes.ensure(np * 256 * sizeof(uint32_t)));
+  PTWM_HIP_TRY(ctx.h_enc.ensure(b_pl + b_tj));
+  PTWM_HIP_TRY(ctx.h_tables.ensure(np * sizeof(TableInfo)));
+  uint8_t* const h = static_cast<uint8_t*>(ctx.h_enc.ptr);
+  std::memcpy(h, planes.data(), b_pl);
+  TableJob* const tj = reinterpret_cast<TableJob*>(h + b_pl);
+  for (uint32_t p = 0; p < np; ++p) tj[p] = TableJob{kind, p, 1, 0};
+  uint8_t* const d = static_cast<uint8_t*>(ctx.enc_planes.ptr);
+  uint32_t* const hist = static_cast<uint32_t*>(ctx.enc_hist.ptr);
+  TableInfo* const out = static_cast<TableInfo*>(ctx.h_tables.ptr);
+  PTWM_HIP_TRY(hipMemcpyAsync(d, h, b_pl + b_tj, hipMemcpyHostToDevice, s));
+  PTWM_HIP_TRY(hipMemsetAsync(hist, 0, np * 256 * sizeof(uint32_t), s));
+  PTWM_HIP_TRY(launch_ilv_hist(reinterpret_cast<const IlvEncPlane*>(d), np, max_n, hist, s));
+  PTWM_HIP_TRY(launch_code_tables(reinterpret_cast<const TableJob*>(d + b_pl), np, hist,
+                                  static_cast<uint32_t*>(ctx.enc_codes.ptr), nullptr, out, s));
+  PTWM_HIP_TRY(hipStreamSynchronize(s));
+  *info = out;
+  return kOk;
+}
+
 int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
                           uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed) {
   hipStream_t s = ctx.stream;
   if (np == 0) return 0;
   for (uint32_t p = 0; p < np; ++p)
     if ((src[p] & 15u) != 0 || n[p] > 0xFFFFFFFFull) return kInvalidInput;
-  // ---- histograms ----
   std::vector<IlvEncPlane> hp(np);
   uint64_t max_n = 0;
   for (uint32_t p = 0; p < np; ++p) {
     hp[p] = IlvEncPlane{src[p], n[p], p, 0};
     max_n = std::max(max_n, n[p]);
   }
-  PTWM_HIP_TRY(ctx.enc_planes.ensure(np * sizeof(IlvEncPlane)));
-  PTWM_HIP_TRY(ctx.enc_hist.ensure(np * 256 * sizeof(uint32_t)));
-  PTWM_HIP_TRY(ctx.h_enc.ensure(np * 256 * sizeof(uint32_t) + np * sizeof(IlvEncPlane)));
-  std::memcpy(ctx.h_enc.ptr, hp.data(), np * sizeof(IlvEncPlane));
-  PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_planes.ptr, ctx.h_enc.ptr, np * sizeof(IlvEncPlane), hipMemcpyHostToDevice, s));
-  PTWM_HIP_TRY(hipMemsetAsync(ctx.enc_hist.ptr, 0, np * 256 * sizeof(uint32_t), s));
-  PTWM_HIP_TRY(launch_ilv_hist(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr), np, max_n,
-                               static_cast<uint32_t*>(ctx.enc_hist.ptr), s));
-  std::vector<uint32_t> hist(np * 256);
-  PTWM_HIP_TRY(hipMemcpyAsync(hist.data(), ctx.enc_hist.ptr, np * 256 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  PTWM_HIP_TRY(hipStreamSynchronize(s));
-  // ---- code tables ----
-  std::vector<uint32_t> codes(np * 256, 0);
-  std::vector<std::vector<uint8_t>> weights(np);
+  // ---- code tables (code_tables.hip) ----
+  const TableInfo* info = nullptr;
+  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableIlv, &info); rc != kOk) return rc;
   std::vector<uint8_t> codable(np, 0);
-  // planes are independent (each writes its own entries): spread large
-  // batches over host threads
-  auto build_codes = [&](uint32_t p0, uint32_t p1) {
-    for (uint32_t p = p0; p < p1; ++p) {
-      if (n[p] == 0) continue;
-      uint8_t lengths[256];
-      uint16_t rev[256];
-      if (!ilv_lengths_from_freqs(&hist[256 * p], lengths)) continue;
-      if (!huf_canonical(lengths, rev)) continue;
-      for (int sy = 0; sy < 256; ++sy) codes[256 * p + sy] = ((uint32_t)lengths[sy] << 16) | rev[sy];
-      uint8_t w[140];
-      int wl = huf_encode_weights(lengths, w);
-      if (wl < 0) continue;
-      // a coded payload is at least its header, offset table, lane counts
-      // and ceil(code bits / 8): a plane for which that is not shorter than
-      // the stored or packed form is not sized (the form choice below would
-      // not take the coded form)
-      uint64_t bits = 0;
-      for (int sy = 0; sy < 256; ++sy) bits += (uint64_t)hist[256 * p + sy] * lengths[sy];
-      const uint64_t nb = (n[p] + kIlvBlock - 1) / kIlvBlock;
-      const uint64_t lower = align_up(5 + (uint64_t)wl, 4) + 4 * (nb + 1) + 64 * nb + (bits + 7) / 8;
-      const uint64_t stored = n[p] + 1, packed = kPackedHeadBytes + (n[p] + 1) / 2;
-      const uint64_t other = all_nibbles(&hist[256 * p]) && packed < stored ? packed : stored;
-      if (lower >= other) continue;
-      weights[p].assign(w, w + wl);
-      codable[p] = 1;
-    }
-  };
-  const uint32_t hw = std::max(1u, std::thread::hardware_concurrency());
-  const uint32_t nthr = np >= 64 ? std::min<uint32_t>(std::min<uint32_t>(hw, 8), np / 16) : 1;
-  if (nthr <= 1) {
-    build_codes(0, np);
-  } else {
-    std::vector<std::thread> pool;
-    for (uint32_t t = 0; t < nthr; ++t)
-      pool.emplace_back(build_codes, (uint32_t)((uint64_t)np * t / nthr), (uint32_t)((uint64_t)np * (t + 1) / nthr));
-    for (std::thread& th : pool) th.join();
+  for (uint32_t p = 0; p < np; ++p) {
+    if (n[p] == 0 || !info[p].ok) continue;
+    // a coded payload is at least its header, offset table, lane counts
+    // and ceil(code bits / 8): a plane for which that is not shorter than
+    // the stored or packed form is not sized (the form choice below would
+    // not take the coded form)
+    const uint64_t nb = (n[p] + kIlvBlock - 1) / kIlvBlock;
+    const uint64_t lower = align_up(5 + (uint64_t)info[p].head_len, 4) + 4 * (nb + 1) + 64 * nb + (info[p].bits[0] + 7) / 8;
+    const uint64_t stored = n[p] + 1, packed = kPackedHeadBytes + (n[p] + 1) / 2;
+    const uint64_t other = info[p].n_sym <= 16 && packed < stored ? packed : stored;
+    codable[p] = lower < other;
   }
   // ---- size pass over every block of every codable plane ----
   std::vector<IlvEncBlock> blocks;
@@ -167,17 +154,13 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
   const uint32_t nblk = (uint32_t)blocks.size();
   std::vector<uint32_t> bbytes(nblk);
   if (nblk) {
-    PTWM_HIP_TRY(ctx.enc_codes.ensure(codes.size() * sizeof(uint32_t)));
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(IlvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_lane_words.ensure((size_t)nblk * 64));
     PTWM_HIP_TRY(ctx.enc_block_bytes.ensure(nblk * sizeof(uint32_t)));
-    PTWM_HIP_TRY(ctx.h_enc.ensure(codes.size() * 4 + nblk * sizeof(IlvEncBlock) + nblk * 4 + 64));
-    uint8_t* hb = static_cast<uint8_t*>(ctx.h_enc.ptr);
-    std::memcpy(hb, codes.data(), codes.size() * 4);
-    std::memcpy(hb + codes.size() * 4, blocks.data(), nblk * sizeof(IlvEncBlock));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_codes.ptr, hb, codes.size() * 4, hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_blocks.ptr, hb + codes.size() * 4, nblk * sizeof(IlvEncBlock),
-                                hipMemcpyHostToDevice, s));
+    PTWM_HIP_TRY(ctx.h_enc.ensure(nblk * sizeof(IlvEncBlock)));
+    std::memcpy(ctx.h_enc.ptr, blocks.data(), nblk * sizeof(IlvEncBlock));
+    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_blocks.ptr, ctx.h_enc.ptr, nblk * sizeof(IlvEncBlock), hipMemcpyHostToDevice,
+                                s));
     PTWM_HIP_TRY(launch_ilv_size(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
                                  static_cast<const IlvEncBlock*>(ctx.enc_blocks.ptr), nblk,
                                  static_cast<const uint32_t*>(ctx.enc_codes.ptr),
@@ -198,11 +181,11 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
     if (codable_p) {
       uint64_t d = 0;
       for (uint32_t b = 0; b < nbs[p]; ++b) d += bbytes[first_block[p] + b];
-      head[p] = align_up(5 + weights[p].size(), 4);
+      head[p] = align_up(5 + (uint64_t)info[p].head_len, 4);
       pay = head[p] + 4ull * (nbs[p] + 1) + d;
       codable_p = d <= 0xFFFFFFFFull;
     }
-    form[p] = ilv_choose_form(n[p], all_nibbles(&hist[256 * p]), codable_p, pay, identity_fallback, &res[p].len);
+    form[p] = ilv_choose_form(n[p], info[p].n_sym <= 16, codable_p, pay, identity_fallback, &res[p].len);
     res[p].coded = form[p] == kFormCoded ? 1 : 0;
     res[p].codec = form[p] == kFormIdentity ? kCodecIdentity : kCodecHuffIlv;
     off += res[p].len;
@@ -231,7 +214,7 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
     h[0] = 1;
     uint32_t nn = (uint32_t)n[p];
     std::memcpy(h + 1, &nn, 4);
-    std::memcpy(h + 5, weights[p].data(), weights[p].size());
+    std::memcpy(h + 5, info[p].head, info[p].head_len);
     uint32_t* tab = reinterpret_cast<uint32_t*>(h + head[p]);
     uint64_t acc = 0;
     const uint64_t data_dev = dst + head[p] + 4ull * (nbs[p] + 1);

@@ -1,9 +1,8 @@
 // rans_host.hip -- host orchestration of the rans_ilv encoder.
 //
-// Per call, any number of planes: histogram kernel (shared with huff_ilv) ->
-// host normalisation (the reference's normalize_freqs) -> size kernel (word
-// counts per block) -> host layout and header / offset-table uploads ->
-// write kernel.  Each plane takes the smallest payload form
+// Per call, any number of planes: histogram kernel and frequency tables
+// (ilv_plane_tables, shared with huff_ilv) -> size kernel (word counts per
+// block) -> host layout and header / offset-table uploads -> write kernel.  Each plane takes the smallest payload form
 // (ilv_choose_form): coded, packed nibbles or stored.  Decode runs through ilv_decode_tensors (family
 // kFamilyRans).
 #include <hip/hip_runtime.h>
@@ -12,7 +11,6 @@
 #include <cstring>
 #include <vector>
 
-#include "huffman_host.h"
 #include "ilv_host.h"
 #include "rans_ilv.h"
 #include "runtime.h"
@@ -27,40 +25,17 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   if (np == 0) return 0;
   for (uint32_t p = 0; p < np; ++p)
     if ((src[p] & 15u) != 0 || n[p] > 0xFFFFFFFFull) return kInvalidInput;
-  // ---- histograms ----
   std::vector<IlvEncPlane> hp(np);
   uint64_t max_n = 0;
   for (uint32_t p = 0; p < np; ++p) {
     hp[p] = IlvEncPlane{src[p], n[p], p, 0};
     max_n = std::max(max_n, n[p]);
   }
-  PTWM_HIP_TRY(ctx.enc_planes.ensure(np * sizeof(IlvEncPlane)));
-  PTWM_HIP_TRY(ctx.enc_hist.ensure(np * 256 * sizeof(uint32_t)));
-  PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_planes.ptr, hp.data(), np * sizeof(IlvEncPlane), hipMemcpyHostToDevice, s));
-  PTWM_HIP_TRY(hipMemsetAsync(ctx.enc_hist.ptr, 0, np * 256 * sizeof(uint32_t), s));
-  PTWM_HIP_TRY(launch_ilv_hist(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr), np, max_n,
-                               static_cast<uint32_t*>(ctx.enc_hist.ptr), s));
-  std::vector<uint32_t> hist(np * 256);
-  PTWM_HIP_TRY(hipMemcpyAsync(hist.data(), ctx.enc_hist.ptr, np * 256 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  PTWM_HIP_TRY(hipStreamSynchronize(s));
-  // ---- frequency tables: per symbol f | cum << 16; headers ----
-  std::vector<uint32_t> syms(np * 256, 0);
-  std::vector<std::vector<uint8_t>> header(np);
+  // ---- frequency tables (code_tables.hip): per symbol f | cum << 16 ----
+  const TableInfo* info = nullptr;
+  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableRansIlv, &info); rc != kOk) return rc;
   std::vector<bool> codable(np, false);
-  for (uint32_t p = 0; p < np; ++p) {
-    if (n[p] == 0) continue;
-    uint16_t f[256], cum[256];
-    int max_sym = 0;
-    if (!rans_normalize_freqs(&hist[256 * p], f, cum, &max_sym)) continue;
-    for (int sy = 0; sy < 256; ++sy) syms[256 * p + sy] = (uint32_t)f[sy] | ((uint32_t)cum[sy] << 16);
-    std::vector<uint8_t>& h = header[p];
-    h.push_back((uint8_t)max_sym);
-    for (int i = 0; i <= max_sym; ++i) {
-      h.push_back((uint8_t)f[i]);
-      h.push_back((uint8_t)(f[i] >> 8));
-    }
-    codable[p] = true;
-  }
+  for (uint32_t p = 0; p < np; ++p) codable[p] = n[p] != 0 && info[p].ok;
   // ---- size pass over every block of every codable plane ----
   std::vector<RilvEncBlock> blocks;
   std::vector<uint32_t> first_block(np, 0), nbs(np, 0);
@@ -73,10 +48,8 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   const uint32_t nblk = (uint32_t)blocks.size();
   std::vector<uint32_t> bwords(nblk);
   if (nblk) {
-    PTWM_HIP_TRY(ctx.enc_codes.ensure(syms.size() * sizeof(uint32_t)));
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(RilvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_block_bytes.ensure(nblk * sizeof(uint32_t)));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_codes.ptr, syms.data(), syms.size() * 4, hipMemcpyHostToDevice, s));
     PTWM_HIP_TRY(
         hipMemcpyAsync(ctx.enc_blocks.ptr, blocks.data(), nblk * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
     PTWM_HIP_TRY(launch_rilv_size(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
@@ -98,11 +71,11 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     if (codable_p) {
       uint64_t d = 0;
       for (uint32_t b = 0; b < nbs[p]; ++b) d += align_up(kRilvBlockHead + 2ull * bwords[first_block[p] + b], 4);
-      head[p] = align_up(5 + header[p].size(), 4);
+      head[p] = align_up(5 + (uint64_t)info[p].head_len, 4);
       pay = head[p] + 4ull * (nbs[p] + 1) + d;
       codable_p = d <= 0xFFFFFFFFull;
     }
-    form[p] = ilv_choose_form(n[p], all_nibbles(&hist[256 * p]), codable_p, pay, identity_fallback, &res[p].len);
+    form[p] = ilv_choose_form(n[p], info[p].n_sym <= 16, codable_p, pay, identity_fallback, &res[p].len);
     res[p].coded = form[p] == kFormCoded ? 1 : 0;
     res[p].codec = form[p] == kFormIdentity ? kCodecIdentity : kCodecRansIlv;
     off += res[p].len;
@@ -128,7 +101,7 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     hbuf[0] = 1;
     const uint32_t nn = (uint32_t)n[p];
     std::memcpy(hbuf.data() + 1, &nn, 4);
-    std::memcpy(hbuf.data() + 5, header[p].data(), header[p].size());
+    std::memcpy(hbuf.data() + 5, info[p].head, info[p].head_len);
     uint32_t* tab = reinterpret_cast<uint32_t*>(hbuf.data() + head[p]);
     uint64_t acc = 0;
     const uint64_t data_dev = dst + hbuf.size();

@@ -72,8 +72,6 @@ class RefEncoder {
   std::vector<JobInfo> info_;
   std::vector<RefSegDev> segs_;
   std::vector<uint64_t> seg_len_;   // bytes of each segment's stream
-  std::vector<uint32_t> huf_codes_;  // per job 256 x (len << 16 | rev code)
-  std::vector<uint32_t> rans_tab_;   // per job 256 x 4 words
   uint64_t pack_words_ = 0;
 };
 

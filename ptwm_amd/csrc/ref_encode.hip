@@ -11,9 +11,9 @@
 // One call encodes a batch of jobs (each one payload: a whole plane or one
 // chunk of a chunked plane):
 //   1. histogram per job (ref_hist_kernel);
-//   2. host: code tables per job (huffman_host.cpp: the reference tree,
-//      canonical codes and weights header; rANS: normalize_freqs and the
-//      EncSymbol reciprocal parameters of rans/compress.rs:35-122);
+//   2. code tables per job (code_tables.hip: the reference tree, canonical
+//      codes and weights header; rANS: normalize_freqs and the EncSymbol
+//      reciprocal parameters of rans/compress.rs:35-122);
 //   3. Huffman: bits per segment from the segment's histogram and the code
 //      lengths (the histograms are taken per split_four segment); rANS:
 //      each segment encoded by one lane into scratch (ref_rans_kernel; a
@@ -33,14 +33,12 @@
 #include <algorithm>
 #include <cstring>
 
-#include "huffman_host.h"
+#include "code_tables.h"
 
 namespace ptwm {
 
 namespace {
 
-constexpr uint32_t kRansProbBits = 11;
-constexpr uint32_t kRansScale = 1u << kRansProbBits;
 constexpr uint32_t kRansL = 1u << 23;
 
 __device__ __forceinline__ uint8_t gbyte(uint64_t a) {
@@ -392,29 +390,6 @@ __global__ void __launch_bounds__(256) ref_copy_kernel(const RefCopyOp* __restri
   for (uint64_t i = fwd + t; i < op.n; i += 256) g_st<uint8_t>(op.dst + i, gbyte(op.src + op.n - 1 - (i - fwd)));
 }
 
-// ---- host restatements of the reference's table construction ----
-
-// EncSymbol (rans/compress.rs:35-68) packed for ref_rans_kernel:
-// {rcp, bias, cmpl | shift << 24, freq << 20}.
-void rans_encsym(uint32_t start, uint32_t freq, uint32_t out[4]) {
-  uint32_t rcp, bias, shift;
-  if (freq < 2) {
-    bias = start + kRansScale - 1;
-    rcp = 0xFFFFFFFFu;
-    shift = 0;
-  } else {
-    uint32_t sh = 0;
-    while (freq > (1u << sh)) ++sh;
-    rcp = (uint32_t)((((uint64_t)1 << (sh + 31)) + freq - 1) / freq);
-    bias = start;
-    shift = sh - 1;
-  }
-  out[0] = rcp;
-  out[1] = bias;
-  out[2] = (kRansScale - freq) | (shift << 24);  // a 24-bit multiply reads the complement alone
-  out[3] = freq << 20;                            // x at or above it sheds a byte
-}
-
 void split_four(uint64_t len, uint64_t start[4], uint64_t n[4]) {
   const uint64_t q = len / 4, r = len % 4;
   uint64_t off = 0;
@@ -441,149 +416,105 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
   info_.assign(nj, JobInfo{});
   segs_.clear();
   if (nj == 0) return kOk;
-  // ---- 1. histograms, one per split_four segment (stream_frame.rs:11-62) ----
+  // ---- 1. histograms, one per split_four segment (stream_frame.rs:11-62),
+  // 2. the jobs' tables, 3. the rANS segments, with one wait at the end ----
   std::vector<RefJobDev> jd;
-  std::vector<uint32_t> sub0(nj, 0);
-  uint64_t max_n = 0;
+  std::vector<TableJob> tj(nj, TableJob{kTableHuffman, 0, 0, 0});
+  std::vector<RefSegDev> rsegs;  // the rANS segments, and their indexes in segs_
+  std::vector<uint32_t> ridx;
+  uint64_t max_n = 0, scratch_words = 0, rans_scratch = 0;
   for (uint32_t j = 0; j < nj; ++j) {
     if (jobs[j].codec != kCodecHuffman && jobs[j].codec != kCodecRans) return kUnsupported;
-    sub0[j] = (uint32_t)jd.size();
-    if (jobs[j].n == 0) continue;
-    uint64_t st[4], sn[4];
-    split_four(jobs[j].n, st, sn);
-    for (int i = 0; i < 4; ++i) jd.push_back(RefJobDev{jobs[j].src + st[i], sn[i]});
-    max_n = std::max(max_n, sn[0]);
-  }
-  const uint32_t nsub = (uint32_t)jd.size();
-  std::vector<uint32_t> seg_hist((size_t)nsub * 256);
-  if (nsub) {
-    PTWM_HIP_TRY(ctx.ref_jobs.ensure(nsub * sizeof(RefJobDev)));
-    PTWM_HIP_TRY(ctx.ref_hist.ensure((size_t)nsub * 256 * sizeof(uint32_t)));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.ref_jobs.ptr, jd.data(), nsub * sizeof(RefJobDev), hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(hipMemsetAsync(ctx.ref_hist.ptr, 0, (size_t)nsub * 256 * sizeof(uint32_t), s));
-    uint64_t hb = (max_n / 16 + 255) / 256;
-    hb = std::max<uint64_t>(1, std::min<uint64_t>(hb, 256));
-    for (uint32_t j0 = 0; j0 < nsub; j0 += 65535) {
-      const uint32_t cnt = std::min<uint32_t>(65535, nsub - j0);
-      hipLaunchKernelGGL(ref_hist_kernel, dim3((uint32_t)hb, cnt), dim3(256), 0, s,
-                         static_cast<const RefJobDev*>(ctx.ref_jobs.ptr) + j0,
-                         static_cast<uint32_t*>(ctx.ref_hist.ptr) + 256ull * j0);
-      PTWM_HIP_TRY(hipGetLastError());
-    }
-    PTWM_HIP_TRY(hipMemcpyAsync(seg_hist.data(), ctx.ref_hist.ptr, seg_hist.size() * 4, hipMemcpyDeviceToHost, s));
-    PTWM_HIP_TRY(hipStreamSynchronize(s));
-  }
-  std::vector<uint32_t> hist((size_t)nj * 256, 0);
-  for (uint32_t j = 0; j < nj; ++j)
-    if (jobs[j].n)
-      for (int i = 0; i < 4; ++i)
-        for (int b = 0; b < 256; ++b) hist[256ull * j + b] += seg_hist[256ull * (sub0[j] + i) + b];
-  // ---- 2. tables; segments ----
-  huf_codes_.assign((size_t)nj * 256, 0);
-  rans_tab_.assign((size_t)nj * 256 * 4, 0);
-  uint64_t scratch_words = 0, rans_scratch = 0;
-  for (uint32_t j = 0; j < nj; ++j) {
     JobInfo& I = info_[j];
-    const uint64_t n = jobs[j].n;
     I.raw = true;
+    const uint64_t n = jobs[j].n;
     if (n == 0) continue;
-    const uint32_t* h = &hist[256ull * j];
-    if (jobs[j].codec == kCodecHuffman) {
-      uint8_t lengths[256];
-      uint16_t rev[256];
-      if (!huf_lengths_from_freqs(h, lengths) || !huf_canonical(lengths, rev)) continue;
-      uint8_t w[140];
-      const int wl = huf_encode_weights(lengths, w);
-      if (wl < 0) continue;
-      I.header.assign(w, w + wl);
-      for (int sy = 0; sy < 256; ++sy) huf_codes_[256ull * j + sy] = ((uint32_t)lengths[sy] << 16) | rev[sy];
-    } else {
-      uint16_t f[256], cum[256];
-      int max_sym = 0;
-      if (!rans_normalize_freqs(h, f, cum, &max_sym)) continue;
-      I.header.push_back((uint8_t)max_sym);
-      for (int i = 0; i <= max_sym; ++i) {
-        I.header.push_back((uint8_t)f[i]);
-        I.header.push_back((uint8_t)(f[i] >> 8));
-      }
-      for (int sy = 0; sy < 256; ++sy) rans_encsym(cum[sy], f[sy], &rans_tab_[(256ull * j + sy) * 4]);
-    }
-    I.raw = false;
+    const bool rans = jobs[j].codec == kCodecRans;
+    tj[j] = TableJob{rans ? kTableRans : kTableHuffman, (uint32_t)jd.size(), 4, 0};
     uint64_t st[4], sn[4];
     split_four(n, st, sn);
+    I.raw = false;
     I.seg0 = (uint32_t)segs_.size();
     for (int i = 0; i < 4; ++i) {
+      jd.push_back(RefJobDev{jobs[j].src + st[i], sn[i]});
       RefSegDev g{};
       g.src = jobs[j].src + st[i];
       g.n = sn[i];
       g.table = j;
-      if (jobs[j].codec == kCodecRans) {
+      if (rans) {
         g.scratch_byte = rans_scratch;
         rans_scratch = align_up(rans_scratch + 4 + 2 * sn[i] + kRansEncSlack, 16);
+        ridx.push_back((uint32_t)segs_.size());
+        rsegs.push_back(g);
       }
       segs_.push_back(g);
     }
+    max_n = std::max(max_n, sn[0]);
   }
-  const uint32_t ns = (uint32_t)segs_.size();
+  const uint32_t ns = (uint32_t)segs_.size(), nr = (uint32_t)rsegs.size();
   seg_len_.assign(ns, 0);
   if (ns) {
-    PTWM_HIP_TRY(ctx.ref_segs.ensure(ns * sizeof(RefSegDev)));
-    PTWM_HIP_TRY(ctx.ref_seglen.ensure(ns * sizeof(unsigned long long)));
-    PTWM_HIP_TRY(ctx.ref_codes.ensure(huf_codes_.size() * 4));
-    PTWM_HIP_TRY(ctx.ref_rans_tab.ensure(rans_tab_.size() * 4));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.ref_segs.ptr, segs_.data(), ns * sizeof(RefSegDev), hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.ref_codes.ptr, huf_codes_.data(), huf_codes_.size() * 4, hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(
-        hipMemcpyAsync(ctx.ref_rans_tab.ptr, rans_tab_.data(), rans_tab_.size() * 4, hipMemcpyHostToDevice, s));
-    // ---- 3. Huffman bits per segment (its histogram x code lengths); rANS segments encoded ----
-    std::vector<unsigned long long> bits(ns, 0);
-    for (uint32_t g = 0; g < ns; ++g) {
-      const uint32_t j = segs_[g].table;
-      if (jobs[j].codec != kCodecHuffman) continue;
-      const uint32_t* h = &seg_hist[256ull * (sub0[j] + (g - info_[j].seg0))];
-      for (int b = 0; b < 256; ++b) bits[g] += (unsigned long long)h[b] * (huf_codes_[256ull * j + b] >> 16);
-    }
-    // the rANS kernel gets the rANS segments only (a Huffman job's rANS
-    // table row is empty)
-    std::vector<RefSegDev> rsegs;
-    std::vector<uint32_t> ridx;
-    for (uint32_t g = 0; g < ns; ++g)
-      if (jobs[segs_[g].table].codec == kCodecRans) {
-        rsegs.push_back(segs_[g]);
-        ridx.push_back(g);
-      }
-    const uint32_t nr = (uint32_t)rsegs.size();
-    std::vector<unsigned long long> rlen(nr, 0);
+    const size_t b_jd = ns * sizeof(RefJobDev), b_tj = nj * sizeof(TableJob), b_rs = nr * sizeof(RefSegDev);
+    PTWM_HIP_TRY(ctx.ref_jobs.ensure(b_jd + b_tj + b_rs));
+    PTWM_HIP_TRY(ctx.h_ref.ensure(b_jd + b_tj + b_rs));
+    PTWM_HIP_TRY(ctx.ref_hist.ensure((size_t)ns * 256 * sizeof(uint32_t)));
+    PTWM_HIP_TRY(ctx.ref_codes.ensure((size_t)nj * 256 * sizeof(uint32_t)));
+    PTWM_HIP_TRY(ctx.h_tables.ensure(nj * sizeof(TableInfo) + nr * sizeof(unsigned long long)));
     if (nr) {
+      PTWM_HIP_TRY(ctx.ref_rans_tab.ensure((size_t)nj * 256 * sizeof(uint4)));
       PTWM_HIP_TRY(ctx.ref_rans_scratch.ensure(rans_scratch));
-      PTWM_HIP_TRY(ctx.ref_rans_segs.ensure(nr * sizeof(RefSegDev)));
-      PTWM_HIP_TRY(ctx.ref_rans_len.ensure(nr * sizeof(unsigned long long)));
-      PTWM_HIP_TRY(
-          hipMemcpyAsync(ctx.ref_rans_segs.ptr, rsegs.data(), nr * sizeof(RefSegDev), hipMemcpyHostToDevice, s));
-      hipLaunchKernelGGL(ref_rans_kernel, dim3((nr + kRansEncLanes - 1) / kRansEncLanes), dim3(kRansEncLanes), 0, s,
-                         static_cast<const RefSegDev*>(ctx.ref_rans_segs.ptr), nr,
-                         static_cast<const uint4*>(ctx.ref_rans_tab.ptr),
-                         static_cast<uint8_t*>(ctx.ref_rans_scratch.ptr),
-                         static_cast<unsigned long long*>(ctx.ref_rans_len.ptr));
+    }
+    uint8_t* const h = static_cast<uint8_t*>(ctx.h_ref.ptr);
+    std::memcpy(h, jd.data(), b_jd);
+    std::memcpy(h + b_jd, tj.data(), b_tj);
+    if (nr) std::memcpy(h + b_jd + b_tj, rsegs.data(), b_rs);
+    uint8_t* const d = static_cast<uint8_t*>(ctx.ref_jobs.ptr);
+    TableInfo* const info = static_cast<TableInfo*>(ctx.h_tables.ptr);
+    unsigned long long* const rlen = reinterpret_cast<unsigned long long*>(info + nj);
+    uint32_t* const hist = static_cast<uint32_t*>(ctx.ref_hist.ptr);
+    uint4* const rtab = static_cast<uint4*>(ctx.ref_rans_tab.ptr);
+    PTWM_HIP_TRY(hipMemcpyAsync(d, h, b_jd + b_tj + b_rs, hipMemcpyHostToDevice, s));
+    PTWM_HIP_TRY(hipMemsetAsync(hist, 0, (size_t)ns * 256 * sizeof(uint32_t), s));
+    uint64_t hb = (max_n / 16 + 255) / 256;
+    hb = std::max<uint64_t>(1, std::min<uint64_t>(hb, 256));
+    for (uint32_t j0 = 0; j0 < ns; j0 += 65535) {
+      const uint32_t cnt = std::min<uint32_t>(65535, ns - j0);
+      hipLaunchKernelGGL(ref_hist_kernel, dim3((uint32_t)hb, cnt), dim3(256), 0, s,
+                         reinterpret_cast<const RefJobDev*>(d) + j0, hist + 256ull * j0);
       PTWM_HIP_TRY(hipGetLastError());
-      PTWM_HIP_TRY(hipMemcpyAsync(rlen.data(), ctx.ref_rans_len.ptr, nr * 8, hipMemcpyDeviceToHost, s));
+    }
+    PTWM_HIP_TRY(launch_code_tables(reinterpret_cast<const TableJob*>(d + b_jd), nj, hist,
+                                    static_cast<uint32_t*>(ctx.ref_codes.ptr), rtab, info, s));
+    if (nr) {
+      hipLaunchKernelGGL(ref_rans_kernel, dim3((nr + kRansEncLanes - 1) / kRansEncLanes), dim3(kRansEncLanes), 0, s,
+                         reinterpret_cast<const RefSegDev*>(d + b_jd + b_tj), nr, rtab,
+                         static_cast<uint8_t*>(ctx.ref_rans_scratch.ptr), rlen);
+      PTWM_HIP_TRY(hipGetLastError());
     }
     PTWM_HIP_TRY(hipStreamSynchronize(s));
-    std::vector<unsigned long long> rlen_of(ns, 0);
-    for (uint32_t k = 0; k < nr; ++k) {
-      if (rlen[k] < 4) return kInternal;  // every rANS stream holds at least x_final
-      rlen_of[ridx[k]] = rlen[k];
-    }
-    for (uint32_t g = 0; g < ns; ++g) {
-      const RefJob& J = jobs[segs_[g].table];
-      if (J.codec == kCodecHuffman) {
-        seg_len_[g] = (bits[g] + 7) / 8;
-        segs_[g].words = (bits[g] + 31) / 32;
+    for (uint32_t j = 0; j < nj; ++j) {
+      JobInfo& I = info_[j];
+      if (I.raw) continue;
+      const TableInfo& T = info[j];
+      if (!T.ok) {
+        I.raw = true;
+        continue;
+      }
+      I.header.assign(T.head, T.head + T.head_len);
+      if (jobs[j].codec != kCodecHuffman) continue;
+      for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t g = I.seg0 + i;
+        seg_len_[g] = (T.bits[i] + 7) / 8;
+        segs_[g].words = (T.bits[i] + 31) / 32;
         segs_[g].scratch_word = scratch_words;
         scratch_words += segs_[g].words + 1;
-      } else {
-        seg_len_[g] = rlen_of[g];
       }
+    }
+    for (uint32_t k = 0; k < nr; ++k) {
+      const uint32_t g = ridx[k];
+      if (info_[segs_[g].table].raw) continue;
+      if (rlen[k] < 4) return kInternal;  // every rANS stream holds at least x_final
+      seg_len_[g] = rlen[k];
     }
   }
   pack_words_ = scratch_words;

@@ -88,8 +88,11 @@ struct DevCtx {
   DeviceBuffer ilv_args, ilv_realign, realign_jobs;
   PinnedBuffer h_realign;
   // reference-format (Huffman / rANS) encoder scratch
-  DeviceBuffer ref_jobs, ref_hist, ref_segs, ref_seglen, ref_codes, ref_rans_tab, ref_rans_segs, ref_rans_scratch,
-      ref_rans_len, ref_hdr, ref_pack, ref_ops;
+  DeviceBuffer ref_jobs, ref_hist, ref_segs, ref_seglen, ref_codes, ref_rans_tab, ref_rans_scratch, ref_hdr, ref_pack,
+      ref_ops;
+  PinnedBuffer h_ref;
+  // what the encoders' table builds tell the host (TableInfo, host-coherent)
+  PinnedBuffer h_tables;
   PinnedBuffer h_enc, h_ilv;
   // fused-decode status words, written by the kernels (host-coherent)
   PinnedBuffer h_ilv_status;

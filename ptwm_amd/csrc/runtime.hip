@@ -125,6 +125,7 @@ DevCtx* get_ctx(uint32_t ord) {
   ctx->h_ilv_status.flags = hipHostMallocCoherent;
   ctx->h_job_status.flags = hipHostMallocCoherent;
   ctx->h_crc.flags = hipHostMallocCoherent;
+  ctx->h_tables.flags = hipHostMallocCoherent;
   // the allocation-free decode's scratch on this device (the device is
   // current): its address, or null, and the entry point then reports
   // MissingCapability
