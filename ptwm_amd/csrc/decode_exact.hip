@@ -34,14 +34,15 @@ constexpr uint32_t kRansProbBits = 11;
 constexpr uint32_t kRansScale = 1u << kRansProbBits;
 constexpr uint32_t kRansL = 1u << 23;
 // rANS stream bytes reach the four chains through one LDS ring per chain:
-// kRansRing bytes (a power of two) plus a copy of its first granule after
-// its end, so that the byte after the ring's last one is read at the next
-// address.  Each round the wavefront stages up to kRansStageGranules
-// 16-byte granules per chain (global loads issued before the round's decode
-// and written to the rings after it) and every chain decodes up to
-// kRansRound symbols from what is staged.
+// kRansRing bytes (a power of two) plus a copy of its first kRansRingPad
+// bytes after its end, so that a round's reads run on past the ring's last
+// byte without a wrap.  Each round the wavefront stages up to
+// kRansStageGranules 16-byte granules per chain (global loads issued before
+// the round's decode and written to the rings after it) and every chain
+// decodes up to kRansRound symbols from what is staged.
 constexpr uint32_t kRansRing = 2048;
-constexpr uint32_t kRansRingPad = 16;
+constexpr uint32_t kRansRingPad = 528;        // a round's 512 bytes and a word read at their end
+constexpr uint32_t kAtMask = 8 * (2 * kRansScale - 1);  // an entry's byte address
 constexpr uint32_t kRansStageGranules = 32;   // 2 per lane: 512 bytes per chain per round
 constexpr uint32_t kRansRound = 256;          // <= 2 bytes per symbol: 512 bytes per chain
 constexpr uint32_t kTansStageWords = 1024;    // tANS stream words staged at a time (4 KiB)
@@ -261,12 +262,11 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
   __shared__ SharedHeader h;
   __shared__ uint16_t rev[256];
   __shared__ uint8_t sorted_sym[256];              // Huffman: symbols by (length, symbol)
-  // rANS: {freq | sym << 24, slot - start} per slot; tANS: one u32 per slot;
-  // Huffman: (len << 8) | sym per window
-  __shared__ __align__(16) uint32_t table_mem[(kRans ? 2 : 1) * kRansScale];
+  // rANS: {2 freq | sym << 24, 2 (slot - start) + bit} per slot and lookahead
+  // bit; Huffman: (len << 8) | sym per window
+  __shared__ __align__(16) uint32_t table_mem[(kRans ? 4 : 1) * kRansScale];
   __shared__ uint8_t hdr_stage[kHdrStage];   // Huffman: weights header and jump table
   uint2* table64 = reinterpret_cast<uint2*>(table_mem);
-  uint32_t* table32 = table_mem;
   uint16_t* table16 = reinterpret_cast<uint16_t*>(table_mem);
 
   const uint32_t lane = threadIdx.x;
@@ -565,13 +565,18 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
     cum[256] = (uint16_t)run;
   }
   __syncthreads();
-  // slot i of symbol s: {freq | s << 24, i - start}, so that one 24-bit
-  // multiply-add, freq * (x >> 11) + (i - start), is the state update
+  // Slot i of symbol s, as entries 2 i and 2 i + 1 for the state y = 2 x + (a
+  // lookahead bit): {2 freq | s << 24, 2 (i - start) + bit}, so that one
+  // 24-bit multiply-add, 2 freq * (y >> 12) + entry.y, is the state update
+  // and keeps the bit.
   for (uint32_t s = lane; s < 256; s += 64) {
-    const uint32_t f = rev[s], st = cum[s];
-    for (uint32_t j = 0; j < f; ++j) table64[st + j] = make_uint2(f | (s << 24), j);
+    const uint32_t f = rev[s], st = 2 * cum[s];
+    for (uint32_t j = 0; j < 2 * f; ++j) table64[st + j] = make_uint2(2 * f | (s << 24), j);
   }
-  // Four lanes run the four serial state chains (decompress.rs:80-111).
+  // The four serial state chains (decompress.rs:80-111).  Chain c runs in
+  // every lane with (lane & 3) == c, the sixteen of them alike and storing
+  // the same bytes: the instructions of a step issue faster with all lanes
+  // active (52 cycles against 63 for eight of them with 16 active).
   __shared__ __align__(16) uint8_t ring[4][kRansRing + kRansRingPad];
   uint64_t s4[4], e4[4];
   split_four(job.dst_len, s4, e4);
@@ -582,7 +587,7 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
   const uint64_t out = reinterpret_cast<uint64_t>(dst);
   uint32_t x = 0, q = 4;  // state; next stream byte to read
   bool good = true, done = true, pending = false;
-  if (lane < 4 && k != end) {
+  if (k != end) {
     if (sl < 4) good = false;
     else {
       const uint8_t* st = enc + h.seg_src[c];
@@ -619,8 +624,8 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
     if (g1 < upto) v1 = g_ld<u32x4>(sgbase + 16ull * g1);
     // decode what is staged: stream bytes [.., avail) of this lane's chain
     const uint32_t sg_mine = (uint32_t)__shfl((int)s_staged, (int)(16 * c), 64);
-    const bool any = __ballot(lane < 4 && !done) != 0;
-    if (lane < 4 && !done) {
+    const bool any = __ballot(!done) != 0;
+    if (!done) {
       const uint32_t avail = sg_mine ? min(16 * sg_mine - my_off, sl) : 0u;
       uint32_t n = 0;
       auto rb = [&](uint32_t o) -> uint32_t { return my_ring[(o + my_off) & (kRansRing - 1)]; };
@@ -636,55 +641,114 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
           if (done || suspend) break;
           pending = false;
         }
-        // Fast stretch: a normalised state (x >= L) decodes to at least
-        // x >> 11 >= 2^12, so at most two bytes renormalise it; with two
-        // staged bytes per step in hand the state stays normalised through
-        // the stretch and needs no checks.  One byte is taken when the
-        // decoded x1 < 2^23, a second when (x1 << 8 | b0) < 2^23, i.e.
-        // x1 < 2^15.
-        if (x >= kRansL) {
+        // Fast stretch: a normalised state (L <= x < 2^31; only a stream's
+        // first state can lie above) decodes to x1 in [2^12, 2^31), so at
+        // most two bytes renormalise it; with two staged bytes per step in
+        // hand the state stays normalised through the stretch and needs no
+        // checks.  The bytes it takes are clz(x1) - 1 (1..18) bits rounded
+        // down to whole bytes.
+        //
+        // A step's time is its serial chain, so that is kept short.  The
+        // state is held as y = 2 x + b, b the top bit of the next stream
+        // byte: clz(y1) is clz(x1) - 1 without the subtraction, and b stays
+        // in place through the update because the table is indexed with it.
+        // The shift by sh | 3 gives the next entry's byte address beside the
+        // state, a mask away.  The chain is then table read, mad, clz,
+        // and-or, 64-bit shift, mask: about 64 cycles for the read and 5 for
+        // each instruction, and all else of a step, some ten instructions,
+        // is issued while the read is under way.  A 16 MiB plane in 256 KiB
+        // chunks, 65536 steps a chain, takes 3.4 ms (4.5 with the state as x
+        // and the other work in the chain).
+        if (x >= kRansL && (int32_t)x >= 0) {
           uint32_t m = min(end - k, kRansRound - n);
           m = min(m, (avail - min(q, avail)) / 2);
-          n += m;
-          // Straight-line step: the bytes renormalising x1 are its leading
-          // zero count rounded down to whole bytes (clz(x1) - 1 in 1..18 for
-          // x1 in [2^12, 2^31)), shifted in from the top of the next two
-          // stream bytes in one 64-bit shift.  qb is the ring read position
-          // in bits.
-          uint32_t qb = 8 * (q + my_off);
-          auto step = [&]() -> uint32_t {
-            const uint32_t idx = x & (kRansScale - 1);
-            const uint2 e = table64[idx];
-            uint16_t b01;
-            __builtin_memcpy(&b01, my_ring + __builtin_amdgcn_ubfe(qb, 3, 11), 2);
-            const uint32_t x1 = __umul24(e.x, x >> kRansProbBits) + e.y;
-            const uint32_t sh = ((uint32_t)__builtin_clz(x1) - 1u) & ~7u;
-            // [b0 b1 0 0] from the top byte down
-            const uint32_t w = __builtin_amdgcn_perm(0u, (uint32_t)b01, 0x00010C0Cu);
-            x = (uint32_t)(((((uint64_t)x1 << 32) | w) << sh) >> 32);
+          if (m) {
+            n += m;
+            const uint32_t p0 = (q + my_off) & (kRansRing - 1);
+            uint32_t qb = 8 * (c * (kRansRing + kRansRingPad) + p0);  // read position in ring[0], in bits
+            const uint32_t q0 = qb;
+            // v << sh: the state y on top, the stream bits after it below;
+            // at: the next entry's byte address
+            uint64_t v = (uint64_t)(2 * x + (my_ring[p0] >> 7)) << 32;
+            uint32_t sh = 0, at = (8 * (2 * x + (my_ring[p0] >> 7))) & kAtMask;
+            // the eight stream bytes from bit position o, first byte on top
+            auto raw = [&](uint32_t o) -> uint64_t {
+              uint64_t r;
+              __builtin_memcpy(&r, &ring[0][0] + (o >> 3), 8);
+              return r;
+            };
+            auto entry = [&]() { return *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(table_mem) + at); };
+            // the step's chain: lo is the stream bits that follow the state
+            auto chain = [&](const uint2 e, uint32_t ys, uint32_t lo) {
+              const uint32_t y1 = __umul24(e.x, ys) + e.y;
+              const uint32_t lead = (uint32_t)__builtin_clz(y1);
+              uint32_t sh3;  // (lead & ~7) | 3 in one instruction, not as sh | 3 after it
+              asm("v_and_or_b32 %0, %1, -8, 3" : "=v"(sh3) : "v"(lead));
+              v = (uint64_t)y1 << 32 | lo;
+              at = (uint32_t)((v << sh3) >> 32) & kAtMask;
+              sh = lead & ~7u;
+            };
+            auto step1 = [&]() -> uint32_t {
+              const uint2 e = entry();
+              const uint32_t ys = (uint32_t)((v << sh) >> 32) >> (kRansProbBits + 1);
+              qb += sh;
+              chain(e, ys, (uint32_t)(__builtin_bswap64(raw(qb)) << 1 >> 32));
+              return e.x;
+            };
+            // single steps up to a 4-byte aligned output address, then whole
+            // output words of four symbols, then single steps
+            for (; m && ((out + k) & 3u); --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step1() >> 24));
+            // Four steps, each: table read, everything that the read's
+            // latency covers, chain.  The stream window is read in the odd
+            // steps, at the position before the step's own shift, and used
+            // in the next: after two steps' shifts and the lookahead bit it
+            // has 31 bits left, of which a step takes at most 16.
+            uint64_t r = raw(qb), w = 0;
+            auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+            uint32_t sym[4];  // the entries of four steps, the symbols in their top bytes
+            auto put = [&](uint32_t at_k) {  // [a3 b3 d3 f3], low byte first
+              g_st<uint32_t>(out + at_k, __builtin_amdgcn_perm(sym[1], sym[0], 0x0C0C0703u) |
+                                             __builtin_amdgcn_perm(sym[3], sym[2], 0x07030C0Cu));
+            };
+            auto four = [&](bool after) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const uint2 e = entry();
+                fence();
+                const uint32_t ys = (uint32_t)((v << sh) >> 32) >> (kRansProbBits + 1);
+                qb += sh;
+                if ((i & 1) == 0) w = __builtin_bswap64(r) << (sh | 1u);
+                else {
+                  w <<= sh;
+                  r = raw(qb);
+                }
+                if (i == 0 && after) put(k - 4);
+                if (i == 3) m -= 4, k += 4;
+                fence();
+                sym[i] = e.x;
+                chain(e, ys, (uint32_t)(w >> 32));
+                fence();
+              }
+            };
+            if (m >= 4) {
+              four(false);
+              while (m >= 4) four(true);
+              put(k - 4);
+            }
+            for (; m; --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step1() >> 24));
             qb += sh;
-            return e.x;
-          };
-          // single steps up to a 4-byte aligned output address, then whole
-          // output words of four symbols, then single steps
-          for (; m && ((out + k) & 3u); --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step() >> 24));
-          for (; m >= 4; m -= 4, k += 4) {
-            // the symbols are the entries' top bytes: [a3 b3 d3 f3], low byte first
-            const uint32_t a = step(), b = step(), d = step(), f = step();
-            const uint32_t w = __builtin_amdgcn_perm(b, a, 0x0C0C0703u) | __builtin_amdgcn_perm(f, d, 0x07030C0Cu);
-            g_st<uint32_t>(out + k, w);
+            const uint32_t y = (uint32_t)((v << sh) >> 32);
+            x = y >> 1;
+            q += (qb - q0) / 8;
           }
-          for (; m; --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step() >> 24));
-          q = qb / 8 - my_off;
         }
         // here pending is false: the last symbol's renormalisation is complete
         if (k == end) { done = true; break; }
         if (n >= kRansRound) break;
         // one careful symbol (unnormalised start, or the staged bytes' end)
-        const uint32_t idx = x & (kRansScale - 1);
-        const uint2 e = table64[idx];
+        const uint2 e = table64[2 * (x & (kRansScale - 1))];
         g_st<uint8_t>(out + k, (uint8_t)(e.x >> 24));
-        x = __umul24(e.x, x >> kRansProbBits) + e.y;
+        x = __umul24((e.x & 0xFFFFFFu) >> 1, x >> kRansProbBits) + (e.y >> 1);
         ++k;
         ++n;
         pending = true;
@@ -695,11 +759,13 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
     // held bytes consumed before the round began)
     if (g0 < upto) {
       *reinterpret_cast<u32x4*>(&ring[sc][(16 * g0) & (kRansRing - 1)]) = v0;
-      if (((16 * g0) & (kRansRing - 1)) == 0) *reinterpret_cast<u32x4*>(&ring[sc][kRansRing]) = v0;
+      if (((16 * g0) & (kRansRing - 1)) < kRansRingPad)
+        *reinterpret_cast<u32x4*>(&ring[sc][kRansRing + ((16 * g0) & (kRansRing - 1))]) = v0;
     }
     if (g1 < upto) {
       *reinterpret_cast<u32x4*>(&ring[sc][(16 * g1) & (kRansRing - 1)]) = v1;
-      if (((16 * g1) & (kRansRing - 1)) == 0) *reinterpret_cast<u32x4*>(&ring[sc][kRansRing]) = v1;
+      if (((16 * g1) & (kRansRing - 1)) < kRansRingPad)
+        *reinterpret_cast<u32x4*>(&ring[sc][kRansRing + ((16 * g1) & (kRansRing - 1))]) = v1;
     }
     s_staged = max(s_staged, upto);
     __syncthreads();

@@ -1,0 +1,85 @@
+"""The reference rANS chains on the device, at the sizes where they can go
+wrong, against the oracle byte for byte: segments around the encoder's 32-step
+batches at any source alignment, alphabets that shed no byte, one and two per
+step, segment counts around a workgroup's sixteen; decode rounds of 256
+symbols and their ends, first states above and below the normalised range, and
+streams whose bytes run out."""
+import numpy as np
+import pytest
+
+import oracle as O
+from ptwm_amd import api, ids
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+SIZES = [1, 3, 4, 5, 31 * 4, 32 * 4, 33 * 4 + 1, 63 * 4 + 3, 65 * 4 + 2, 257 * 4, 1023 * 4 + 3, 3001 * 4 + 2]
+
+
+def symbols(kind, n, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "one":
+        return np.full(n, 200, np.uint8)
+    if kind == "rare":  # frequencies near 1 and near 2^11: two bytes in some steps, none in most
+        return np.where(rng.random(n) < 0.99, 7, rng.integers(0, 256, n)).astype(np.uint8)
+    if kind == "flat":  # every frequency 8: a byte in every step
+        return rng.integers(0, 256, n).astype(np.uint8)
+    return rng.geometric(0.3, n).clip(0, 255).astype(np.uint8)
+
+
+def device(a, offset=0):
+    t = torch.zeros(len(a) + offset + 16, dtype=torch.uint8, device="cuda:0")
+    t[offset:offset + len(a)].copy_(torch.from_numpy(np.array(a, np.uint8)))
+    return t[offset:offset + len(a)]
+
+
+def decode(payload, n):
+    dst = torch.zeros(n, dtype=torch.uint8, device="cuda:0")
+    try:
+        got = api.plane_codec_decode_cuda(ids.PLANE_CODEC_LABEL, "rans", b"", device(np.frombuffer(payload, np.uint8)),
+                                          dst, 0)
+    except Exception:  # noqa: BLE001
+        return None
+    return dst.cpu().numpy().tobytes()[:got]
+
+
+@pytest.mark.parametrize("kind", ["one", "rare", "flat", "geometric"])
+def test_sizes(kind):
+    for k, n in enumerate(SIZES):
+        plane = symbols(kind, n, n)
+        print(kind, n, flush=True)
+        out = torch.zeros(2 * n + 4096, dtype=torch.uint8, device="cuda:0")
+        used = api.plane_codec_encode_cuda(ids.PLANE_CODEC_LABEL, "rans", b"", device(plane, 5 * k % 37), out, 0)
+        want = O.codec_encode(O.CODEC_RANS, plane.tobytes())
+        assert out[:used].cpu().numpy().tobytes() == want
+        assert decode(want, n) == plane.tobytes()
+
+
+@pytest.mark.parametrize("chunks", [1, 4, 5, 17])
+def test_segment_counts(chunks):
+    plane = np.concatenate([symbols("rare" if c % 2 else "geometric", 2100, c) for c in range(chunks)])[:-7]
+    out = torch.zeros(2 * len(plane) + (1 << 16), dtype=torch.uint8, device="cuda:0")
+    used, _ = api.encode_tensor_ref_cuda(6, [O.CODEC_RANS], 2100, device(plane), out, 0)
+    want, _ = O.encode_plane_chunked(O.CODEC_RANS, plane.tobytes(), 2100)
+    assert out[:used].cpu().numpy().tobytes() == want
+
+
+@pytest.mark.parametrize("state", [0, 1, 1 << 11, (1 << 23) - 1, 1 << 23, (1 << 31) - 1, 1 << 31, (1 << 32) - 1])
+@pytest.mark.parametrize("kind", ["one", "rare", "geometric"])
+def test_first_states(kind, state):
+    """Any 32-bit first state and cut or padded streams: accepted or refused as the reference does."""
+    plane = symbols(kind, 5000, 11)
+    good = O.codec_encode(O.CODEC_RANS, plane.tobytes())
+    at = 5 + 1 + 2 * (good[5] + 1)  # the jump table: four lengths, then the streams
+    lens = np.frombuffer(good[at:at + 16], "<u4")
+    for seg in (0, 3):
+        first = at + 16 + int(lens[:seg].sum())
+        bad = bytearray(good)
+        bad[first:first + 4] = int(state).to_bytes(4, "little")
+        for payload in (bytes(bad), bytes(bad[:-1]), bytes(bad) + b"\x5a"):
+            print(kind, state, seg, len(payload), flush=True)
+            try:
+                want = O.codec_decode(O.CODEC_RANS, payload, len(plane))
+            except O.OracleError:
+                want = None
+            assert decode(payload, len(plane)) == want
