@@ -281,15 +281,17 @@ __global__ void __launch_bounds__(kThreads) code_tables_kernel(const TableJob* _
       if (J.kind == kTableRansIlv) {
         codes[256ull * j + t] = f | start << 16;
       } else {
-        // EncSymbol (rans/compress.rs:35-68): {rcp, bias, cmpl | shift << 24, freq << 20}
+        // EncSymbol (rans/compress.rs:35-68): {rcp, bias, cmpl | shift << 24},
+        // and the thresholds that ref_encode.hip's shed takes
         uint4 e;
         if (f < 2) {
-          e = make_uint4(kNone, start + kScale - 1, kScale - f, f << 20);
+          e = make_uint4(kNone, start + kScale - 1, kScale - f, 0u);
         } else {
           const uint32_t sh = 32u - (uint32_t)__builtin_clz(f - 1u);  // 2^sh >= f
           const uint32_t rcp = (uint32_t)(((1ull << (sh + 31)) + f - 1) / f);
-          e = make_uint4(rcp, start, (kScale - f) | (sh - 1) << 24, f << 20);
+          e = make_uint4(rcp, start, (kScale - f) | (sh - 1) << 24, 0u);
         }
+        if (f) e.w = ((f << 4) - 1u) | ((min(f, 8u) << 12) - 1u) << 16;
         rans[256ull * j + t] = e;
       }
       if (t < n_sym) {

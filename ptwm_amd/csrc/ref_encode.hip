@@ -45,6 +45,12 @@ __device__ __forceinline__ uint8_t gbyte(uint64_t a) {
   return *(const __attribute__((address_space(1))) uint8_t*)(uintptr_t)a;
 }
 
+// a word store at any address
+__device__ __forceinline__ void g_st_u32_any(uint64_t a, uint32_t v) {
+  typedef uint32_t __attribute__((aligned(1))) u32_any;
+  *(__attribute__((address_space(1))) u32_any*)(uintptr_t)a = v;
+}
+
 // atomic OR into global memory (not a flat atomic: see g_ld)
 __device__ __forceinline__ void or_global(uint32_t* p, uint32_t v) {
   __hip_atomic_fetch_or((__attribute__((address_space(1))) uint32_t*)(uintptr_t)p, v, __ATOMIC_RELAXED,
@@ -232,139 +238,207 @@ __global__ void __launch_bounds__(256) ref_huf_pack_kernel(const RefSegDev* __re
   }
 }
 
-// rANS: one lane encodes one segment backward (encode_stream_into,
+// rANS: each segment encoded backward (encode_stream_into,
 // rans/compress.rs:140-185) into its scratch area: [x_final u32 LE][renorm
 // bytes in emission order]; seg_len = 4 + renorm bytes.  Table entries per
-// symbol: {rcp, bias, cmpl | shift << 24, freq << 20}.
+// symbol: {rcp, bias, cmpl | shift << 24, the two thresholds} (the
+// thresholds: see shed).
 //
-// The state chain is serial by the format, so a step is kept short:
-// - the segment's symbols arrive as 16-byte aligned blocks, walked from the
-//   last to the first, each loaded four blocks ahead (a step takes exactly
-//   one symbol, so the schedule is fixed; aligned blocks that hold a byte of
-//   the segment never cross a page, so reading them whole is in bounds);
-// - the tables of the workgroup's jobs sit in LDS, and a block's sixteen
-//   entries, which depend on its symbols only, are read before its steps;
-// - x sheds its low byte while x >= freq << 20 (at most twice): both tests
-//   and both shifts run side by side, and the two low bytes of x go to the
-//   lane's LDS output buffer every step (a byte not shed is overwritten by
-//   the next step's); the buffer's whole words go to the scratch after each
-//   block as a fixed nine word stores.
-constexpr uint32_t kRansEncLanes = 64;                    // segments per workgroup
-constexpr uint32_t kRansEncJobs = kRansEncLanes / 4 + 1;  // job tables a workgroup can span
-constexpr uint32_t kRansEncOut = 48;                      // output buffer bytes per lane (3 + 32, words)
-constexpr uint64_t kRansEncSlack = 64;                    // scratch bytes past a segment's stream the flush may write
+// The state chain is serial by the format, and a wavefront issues one
+// instruction per 5.2 cycles whether they depend on each other or not, so
+// the kernel's time is a segment's symbols times the instructions of a step
+// in the wave that holds the states.  That wave (wave 0, one lane per
+// segment) is left with the state alone, eight instructions and one table
+// entry read from a fixed place; the two other waves work beside it on the
+// batches (kRansEncBatch symbols, aligned, last first) before and after:
+// - wave 2 loads the symbols, two batches ahead, and lays their entries in
+//   LDS in the order of the steps (identity entries for positions outside
+//   the segment, which so need no test);
+// - wave 1 takes the states of the batch before and stores the bytes that
+//   they shed (four lanes per segment, each with a quarter of the steps).
+// A workgroup has sixteen segments: with their entries, three batches of
+// 8 KiB, LDS allows three workgroups per CU, and the entry reads and the
+// stores, each lane's at its own address, stay far below the chain's time.
+// A 16 MiB plane in 256 KiB chunks, 65536 steps, takes 2.0 ms: 70 cycles a
+// step, 52 of them the state's (3.3 ms, 122 cycles, with one wave doing all).
+constexpr uint32_t kRansEncSegs = 16;                    // segments per workgroup
+constexpr uint32_t kRansEncJobs = kRansEncSegs / 4 + 1;  // job tables a workgroup can span
+constexpr uint32_t kRansEncBatch = 32;                   // steps
+constexpr uint32_t kRansEncThreads = 192;
 
-__global__ void __launch_bounds__(kRansEncLanes) ref_rans_kernel(const RefSegDev* __restrict__ segs, uint32_t n_segs,
-                                                                 const uint4* __restrict__ tables,
-                                                                 uint8_t* __restrict__ scratch,
-                                                                 unsigned long long* __restrict__ seg_len) {
-  __shared__ uint4 tab[kRansEncJobs][257];  // + the identity entry
-  __shared__ __align__(16) uint8_t obuf[kRansEncLanes * kRansEncOut];
-  const uint32_t s0 = blockIdx.x * kRansEncLanes, lane = threadIdx.x;
-  const uint32_t s = s0 + lane;
-  const uint32_t last = min(n_segs, s0 + kRansEncLanes) - 1;
+// Bytes that state x sheds before the symbol of thresholds th: one if
+// x >= freq << 20 and another if x >= freq << 28.  x is below 2^31 and both
+// thresholds' low 16 bits are zero, so the upper half of x decides, below
+// 2^15: th holds (freq << 4) - 1 and (min(freq, 8) << 12) - 1, and the
+// signs of th - (x >> 16) are counted.
+__device__ __forceinline__ uint32_t shed(uint32_t x, uint32_t th) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const u16x2 v = __builtin_bit_cast(u16x2, x);
+  const u16x2 d = __builtin_bit_cast(u16x2, th) - v.yy;
+  return (uint32_t)__builtin_popcount(__builtin_bit_cast(uint32_t, d) & 0x80008000u);
+}
+
+__global__ void __launch_bounds__(kRansEncThreads) ref_rans_kernel(const RefSegDev* __restrict__ segs, uint32_t n_segs,
+                                                                   const u32x4* __restrict__ tables,
+                                                                   uint8_t* __restrict__ scratch,
+                                                                   unsigned long long* __restrict__ seg_len) {
+  constexpr uint32_t N = kRansEncSegs, B = kRansEncBatch;
+  __shared__ u32x4 tab[kRansEncJobs][257];  // + the identity entry
+  __shared__ u32x4 ent[3][B][N];            // a batch's entries, step by step
+  __shared__ u32x4 state[2][B / 4][N];      // the states before its steps
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t n_here = min(N, n_segs - blockIdx.x * N);
+  const uint32_t g = lane & (N - 1);  // this lane's segment (in waves 1 and 2, with three others)
+  const RefSegDev S = segs[blockIdx.x * N + min(g, n_here - 1)];
   // A job's four segments are consecutive, so the workgroup's segments form
   // runs of one job each (at most kRansEncJobs): run r's table goes to tab[r].
-  const uint32_t job = segs[min(s, last)].table;
-  const uint32_t prev_job = (uint32_t)__shfl_up((int)job, 1, 64);
-  const uint64_t starts = __ballot(lane == 0 || prev_job != job);
-  const uint32_t slot = (uint32_t)__popcll(starts & ((2ull << lane) - 1)) - 1;
+  const uint32_t prev_job = (uint32_t)__shfl((int)S.table, (int)(g ? g - 1 : 0), 64);
+  const uint64_t starts = __ballot(lane < N && (g == 0 || prev_job != S.table));
+  const uint32_t slot = (uint32_t)__popcll(starts & ((2ull << g) - 1)) - 1;
   uint64_t rest = starts;
   for (uint32_t r = 0; rest; ++r) {
     const uint32_t at = (uint32_t)__builtin_ctzll(rest);
     rest &= rest - 1;
-    const uint32_t jr = (uint32_t)__builtin_amdgcn_readlane((int)job, at);
-    for (uint32_t i = lane; i < 256; i += kRansEncLanes) tab[r][i] = tables[256ull * jr + i];
-    // identity: rcp 0, bias 0, cmpl 0, no byte shed below 2^32 - 1
-    if (lane == 0) tab[r][256] = make_uint4(0u, 0u, 0u, 0xFFFFFFFFu);
+    const uint32_t jr = (uint32_t)__builtin_amdgcn_readlane((int)S.table, at);
+    for (uint32_t i = threadIdx.x; i < 256; i += kRansEncThreads) tab[r][i] = tables[256ull * jr + i];
+    // identity: rcp 0, bias 0, cmpl 0, no byte shed
+    if (threadIdx.x == 0) tab[r][256] = u32x4_make(0u, 0u, 0u, 0x7FFF7FFFu);
   }
-  __syncthreads();
-  if (s >= n_segs) return;
-  const RefSegDev S = segs[s];
-  const uint4* const T = tab[slot];
+  // Batch b of the segment: the symbols of the aligned block top - b B.
+  const uint64_t n = g < n_here ? S.n : 0;
+  const uint64_t first = S.src, end = S.src + n;  // symbols [first, end)
+  const uint64_t top = n ? (end - 1) & ~(uint64_t)(B - 1) : 0;
+  const uint64_t count = n ? (top - (first & ~(uint64_t)(B - 1))) / B + 1 : 0;
+  uint64_t batches = count;
+  for (uint32_t d = 1; d < N; d <<= 1) batches = max(batches, (uint64_t)__shfl_xor((unsigned long long)batches, d, 64));
+  batches = (uint64_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)batches) |
+            (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(batches >> 32)) << 32;
   const uint64_t out = reinterpret_cast<uint64_t>(scratch + S.scratch_byte);
-  uint8_t* const ob = obuf + lane * kRansEncOut;
-  uint32_t x = kRansL;
-  uint64_t nb = 4;  // stream bytes stored after x_final
-  uint32_t E = 0;   // bytes in ob
-  if (S.n) {
-    const uint64_t first = S.src, end = S.src + S.n;  // symbols [first, end)
-    const uint64_t b_lo = first & ~15ull;
-    uint64_t blk = (end - 1) & ~15ull;  // block holding the last symbol
-    // one step (rans/compress.rs:150-167)
-    auto step = [&](const uint4 e) {
-      const bool n1 = x >= e.w, n2 = (x >> 8) >= e.w;
-      const uint32_t xs = n2 ? x >> 16 : n1 ? x >> 8 : x;
-      ob[E] = (uint8_t)x;  // byte stores: a 16-bit LDS store needs an even address
-      ob[E + 1] = (uint8_t)(x >> 8);
-      E += (uint32_t)n1 + (uint32_t)n2;
-      const uint32_t q = __umulhi(xs, e.x) >> (e.z >> 24);
-      x = xs + e.y + __umul24(q, e.z);
-    };
-    // One 16-symbol block, last symbol first.  In the segment's first and
-    // last blocks, positions outside the segment take the identity entry.
-    // Every symbol of the data has a nonzero frequency (the table is
-    // normalised from the same bytes' histogram).
-    auto block = [&](const u32x4 v, uint64_t at) {
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      uint4 e[16];
-      if (at >= first && at + 16 <= end) {
+  __syncthreads();  // the tables
+
+  // Wave 2, lane (c, g): symbol words c and c + 4 of the batch's eight.  A
+  // word is read if it holds a symbol of the segment: an aligned word that
+  // holds one byte in bounds is in bounds.
+  const uint32_t c = lane / N;
+  auto word_at = [&](uint64_t b, uint32_t k) { return top - b * B + 4 * k; };
+  auto load = [&](uint64_t b, uint32_t k) -> uint32_t {
+    const uint64_t a = word_at(b, k);
+    return b < count && a < end && a + 4 > first ? g_ld<uint32_t>(a) : 0u;
+  };
+  auto lay = [&](uint64_t b, uint32_t buf, uint32_t k, uint32_t w) {
+    const uint64_t a = word_at(b, k);
+    const u32x4* const T = tab[slot];
+    uint32_t sym[4];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) e[i] = T[(w[i >> 2] >> (8 * (i & 3))) & 0xFFu];
-      } else {
+    for (uint32_t i = 0; i < 4; ++i) sym[i] = (w >> (8 * i)) & 0xFFu;
+    if (!(b < count && a >= first && a + 4 <= end))
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint64_t a = at + (uint64_t)i;
-          e[i] = T[a >= first && a < end ? (w[i >> 2] >> (8 * (i & 3))) & 0xFFu : 256u];
-        }
-      }
+      for (uint32_t i = 0; i < 4; ++i)
+        if (!(b < count && a + i >= first && a + i < end)) sym[i] = 256;
 #pragma unroll
-      for (int i = 15; i >= 0; --i) step(e[i]);
-      // whole words of the buffer to the scratch (nine stores: at most 3 + 32
-      // bytes; words past the last whole one are rewritten by later flushes)
-      const uint32_t* o32 = reinterpret_cast<const uint32_t*>(ob);
-#pragma unroll
-      for (int k = 0; k < 9; ++k) g_st<uint32_t>(out + nb + 4 * k, o32[k]);
-      const uint32_t nd = E >> 2;
-      nb += 4 * nd;
-      *reinterpret_cast<uint32_t*>(ob) = o32[nd];
-      E &= 3;
-    };
-    // four blocks in flight, each slot refilled with the block four below
-    // it; every load is issued (below the segment's first block it reads
-    // that block again) so that the wait before a block's use counts the
-    // loads and stores issued after it
-    auto at_or_lo = [&](uint64_t a) { return a >= b_lo + 64 ? a - 64 : b_lo; };
-    u32x4 r0 = g_ld<u32x4>(blk);
-    u32x4 r1 = g_ld<u32x4>(blk >= b_lo + 16 ? blk - 16 : b_lo);
-    u32x4 r2 = g_ld<u32x4>(blk >= b_lo + 32 ? blk - 32 : b_lo);
-    u32x4 r3 = g_ld<u32x4>(blk >= b_lo + 48 ? blk - 48 : b_lo);
-    for (;;) {
-      block(r0, blk);
-      if (blk == b_lo) break;
-      r0 = g_ld<u32x4>(at_or_lo(blk));
-      blk -= 16;
-      block(r1, blk);
-      if (blk == b_lo) break;
-      r1 = g_ld<u32x4>(at_or_lo(blk));
-      blk -= 16;
-      block(r2, blk);
-      if (blk == b_lo) break;
-      r2 = g_ld<u32x4>(at_or_lo(blk));
-      blk -= 16;
-      block(r3, blk);
-      if (blk == b_lo) break;
-      r3 = g_ld<u32x4>(at_or_lo(blk));
-      blk -= 16;
-    }
+    for (uint32_t i = 0; i < 4; ++i) ent[buf][B - 1 - (4 * k + i)][g] = T[sym[i]];
+  };
+  uint32_t w0 = 0, w1 = 0, v0 = 0, v1 = 0;  // words of the next batch, and of the one after it
+  if (wave == 2) {
+    w0 = load(0, c), w1 = load(0, c + 4);
+    v0 = load(1, c), v1 = load(1, c + 4);
   }
-  for (uint32_t k = 0; k < E; ++k) g_st<uint8_t>(out + nb + k, ob[k]);
-  nb += E;
-  g_st<uint8_t>(out, (uint8_t)x);
-  g_st<uint8_t>(out + 1, (uint8_t)(x >> 8));
-  g_st<uint8_t>(out + 2, (uint8_t)(x >> 16));
-  g_st<uint8_t>(out + 3, (uint8_t)(x >> 24));
-  seg_len[s] = nb;
+  uint32_t x = kRansL;     // wave 0
+  uint32_t last = 0;       // wave 1: the last four bytes of the stream
+  uint64_t pos = out + 4;  //         and its end
+  uint32_t buf = 0;        // b mod 3
+  // Pass b: batch b laid, batch b - 1 coded, batch b - 2 stored.
+  for (uint64_t b = 0; b < batches + 2; ++b) {
+    const uint32_t buf1 = buf == 0 ? 2 : buf - 1, buf2 = buf == 2 ? 0 : buf + 1;  // of b - 1, b - 2
+    if (wave == 2) {
+      const uint32_t n0 = load(b + 2, c), n1 = load(b + 2, c + 4);
+      if (b < batches) {
+        lay(b, buf, c, w0);
+        lay(b, buf, c + 4, w1);
+      }
+      w0 = v0, w1 = v1, v0 = n0, v1 = n1;
+    } else if (wave == 0 && b >= 1 && b <= batches) {
+      // all four lanes of a segment do the same: with 16 active lanes a step
+      // takes 63 cycles, with 64 of them 52
+      const u32x4(*E)[N] = ent[buf1];
+      u32x4(*X)[N] = state[(b - 1) & 1];
+      u32x4 e[8], f[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = E[i][g];
+#pragma unroll
+      for (uint32_t q = 0; q < B / 8; ++q) {
+        // the next eight entries are read in the first four steps, and
+        // waited for once: a wait at each step's entry costs as much as an
+        // instruction
+        asm("" : "+v"(e[0]), "+v"(e[1]), "+v"(e[2]), "+v"(e[3]), "+v"(e[4]), "+v"(e[5]), "+v"(e[6]), "+v"(e[7]));
+        if (q + 1 < B / 8)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f[i] = E[8 * (q + 1) + i][g];
+        uint32_t s[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // one step (rans/compress.rs:150-167)
+          s[i] = x;
+          const uint32_t xs = __builtin_amdgcn_alignbyte(0u, x, shed(x, e[i].w));
+          x = xs + e[i].y + __umul24(__umulhi(xs, e[i].x) >> (e[i].z >> 24), e[i].z);
+        }
+        X[2 * q][g] = u32x4_make(s[0], s[1], s[2], s[3]);
+        X[2 * q + 1][g] = u32x4_make(s[4], s[5], s[6], s[7]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);              // the pk_sub
+          if (i < 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // in the slot after it
+          __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = f[i];
+      }
+    } else if (wave == 1 && b >= 2) {
+      // Lane (c, g): steps 8 c .. 8 c + 7.  What `last` is before each
+      // lane's steps comes from the lanes below; then two steps shed at most
+      // four bytes, those that `last` holds after them, and the word stores
+      // at each two steps' end write right bytes only, also where they
+      // overlap a lower lane's.
+      const u32x4(*E)[N] = ent[buf2];
+      const u32x4(*X)[N] = state[b & 1];
+      const u32x4 xa = X[2 * c][g], xb = X[2 * c + 1][g];
+      const uint32_t s[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+      uint32_t k[8], mine = 0, m = 0;  // bytes shed in the step, by the lane; its last four
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) k[i] = shed(s[i], E[8 * c + i][g].w);
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) {
+        m = __builtin_amdgcn_alignbyte(s[i], m, k[i]);
+        mine += k[i];
+      }
+      uint32_t before = 0, total = 0, l = last;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t nj = (uint32_t)__shfl((int)mine, (int)(N * j + g), 64);
+        const uint32_t mj = (uint32_t)__shfl((int)m, (int)(N * j + g), 64);
+        if (j == c) before = total, last = l;
+        l = mj | (nj < 4 ? l >> (8 * nj) : 0u);
+        total += nj;
+      }
+      uint64_t at = pos + before;
+      pos += total;
+#pragma unroll
+      for (uint32_t i = 0; i < 8; i += 2) {
+        last = __builtin_amdgcn_alignbyte(s[i], last, k[i]);
+        last = __builtin_amdgcn_alignbyte(s[i + 1], last, k[i + 1]);
+        at += k[i] + k[i + 1];
+        if (n) g_st_u32_any(at - 4, last);
+      }
+      last = l;
+    }
+    buf = buf == 2 ? 0 : buf + 1;
+    __syncthreads();
+  }
+  if (wave == 1 && lane < n_here) seg_len[blockIdx.x * N + g] = pos - out;
+  // the stream's first stores reach x_final's bytes too: after them
+  if (wave == 0) state[0][0][g].x = x;
+  __syncthreads();
+  if (wave == 1 && lane < n_here) g_st<uint32_t>(out, state[0][0][g].x);
 }
 
 // Byte copies of a batch of ranges: bytes [0, rev_from) forward, bytes
@@ -443,7 +517,7 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
       g.table = j;
       if (rans) {
         g.scratch_byte = rans_scratch;
-        rans_scratch = align_up(rans_scratch + 4 + 2 * sn[i] + kRansEncSlack, 16);
+        rans_scratch = align_up(rans_scratch + 4 + 2 * sn[i], 16);
         ridx.push_back((uint32_t)segs_.size());
         rsegs.push_back(g);
       }
@@ -486,8 +560,8 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
     PTWM_HIP_TRY(launch_code_tables(reinterpret_cast<const TableJob*>(d + b_jd), nj, hist,
                                     static_cast<uint32_t*>(ctx.ref_codes.ptr), rtab, info, s));
     if (nr) {
-      hipLaunchKernelGGL(ref_rans_kernel, dim3((nr + kRansEncLanes - 1) / kRansEncLanes), dim3(kRansEncLanes), 0, s,
-                         reinterpret_cast<const RefSegDev*>(d + b_jd + b_tj), nr, rtab,
+      hipLaunchKernelGGL(ref_rans_kernel, dim3((nr + kRansEncSegs - 1) / kRansEncSegs), dim3(kRansEncThreads), 0, s,
+                         reinterpret_cast<const RefSegDev*>(d + b_jd + b_tj), nr, reinterpret_cast<const u32x4*>(rtab),
                          static_cast<uint8_t*>(ctx.ref_rans_scratch.ptr), rlen);
       PTWM_HIP_TRY(hipGetLastError());
     }
