@@ -491,14 +491,17 @@ static int64_t encode_tensor_native(uint32_t family, uint32_t chain, uint64_t in
     srcs[i] = reinterpret_cast<uint64_t>(pl[i]);
     lens[i] = plane_len;
   }
-  if (plane_len && launch_split(chain, reinterpret_cast<const uint8_t*>(in_dev_ptr), plane_len, pl, ctx.stream) !=
+  uint32_t* const hist = split_counts(chain) ? ilv_hist_begin(ctx, (uint32_t)np) : nullptr;
+  if (plane_len && launch_split(chain, reinterpret_cast<const uint8_t*>(in_dev_ptr), plane_len, pl, ctx.stream, hist) !=
                        hipSuccess)
     return kInvalidInput;
+  const uint8_t all[4] = {1, 1, 1, 1};
+  const uint8_t* const counted = hist ? all : nullptr;
   IlvEncResult r[4] = {};
   uint64_t needed = 0;
   int64_t rc = family == kFamilyHuff
-                   ? ilv_encode_planes(ctx, srcs, lens, (uint32_t)np, out_dev_ptr, out_cap, true, r, &needed)
-                   : rilv_encode_planes(ctx, srcs, lens, (uint32_t)np, out_dev_ptr, out_cap, true, r, &needed);
+                   ? ilv_encode_planes(ctx, srcs, lens, (uint32_t)np, out_dev_ptr, out_cap, true, r, &needed, counted)
+                   : rilv_encode_planes(ctx, srcs, lens, (uint32_t)np, out_dev_ptr, out_cap, true, r, &needed, counted);
   if (rc == kBufferTooSmall && needed_out) *needed_out = needed;
   if (rc < 0) return rc;
   // decode plan (PTMD v1) for the one tensor
@@ -584,7 +587,12 @@ int64_t ptwm_mi355x_encode_tensors_cuda(uint32_t family, uint32_t n_tensors, con
     }
     PTWM_HIP_TRY(ctx.enc_split.ensure(scratch + 256));
     std::vector<uint64_t> srcs, lens;
+    std::vector<uint8_t> counted;
     uint64_t so = 0;
+    uint32_t planes = 0;
+    for (uint32_t i = b0; i < b1; ++i) planes += (uint32_t)chain_planes(chains[i]);
+    uint32_t* const hist = ilv_hist_begin(ctx, planes);
+    if (!hist) return kInternal;
     for (uint32_t i = b0; i < b1; ++i) {
       const int np = chain_planes(chains[i]);
       const uint64_t pl = in_lens[i] / (uint64_t)chain_ratio(chains[i]);
@@ -595,8 +603,11 @@ int64_t ptwm_mi355x_encode_tensors_cuda(uint32_t family, uint32_t n_tensors, con
         lens.push_back(pl);
         so += (pl + 255) / 256 * 256;
       }
-      if (pl && launch_split(chains[i], reinterpret_cast<const uint8_t*>(in_dev_ptrs[i]), pl, p, ctx.stream) !=
-                    hipSuccess)
+      const size_t row = counted.size();
+      const bool count = split_counts(chains[i]);
+      counted.resize(row + (size_t)np, count);
+      if (pl && launch_split(chains[i], reinterpret_cast<const uint8_t*>(in_dev_ptrs[i]), pl, p, ctx.stream,
+                             count ? hist + 256 * row : nullptr) != hipSuccess)
         return kInvalidInput;
     }
     std::vector<IlvEncResult> r(srcs.size());
@@ -605,9 +616,9 @@ int64_t ptwm_mi355x_encode_tensors_cuda(uint32_t family, uint32_t n_tensors, con
     const uint64_t cap = out_cap > base ? out_cap - base : 0;
     int64_t rc = family == kFamilyHuff
                      ? ilv_encode_planes(ctx, srcs.data(), lens.data(), (uint32_t)srcs.size(), out_dev_ptr + base, cap,
-                                         true, r.data(), &needed)
+                                         true, r.data(), &needed, counted.data())
                      : rilv_encode_planes(ctx, srcs.data(), lens.data(), (uint32_t)srcs.size(), out_dev_ptr + base,
-                                          cap, true, r.data(), &needed);
+                                          cap, true, r.data(), &needed, counted.data());
     if (rc == kBufferTooSmall) {
       // this batch's exact size (the encoder sized it); later batches are
       // only bounded (above)

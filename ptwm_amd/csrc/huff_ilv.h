@@ -65,7 +65,7 @@ struct IlvEncPlane {
   uint64_t src;        // plane bytes (16-byte aligned)
   uint64_t n;
   uint32_t code_slot;  // index of its 256-entry code table
-  uint32_t pad;
+  uint32_t counted;    // its histogram is there already
 };
 
 struct IlvEncBlock {

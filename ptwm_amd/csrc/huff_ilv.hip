@@ -1150,6 +1150,7 @@ __global__ void __launch_bounds__(256) ilv_hist_kernel(const IlvEncPlane* __rest
                                                        uint32_t* __restrict__ hist) {
   __shared__ uint32_t h[256 * kHistStride];
   const IlvEncPlane P = planes[blockIdx.y];
+  if (P.counted) return;
   const uint32_t t = threadIdx.x, copy = t % kHistCopies;
   for (uint32_t i = t; i < 256 * kHistStride; i += 256) h[i] = 0;
   __syncthreads();

@@ -19,9 +19,11 @@ struct IlvEncResult {
 // Encode np planes (16-byte aligned device buffers) into out_dev.  Planes that
 // do not shrink are stored: as Identity payloads when identity_fallback,
 // else as huff_ilv tag-0 payloads.  Returns the bytes used, or
-// kBufferTooSmall with *needed set.
+// kBufferTooSmall with *needed set.  counted[p] != 0: plane p's histogram is
+// row p of ctx.enc_hist already, which ilv_hist_begin made ready.
 int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                          uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed);
+                          uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed,
+                          const uint8_t* counted = nullptr);
 
 // Payload forms of both GPU-native codecs.
 enum IlvForm : uint32_t { kFormStored = 0, kFormCoded = 1, kFormPacked = 2, kFormIdentity = 3 };
@@ -42,15 +44,21 @@ uint32_t ilv_choose_form(uint64_t n, bool nibbles, bool codable, uint64_t coded_
 int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
                          const IlvEncResult* res, const uint32_t* form, std::vector<uint8_t>& keep);
 
+// np rows of 256 zeros in ctx.enc_hist, for counts that the encoders take with
+// `counted`; nullptr on an error.
+uint32_t* ilv_hist_begin(DevCtx& ctx, uint32_t np);
+
 // Histograms and entropy tables (TableKind `kind`) of the planes: the planes
 // to ctx.enc_planes, the tables to ctx.enc_codes; *info: what the host needs
-// of them, valid until the next table build.  Blocks until done.
+// of them, valid until the next table build.  begun: ilv_hist_begin was
+// called for these planes.  Blocks until done.
 int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, uint64_t max_n, uint32_t kind,
-                         const TableInfo** info);
+                         bool begun, const TableInfo** info);
 
 // The same for the rans_ilv codec (rans_host.hip).
 int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                           uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed);
+                           uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed,
+                           const uint8_t* counted = nullptr);
 
 // Decode and merge the given tensors (fused path; each tensor's coded planes
 // are of its codec family).  crc: the sums of the n_acc plane-CRC

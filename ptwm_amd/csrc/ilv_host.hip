@@ -87,13 +87,20 @@ int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, ui
   return kOk;
 }
 
+uint32_t* ilv_hist_begin(DevCtx& ctx, uint32_t np) {
+  const size_t bytes = (size_t)np * 256 * sizeof(uint32_t);
+  if (ctx.enc_hist.ensure(bytes) != hipSuccess || hipMemsetAsync(ctx.enc_hist.ptr, 0, bytes, ctx.stream) != hipSuccess)
+    return nullptr;
+  return static_cast<uint32_t*>(ctx.enc_hist.ptr);
+}
+
 int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, uint64_t max_n, uint32_t kind,
-                         const TableInfo** info) {
+                         bool begun, const TableInfo** info) {
   hipStream_t s = ctx.stream;
   const uint32_t np = (uint32_t)planes.size();
   const size_t b_pl = np * sizeof(IlvEncPlane), b_tj = np * sizeof(TableJob);
   PTWM_HIP_TRY(ctx.enc_planes.ensure(b_pl + b_tj));
-  PTWM_HIP_TRY(ctx.enc_hist.ensure(np * 256 * sizeof(uint32_t)));
+  if (!begun && !ilv_hist_begin(ctx, np)) return kInternal;
   PTWM_HIP_TRY(ctx.enc_codes.ensure(np * 256 * sizeof(uint32_t)));
   PTWM_HIP_TRY(ctx.h_enc.ensure(b_pl + b_tj));
   PTWM_HIP_TRY(ctx.h_tables.ensure(np * sizeof(TableInfo)));
@@ -105,8 +112,8 @@ int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, ui
   uint32_t* const hist = static_cast<uint32_t*>(ctx.enc_hist.ptr);
   TableInfo* const out = static_cast<TableInfo*>(ctx.h_tables.ptr);
   PTWM_HIP_TRY(hipMemcpyAsync(d, h, b_pl + b_tj, hipMemcpyHostToDevice, s));
-  PTWM_HIP_TRY(hipMemsetAsync(hist, 0, np * 256 * sizeof(uint32_t), s));
-  PTWM_HIP_TRY(launch_ilv_hist(reinterpret_cast<const IlvEncPlane*>(d), np, max_n, hist, s));
+  if (!std::all_of(planes.begin(), planes.end(), [](const IlvEncPlane& p) { return p.counted != 0; }))
+    PTWM_HIP_TRY(launch_ilv_hist(reinterpret_cast<const IlvEncPlane*>(d), np, max_n, hist, s));
   PTWM_HIP_TRY(launch_code_tables(reinterpret_cast<const TableJob*>(d + b_pl), np, hist,
                                   static_cast<uint32_t*>(ctx.enc_codes.ptr), nullptr, out, s));
   PTWM_HIP_TRY(hipStreamSynchronize(s));
@@ -115,7 +122,8 @@ int64_t ilv_plane_tables(DevCtx& ctx, const std::vector<IlvEncPlane>& planes, ui
 }
 
 int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                          uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed) {
+                          uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed,
+                          const uint8_t* counted) {
   hipStream_t s = ctx.stream;
   if (np == 0) return 0;
   for (uint32_t p = 0; p < np; ++p)
@@ -123,12 +131,12 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
   std::vector<IlvEncPlane> hp(np);
   uint64_t max_n = 0;
   for (uint32_t p = 0; p < np; ++p) {
-    hp[p] = IlvEncPlane{src[p], n[p], p, 0};
+    hp[p] = IlvEncPlane{src[p], n[p], p, counted ? counted[p] : 0u};
     max_n = std::max(max_n, n[p]);
   }
   // ---- code tables (code_tables.hip) ----
   const TableInfo* info = nullptr;
-  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableIlv, &info); rc != kOk) return rc;
+  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableIlv, counted != nullptr, &info); rc != kOk) return rc;
   std::vector<uint8_t> codable(np, 0);
   for (uint32_t p = 0; p < np; ++p) {
     if (n[p] == 0 || !info[p].ok) continue;

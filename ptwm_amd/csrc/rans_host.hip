@@ -20,7 +20,8 @@ namespace ptwm {
 static inline uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
 int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                           uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed) {
+                           uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed,
+                           const uint8_t* counted) {
   hipStream_t s = ctx.stream;
   if (np == 0) return 0;
   for (uint32_t p = 0; p < np; ++p)
@@ -28,12 +29,12 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   std::vector<IlvEncPlane> hp(np);
   uint64_t max_n = 0;
   for (uint32_t p = 0; p < np; ++p) {
-    hp[p] = IlvEncPlane{src[p], n[p], p, 0};
+    hp[p] = IlvEncPlane{src[p], n[p], p, counted ? counted[p] : 0u};
     max_n = std::max(max_n, n[p]);
   }
   // ---- frequency tables (code_tables.hip): per symbol f | cum << 16 ----
   const TableInfo* info = nullptr;
-  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableRansIlv, &info); rc != kOk) return rc;
+  if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableRansIlv, counted != nullptr, &info); rc != kOk) return rc;
   std::vector<bool> codable(np, false);
   for (uint32_t p = 0; p < np; ++p) codable[p] = n[p] != 0 && info[p].ok;
   // ---- size pass over every block of every codable plane ----

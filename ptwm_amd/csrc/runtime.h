@@ -181,8 +181,11 @@ bool fused_eligible(const PlanTensor& T, uint64_t out_dev);
 // kernel launchers (transform.hip; the decode launchers are in decode_sync.h)
 hipError_t launch_merge(uint32_t chain, const uint8_t* const* planes, uint64_t plane_len, uint8_t* out,
                         hipStream_t stream);
+// hist: also add the planes' histograms there, 256 counts each in order (only
+// where split_counts).
+bool split_counts(uint32_t chain);
 hipError_t launch_split(uint32_t chain, const uint8_t* in, uint64_t plane_len, uint8_t* const* planes,
-                        hipStream_t stream);
+                        hipStream_t stream, uint32_t* hist = nullptr);
 hipError_t launch_copy(const uint8_t* in, uint8_t* out, uint64_t n, hipStream_t stream);
 
 

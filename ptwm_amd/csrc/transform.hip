@@ -8,6 +8,8 @@
 // Semantics follow transforms/fusion.rs (forward :35-94,208-255,329-338,
 // 431-440; inverse :127-194,261-315,376-399,478-501), NibbleSplit
 // (transforms/nibble_split.rs:72-120) and BytePassthrough.
+#include <algorithm>
+
 #include "chain_ops.h"
 #include "ptwm_common.h"
 
@@ -127,9 +129,33 @@ __global__ void __launch_bounds__(256) merge_nibble_kernel(const uint8_t* __rest
 // forward (split): tensor -> planes
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(256) split_ieee16_kernel(const uint8_t* __restrict__ in,
-                                                           uint8_t* __restrict__ p0,
-                                                           uint8_t* __restrict__ p1, uint64_t n) {
+// With kCount the planes' histograms are added to hist (256 counts of p0, then
+// of p1), as ilv_hist_kernel (huff_ilv.hip) counts them: 16 copies per plane
+// and workgroup, copy lane % 16, symbols 17 words apart.  The split is bound by
+// HBM and the counting by LDS atomics, so most of the counting hides here (two
+// bf16 layers of 436 MB: 356 us for the split alone and 220 us for a pass of
+// its own over the planes).  One workgroup of 1024 threads per CU: each ends with
+// 512 atomics on the same words, which cost about 12 ns a workgroup (a 4096 x
+// 4096 tensor: 16.8 us with 256 workgroups, 20.0 with 512 of 512 threads, 26.5
+// with 1024 of them).
+constexpr uint32_t kSplitCopies = 16, kSplitStride = 17;
+
+template <bool kCount>
+__global__ void __launch_bounds__(kCount ? 1024 : 256) split_ieee16_kernel(const uint8_t* __restrict__ in,
+                                                                          uint8_t* __restrict__ p0,
+                                                                          uint8_t* __restrict__ p1, uint64_t n,
+                                                                          uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[kCount ? 2 * 256 * kSplitStride : 1];
+  uint32_t* const h0 = h + threadIdx.x % kSplitCopies;
+  uint32_t* const h1 = h0 + 256 * kSplitStride;
+  if constexpr (kCount) {
+    for (uint32_t i = threadIdx.x; i < 2 * 256 * kSplitStride; i += blockDim.x) h[i] = 0;
+    __syncthreads();
+  }
+  auto count = [&](uint32_t* p, uint32_t w) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) atomicAdd(p + ((w >> (8 * k)) & 0xFFu) * kSplitStride, 1u);
+  };
   const uint64_t nvec = n / 16;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nvec; v += stride) {
@@ -143,6 +169,10 @@ __global__ void __launch_bounds__(256) split_ieee16_kernel(const uint8_t* __rest
     u32x4 a = u32x4_make(a0, a1, a2, a3), b = u32x4_make(b0, b1, b2, b3);
     __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(p0) + v);
     __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(p1) + v);
+    if constexpr (kCount) {
+      count(h0, a0), count(h0, a1), count(h0, a2), count(h0, a3);
+      count(h1, b0), count(h1, b1), count(h1, b2), count(h1, b3);
+    }
   }
   if (blockIdx.x == 0) {
     for (uint64_t i = nvec * 16 + threadIdx.x; i < n; i += blockDim.x) {
@@ -150,7 +180,19 @@ __global__ void __launch_bounds__(256) split_ieee16_kernel(const uint8_t* __rest
       uint32_t r = reorder16x2(v);
       p0[i] = (uint8_t)r;
       p1[i] = (uint8_t)(r >> 8);
+      if constexpr (kCount) {
+        atomicAdd(h0 + (r & 0xFFu) * kSplitStride, 1u);
+        atomicAdd(h1 + ((r >> 8) & 0xFFu) * kSplitStride, 1u);
+      }
     }
+  }
+  if constexpr (kCount) {
+    __syncthreads();
+    if (threadIdx.x >= 512) return;
+    uint32_t sum = 0;  // thread t: count t of the 512
+#pragma unroll
+    for (uint32_t c = 0; c < kSplitCopies; ++c) sum += h[threadIdx.x * kSplitStride + c];
+    if (sum) atomicAdd(hist + threadIdx.x, sum);
   }
 }
 
@@ -280,8 +322,10 @@ hipError_t launch_merge(uint32_t chain, const uint8_t* const* planes, uint64_t p
   return hipGetLastError();
 }
 
+bool split_counts(uint32_t chain) { return chain == kChainIeee16Split2; }
+
 hipError_t launch_split(uint32_t chain, const uint8_t* in, uint64_t plane_len, uint8_t* const* planes,
-                        hipStream_t stream) {
+                        hipStream_t stream, uint32_t* hist) {
   const uint64_t nvec = plane_len / 16;
   dim3 grid = stream_grid(nvec), block(256);
   bool al = aligned16(in);
@@ -290,7 +334,12 @@ hipError_t launch_split(uint32_t chain, const uint8_t* in, uint64_t plane_len, u
   if (!al) return hipErrorInvalidValue;
   switch (chain) {
     case kChainIeee16Split2:
-      hipLaunchKernelGGL(split_ieee16_kernel, grid, block, 0, stream, in, planes[0], planes[1], plane_len);
+      if (hist)
+        hipLaunchKernelGGL(split_ieee16_kernel<true>, dim3((uint32_t)std::clamp<uint64_t>((nvec + 1023) / 1024, 1, 256)),
+                           dim3(1024), 0, stream, in, planes[0], planes[1], plane_len, hist);
+      else
+        hipLaunchKernelGGL(split_ieee16_kernel<false>, grid, block, 0, stream, in, planes[0], planes[1], plane_len,
+                           nullptr);
       break;
     case kChainIeee32Split4:
       hipLaunchKernelGGL(split_ieee32_kernel, grid, block, 0, stream, in, planes[0], planes[1], planes[2],
