@@ -248,15 +248,13 @@ def build_workload(name: str, resident: bool = False, integrity: bool = False) -
 
 
 def kernel_label(wl, crc: bool) -> str:
-    """The dominant kernel's name for a plan variant: huff_ilv kernels carry a
-    second template argument, plane CRC-32 computed in the decode (bf16, fp32
-    and passthrough chains)."""
+    """The dominant kernel's name for a plan variant: the fused kernels carry a
+    second template argument, plane CRC-32 computed in the decode."""
     k = wl.kernel
-    if k == EXACT_ROUTE or k.startswith("rilv"):
+    if k == EXACT_ROUTE:
         return k
-    fused = crc and any(t.chain in (1, 2, 6) for t in wl.plans)
-    k = re.sub(r"<(\d|0x[0-9a-f]+)>", lambda m: f"<{m.group(1)}, {'true' if fused else 'false'}>", k)
-    return k + (" + plane CRC-32 fused" if fused else "")
+    k = re.sub(r"<(\d|0x[0-9a-f]+)>", lambda m: f"<{m.group(1)}, {'true' if crc else 'false'}>", k)
+    return k + (" + plane CRC-32 fused" if crc else "")
 
 
 def np_prod(shape):

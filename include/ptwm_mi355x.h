@@ -105,9 +105,9 @@ int64_t ptwm_hardware_backend_v1_dispatch_decode_cuda(uint8_t state_format_versi
  * payloads (one codec per tensor, at least one coded plane, 4-byte aligned
  * in the input) or unchunked Identity planes, output 16-byte aligned, plane
  * CRC-32 only for the ieee16 / ieee32 / passthrough chains, no tensor XXH64.
- * All device scratch (descriptors, CRC tables and block partials) is one
+ * All device scratch (descriptors, CRC tables and sums) is one
  * fixed array of PTWM_MI355X_NOALLOC_SCRATCH_BYTES per device, and the
- * per-tensor status words a fixed 16 KiB host-coherent pinned area; both
+ * status words and CRC results a fixed host-coherent pinned area; both
  * are set up by ptwm_mi355x_device_init (the device's context: its stream,
  * the array's address, the status area), which the caller runs once per
  * device beforehand, and are held until the process ends.  The call itself

@@ -28,8 +28,8 @@
 // persistent: each takes a contiguous range of 4-block tiles and rebuilds
 // its tables only when the range crosses into the next tensor.
 //
-// Encode: LDS-privatised histograms merged with atomics, host code-table
-// build (256 symbols), a size pass (one wave per block: per-lane bit counts
+// Encode: LDS-privatised histograms merged with atomics, code tables
+// (code_tables.hip), a size pass (one wave per block: per-lane bit counts
 // from the code lengths), a host prefix sum for block offsets, and an encode
 // pass that writes each lane's words at its prefix-summed offset.
 #include "huff_ilv.h"

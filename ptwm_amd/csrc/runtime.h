@@ -174,8 +174,7 @@ int64_t execute_plan_noalloc(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uin
 
 // Whether the tensor is restored by the fused decode kernel (every plane an
 // unchunked GPU-native payload of one codec family or a stored Identity
-// plane, at least one coded, 16-byte aligned output, and a plane CRC only
-// for the chains the fused CRC covers).
+// plane, at least one coded, and 16-byte aligned output).
 bool fused_eligible(const PlanTensor& T, uint64_t out_dev);
 
 // kernel launchers (transform.hip; the decode launchers are in decode_sync.h)

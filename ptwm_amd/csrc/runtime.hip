@@ -330,8 +330,8 @@ int64_t chunk_ranges(DevCtx& ctx, const Plan& plan, uint64_t in_dev, ChunkRanges
 // family with the same chunk boundaries, every chunk but the last a whole
 // number of 16384-symbol blocks, decodes in the fused route as one
 // sub-tensor per chunk: chunk k of every plane restores elements
-// [a_k, a_k + size_k) straight into the output, and the CRC block partials
-// of the sub-tensors follow each other as those of the whole tensor would.
+// [a_k, a_k + size_k) straight into the output, and each
+// block's CRC is weighted by its place in the whole plane.
 bool chunked_fused_eligible(const PlanTensor& T, uint64_t out_dev, const ChunkRanges& cr, size_t t) {
   if (cr.r[t].empty() || ((out_dev + T.out_offset) & 15u)) return false;
   bool any_huff = false, any_rans = false;
