@@ -657,7 +657,7 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
         // and-or, 64-bit shift, mask: about 64 cycles for the read and 5 for
         // each instruction, and all else of a step, some ten instructions,
         // is issued while the read is under way.  A 16 MiB plane in 256 KiB
-        // chunks, 65536 steps a chain, takes 3.4 ms (4.5 with the state as x
+        // chunks, 65536 steps a chain, takes 3.5 ms (4.5 with the state as x
         // and the other work in the chain).
         if (x >= kRansL && (int32_t)x >= 0) {
           uint32_t m = min(end - k, kRansRound - n);
