@@ -27,7 +27,7 @@ struct alignas(16) TableInfo {
   uint32_t n_sym;     // last symbol with a nonzero count, plus one
   uint32_t head_len;  // bytes of `head`
   uint32_t pad;
-  uint64_t bits[4];   // Huffman: code bits of each row
+  uint64_t bits[4];   // Huffman: code bits of each row; kTableRansIlv: [0], rans_ilv_least
   uint8_t head[528];  // the payload's table header (weights, or max_sym and frequencies)
 };
 

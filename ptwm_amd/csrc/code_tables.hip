@@ -280,6 +280,9 @@ __global__ void __launch_bounds__(kThreads) code_tables_kernel(const TableJob* _
       if (t >= n_sym) start = 0;
       if (J.kind == kTableRansIlv) {
         codes[256ull * j + t] = f | start << 16;
+        const double gain = 11.0 - log2((double)max(f, 1u)) - 2.25e-5 * f;  // rans_ilv_least
+        const uint64_t bits = sum_all(S, (uint64_t)((double)h * (gain > 0 ? gain : 0)));
+        if (t == 0) I.bits[0] = bits;
       } else {
         // EncSymbol (rans/compress.rs:35-68): {rcp, bias, cmpl | shift << 24},
         // and the thresholds that ref_encode.hip's shed takes

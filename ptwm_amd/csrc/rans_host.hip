@@ -19,6 +19,17 @@ namespace ptwm {
 
 static inline uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
+// A lower bound of the coded payload's bytes, from `bits`, the sum over the
+// symbols of 11 - log2 f - 2.25e-5 f.  A lane's state x lies in [2^16, 2^32)
+// and a step multiplies it by 2^11 / f, except that rounding x / f down loses
+// a factor of at most 1 + f / x: 2.25e-5 f bits at x >= 2^16, and where a word
+// left just before, log2(33 / 32) (x >= 32 f) twice, as the shift rounds too.
+// So each lane of a block sheds at least (its bits - 16) / 16.0888 words.
+static uint64_t rans_ilv_least(uint64_t bits, uint64_t n_blocks, uint32_t head_len) {
+  const double words = std::max(0.0, ((double)bits - 1024.0 * (double)n_blocks) / 16.1);
+  return align_up(5 + (uint64_t)head_len, 4) + 4 * (n_blocks + 1) + kRilvBlockHead * n_blocks + (uint64_t)(2.0 * words);
+}
+
 int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
                            uint64_t out_cap, bool identity_fallback, IlvEncResult* res, uint64_t* needed,
                            const uint8_t* counted) {
@@ -36,7 +47,19 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   const TableInfo* info = nullptr;
   if (int64_t rc = ilv_plane_tables(ctx, hp, max_n, kTableRansIlv, counted != nullptr, &info); rc != kOk) return rc;
   std::vector<bool> codable(np, false);
-  for (uint32_t p = 0; p < np; ++p) codable[p] = n[p] != 0 && info[p].ok;
+  for (uint32_t p = 0; p < np; ++p) {
+    if (n[p] == 0 || !info[p].ok) continue;
+    // a plane whose coded payload cannot be shorter than the stored or packed
+    // one is not sized: ilv_choose_form would not take it, and the size pass
+    // is a whole run of the encoder.  The 11-bit frequencies of a plane of
+    // mantissa bytes cost more than 8 bits a symbol, so these planes end
+    // here (two bf16 layers, 872 MB: 1763 to 1453 us; MXFP4 14336x2048: 281 to
+    // 243 us)
+    const uint64_t nb = (n[p] + kIlvBlock - 1) / kIlvBlock;
+    const uint64_t stored = n[p] + 1, packed = kPackedHeadBytes + (n[p] + 1) / 2;
+    const uint64_t other = info[p].n_sym <= 16 && packed < stored ? packed : stored;
+    codable[p] = rans_ilv_least(info[p].bits[0], nb, info[p].head_len) < other;
+  }
   // ---- size pass over every block of every codable plane ----
   std::vector<RilvEncBlock> blocks;
   std::vector<uint32_t> first_block(np, 0), nbs(np, 0);
