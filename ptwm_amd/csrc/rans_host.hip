@@ -2,9 +2,11 @@
 //
 // Per call, any number of planes: histogram kernel and frequency tables
 // (ilv_plane_tables, shared with huff_ilv) -> size kernel (word counts per
-// block) -> host layout and header / offset-table uploads -> write kernel.  Each plane takes the smallest payload form
-// (ilv_choose_form): coded, packed nibbles or stored.  Decode runs through ilv_decode_tensors (family
-// kFamilyRans).
+// block, and the words of the first kRilvKeepBlocks) -> host layout and header
+// / offset-table uploads -> the blocks copied to their places, or encoded
+// again past kRilvKeepBlocks.  Each plane takes the smallest payload form
+// (ilv_choose_form): coded, packed nibbles or stored.  Decode runs through
+// ilv_decode_tensors (family kFamilyRans).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -16,6 +18,11 @@
 #include "runtime.h"
 
 namespace ptwm {
+
+// Blocks whose words the size pass keeps: 1 GiB of scratch at most, which is
+// 512 MiB of planes.  Blocks past them, and all where the scratch cannot be
+// had, are encoded twice.
+constexpr uint32_t kRilvKeepBlocks = 32 << 10;
 
 static inline uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
@@ -67,19 +74,25 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     first_block[p] = (uint32_t)blocks.size();
     if (!codable[p]) continue;
     nbs[p] = (uint32_t)((n[p] + kIlvBlock - 1) / kIlvBlock);
-    for (uint32_t b = 0; b < nbs[p]; ++b) blocks.push_back(RilvEncBlock{0, p, b});
+    for (uint32_t b = 0; b < nbs[p]; ++b) blocks.push_back(RilvEncBlock{0, p, b, (uint32_t)blocks.size(), 0});
   }
   const uint32_t nblk = (uint32_t)blocks.size();
   std::vector<uint32_t> bwords(nblk);
+  uint32_t kept = std::min(nblk, kRilvKeepBlocks);
+  if (kept && ctx.enc_keep.ensure(kept * kRilvKeepBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    kept = 0;
+  }
   if (nblk) {
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(RilvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_block_bytes.ensure(nblk * sizeof(uint32_t)));
     PTWM_HIP_TRY(
         hipMemcpyAsync(ctx.enc_blocks.ptr, blocks.data(), nblk * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
     PTWM_HIP_TRY(launch_rilv_size(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
-                                  static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr), nblk,
+                                  static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr), nblk, kept,
                                   static_cast<const uint32_t*>(ctx.enc_codes.ptr),
-                                  static_cast<uint32_t*>(ctx.enc_block_bytes.ptr), s));
+                                  static_cast<uint32_t*>(ctx.enc_block_bytes.ptr),
+                                  static_cast<uint8_t*>(ctx.enc_keep.ptr), s));
     PTWM_HIP_TRY(hipMemcpyAsync(bwords.data(), ctx.enc_block_bytes.ptr, nblk * 4, hipMemcpyDeviceToHost, s));
     PTWM_HIP_TRY(hipStreamSynchronize(s));
   }
@@ -116,7 +129,6 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   if (int64_t rc = ilv_store_planes(ctx, src, n, np, out_dev, res, form.data(), keep); rc != kOk) return rc;
   std::vector<std::vector<uint8_t>> hbufs(np);
   std::vector<RilvEncBlock> live;
-  std::vector<uint32_t> lw;
   for (uint32_t p = 0; p < np; ++p) {
     const uint64_t dst = out_dev + res[p].offset;
     if (!res[p].coded) continue;
@@ -140,16 +152,16 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     PTWM_HIP_TRY(hipMemcpyAsync(reinterpret_cast<void*>(dst), hbuf.data(), hbuf.size(), hipMemcpyHostToDevice, s));
   }
   if (!live.empty()) {
-    // block word counts in the order of `live`
-    for (const RilvEncBlock& bk : live) lw.push_back(bwords[first_block[bk.plane] + bk.block]);
-    PTWM_HIP_TRY(ctx.enc_lane_words.ensure(lw.size() * 4));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_lane_words.ptr, lw.data(), lw.size() * 4, hipMemcpyHostToDevice, s));
+    const RilvEncBlock* const bd = static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr);
+    const uint32_t* const words = static_cast<const uint32_t*>(ctx.enc_block_bytes.ptr);
+    uint32_t n_kept = 0;  // rows rise along `live`
+    while (n_kept < live.size() && live[n_kept].row < kept) ++n_kept;
     PTWM_HIP_TRY(
         hipMemcpyAsync(ctx.enc_blocks.ptr, live.data(), live.size() * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(launch_rilv_encode(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
-                                    static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr), (uint32_t)live.size(),
-                                    static_cast<const uint32_t*>(ctx.enc_codes.ptr),
-                                    static_cast<const uint32_t*>(ctx.enc_lane_words.ptr), s));
+    PTWM_HIP_TRY(launch_rilv_place(bd, n_kept, words, static_cast<const uint8_t*>(ctx.enc_keep.ptr), s));
+    PTWM_HIP_TRY(launch_rilv_encode(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr), bd + n_kept,
+                                    (uint32_t)live.size() - n_kept, static_cast<const uint32_t*>(ctx.enc_codes.ptr),
+                                    words, s));
   }
   PTWM_HIP_TRY(hipStreamSynchronize(s));
   return (int64_t)total;

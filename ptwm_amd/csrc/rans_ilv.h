@@ -25,7 +25,14 @@ struct RilvEncBlock {
   uint64_t dst;     // device address of the block (nw first)
   uint32_t plane;   // index into the IlvEncPlane array
   uint32_t block;   // block index within the plane
+  uint32_t row;     // the size pass's index of the block
+  uint32_t pad;
 };
+
+// What the size pass keeps of its block i, for i below the `kept` it is
+// given: the emitted words at the end of 16384 of them, and the lanes' final
+// states.
+constexpr uint64_t kRilvKeepBytes = 2ull * kIlvBlock + 256;
 
 // Fused decode of the tensors tix[0..m) (indexes into `tensors`, all of
 // chain `chain`, coded planes rans_ilv).  Same tiling and persistence as
@@ -38,9 +45,13 @@ hipError_t launch_rilv_decode(uint32_t chain, const IlvTensor* tensors, const ui
 size_t rilv_decode_lds_bytes(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc);
 hipError_t rilv_decode_occupancy(uint32_t chain, uint32_t n_slots, uint32_t stage_words, bool crc, int* wg_per_cu);
 
-// Encoder passes over blocks: word counts (block_words[i]), then the blocks.
-hipError_t launch_rilv_size(const IlvEncPlane* planes, const RilvEncBlock* blocks, uint32_t n_blocks,
-                            const uint32_t* syms, uint32_t* block_words, hipStream_t stream);
+// Encoder passes over blocks: word counts (block_words[i]) of all and what
+// the first `kept` of them encode to (keep); then the blocks, copied from
+// there (launch_rilv_place) or encoded again (launch_rilv_encode).
+hipError_t launch_rilv_size(const IlvEncPlane* planes, const RilvEncBlock* blocks, uint32_t n_blocks, uint32_t kept,
+                            const uint32_t* syms, uint32_t* block_words, uint8_t* keep, hipStream_t stream);
+hipError_t launch_rilv_place(const RilvEncBlock* blocks, uint32_t n_blocks, const uint32_t* block_words,
+                             const uint8_t* keep, hipStream_t stream);
 hipError_t launch_rilv_encode(const IlvEncPlane* planes, const RilvEncBlock* blocks, uint32_t n_blocks,
                               const uint32_t* syms, const uint32_t* block_words, hipStream_t stream);
 

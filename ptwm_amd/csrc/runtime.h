@@ -84,7 +84,8 @@ struct DevCtx {
   PinnedBuffer h_status;
   PinnedBuffer h_small;
   // huff_ilv encoder / decoder scratch
-  DeviceBuffer enc_planes, enc_hist, enc_codes, enc_blocks, enc_lane_words, enc_block_bytes, enc_pack;
+  DeviceBuffer enc_planes, enc_hist, enc_codes, enc_blocks, enc_lane_words, enc_block_bytes, enc_pack,
+      enc_keep;
   DeviceBuffer ilv_args, ilv_realign, realign_jobs;
   PinnedBuffer h_realign;
   // reference-format (Huffman / rANS) encoder scratch

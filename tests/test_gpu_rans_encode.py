@@ -1,16 +1,24 @@
-"""rans_ilv encoder: the payload equals the format specification's (oracle)
-for planes on both sides of the lines between the coded and the packed or
-stored form, which the encoder decides for some of them without sizing them."""
+"""rans_ilv encoder: blocks whose words the first pass keeps, and those past them.
+
+The payload equals the format specification's (oracle) for blocks of even and
+odd word counts, partial blocks and blocks with hardly a word; and of a plane
+of more blocks than are kept (32768), blocks on both sides of the line decode
+to their symbols in the specification's decoder and the whole plane on the
+device.  The payload equals the specification's too on both sides of the lines
+between the coded and the packed or stored form, which the encoder decides for
+some planes without sizing them.
+"""
 import numpy as np
 import pytest
 
 import oracle as O
-from ptwm_amd import api, ids
+from ptwm_amd import api, ids, plan
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 BLOCK = 16384
+KEPT = 32768
 
 
 def encode(t, out):
@@ -29,3 +37,47 @@ def test_forms_near_the_line(n, k):
         out = torch.full((n + 64,), 7, dtype=torch.uint8, device="cuda:0")
         used = encode(torch.from_numpy(src.copy()).cuda(), out)
         assert out[:used].cpu().numpy().tobytes() == O.rans_ilv_encode(src.tobytes())
+
+
+def symbols(n, p, seed):
+    return np.random.default_rng(seed).geometric(p, n).clip(1, 255).astype(np.uint8) - 1
+
+
+@pytest.mark.parametrize("n", [1, 64, 1023, BLOCK - 1, BLOCK, BLOCK + 1, 3 * BLOCK - 17, 40 * BLOCK + 5])
+@pytest.mark.parametrize("p", [0.9999, 0.8, 0.15])
+def test_payload(n, p):
+    src = symbols(n, p, n)
+    d = torch.from_numpy(src.copy()).cuda()
+    out = torch.full((n + 64,), 7, dtype=torch.uint8, device="cuda:0")
+    used = encode(d, out)
+    got = out.cpu().numpy().tobytes()
+    assert got[:used] == O.rans_ilv_encode(src.tobytes())
+    assert got[used:] == b"\7" * (n + 64 - used)
+
+
+def test_blocks_past_the_kept_ones():
+    n = (KEPT + 3) * BLOCK + 1001
+    g = torch.Generator(device="cuda:0").manual_seed(8)
+    d = (torch.randn(n, generator=g, device="cuda:0") * 2).abs().to(torch.uint8)
+    out = torch.zeros(n + 4096, dtype=torch.uint8, device="cuda:0")
+    used, state = api.encode_tensor_cuda(plan.CHAIN_PASSTHROUGH, d, out, 0, codec="rans_ilv")
+    p = plan.decode_plan(state)[0].planes[0]
+    assert p.codec == ids.CODEC_RANS_ILV and p.payload_len < n // 2
+    back = torch.zeros(n, dtype=torch.uint8, device="cuda:0")
+    api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, state, out[:used],
+                                              back, 0)
+    assert torch.equal(back, d)
+    # the blocks around the line, as a payload of their own: its header and
+    # table entries for them
+    max_sym = int(out[5])
+    head = (5 + 1 + 2 * (max_sym + 1) + 3) // 4 * 4
+    n_blocks = -(-n // BLOCK)
+    base = p.payload_offset
+    table = out[base + head:base + head + 4 * (n_blocks + 1)].cpu().numpy().view(np.uint32)
+    lo, hi = KEPT - 2, KEPT + 2
+    data = base + head + 4 * (n_blocks + 1)
+    h = bytearray(out[base:base + head].cpu().numpy().tobytes())
+    h[1:5] = np.uint32((hi - lo) * BLOCK).tobytes()
+    part = bytes(h) + (table[lo:hi + 1] - table[lo]).astype(np.uint32).tobytes() + \
+        out[data + int(table[lo]):data + int(table[hi])].cpu().numpy().tobytes()
+    assert O.rans_ilv_decode(part, (hi - lo) * BLOCK) == d[lo * BLOCK:hi * BLOCK].cpu().numpy().tobytes()
