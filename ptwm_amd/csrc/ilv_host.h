@@ -37,12 +37,29 @@ enum IlvForm : uint32_t { kFormStored = 0, kFormCoded = 1, kFormPacked = 2, kFor
 uint32_t ilv_choose_form(uint64_t n, bool nibbles, bool codable, uint64_t coded_len, bool identity_fallback,
                          uint64_t* len);
 
-// Write the stored, packed and Identity payloads among res[0..np) (form[p]
-// as chosen above) on ctx.stream: tag bytes and packed headers from `keep`
-// (host memory the caller keeps alive until the stream is synchronised),
-// plane copies and one pack launch.  Returns kOk or an error status.
-int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                         const IlvEncResult* res, const uint32_t* form, std::vector<uint8_t>& keep);
+// What the last encoder pass takes up to the device, in one copy from pinned
+// memory (host) to ctx.enc_pack (dev): the jobs of the payload forms that are
+// copies, the heads of the others (head[p]: plane p's place, its block offset
+// table included) and the block list at `blocks`.  A copy of its own for each
+// head left the device idle for 5 to 15 us between them (huff_ilv: the nine
+// tensors of a small layer 262 to 211 us, two bf16 layers 1105 to 1043 us).
+struct IlvUpload {
+  uint8_t* host;
+  uint8_t* dev;
+  std::vector<size_t> head;
+  size_t blocks, bytes, pack_jobs, store_jobs, head_jobs;
+  uint32_t n_pack, n_store, n_head;
+  uint64_t max_pack, max_store, max_head;
+};
+// Lay it out for res[0..np) (form[p] as chosen above; head_len[p]: the head
+// bytes of coded planes) with block_bytes of block list, and fill in the jobs;
+// the caller writes the coded planes' heads (zeroed) and the block list, then
+// sends it: one copy, then the launches that write the heads and the stored,
+// packed and Identity payloads.
+int64_t ilv_upload_begin(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
+                         const IlvEncResult* res, const uint32_t* form, const uint64_t* head_len, size_t block_bytes,
+                         IlvUpload& u);
+int64_t ilv_upload_send(DevCtx& ctx, const IlvUpload& u);
 
 // np rows of 256 zeros in ctx.enc_hist, for counts that the encoders take with
 // `counted`; nullptr on an error.

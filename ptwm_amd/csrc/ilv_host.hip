@@ -47,43 +47,76 @@ uint32_t ilv_choose_form(uint64_t n, bool nibbles, bool codable, uint64_t coded_
   return form;
 }
 
-int64_t ilv_store_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
-                         const IlvEncResult* res, const uint32_t* form, std::vector<uint8_t>& keep) {
-  hipStream_t s = ctx.stream;
-  // [8 header bytes per plane][pack jobs][store jobs]; the job arrays go
-  // to the device in one upload
-  keep.assign((size_t)np * (8 + sizeof(IlvPackJob) + sizeof(IlvStoreJob)), 0);
-  IlvPackJob* jobs = reinterpret_cast<IlvPackJob*>(keep.data() + 8 * np);
-  IlvStoreJob* sjobs = reinterpret_cast<IlvStoreJob*>(keep.data() + (8 + sizeof(IlvPackJob)) * (size_t)np);
-  uint32_t nj = 0, ns = 0;
-  uint64_t max_n = 0, max_s = 0;
+int64_t ilv_upload_begin(DevCtx& ctx, const uint64_t* src, const uint64_t* n, uint32_t np, uint64_t out_dev,
+                         const IlvEncResult* res, const uint32_t* form, const uint64_t* head_len, size_t block_bytes,
+                         IlvUpload& u) {
+  u = IlvUpload{};
+  std::vector<IlvPackJob> pack;
+  std::vector<IlvStoreJob> store, heads;  // heads: src filled in below
+  std::vector<uint32_t> head_of;
   for (uint32_t p = 0; p < np; ++p) {
     const uint64_t dst = out_dev + res[p].offset;
-    uint8_t* head = keep.data() + 8 * p;
     if (form[p] == kFormIdentity || form[p] == kFormStored) {
       const uint32_t shift = form[p] == kFormStored ? 1u : 0u;
       if (n[p] + shift == 0) continue;
-      sjobs[ns++] = IlvStoreJob{src[p], dst, n[p], shift, 0};
-      max_s = std::max(max_s, n[p] + shift);
-    } else if (form[p] == kFormPacked) {
-      head[0] = 2;
-      const uint32_t nn = (uint32_t)n[p];
-      std::memcpy(head + 1, &nn, 4);
-      PTWM_HIP_TRY(hipMemcpyAsync(reinterpret_cast<void*>(dst), head, kPackedHeadBytes, hipMemcpyHostToDevice, s));
-      jobs[nj++] = IlvPackJob{src[p], dst + kPackedHeadBytes, n[p]};
-      max_n = std::max(max_n, n[p]);
+      store.push_back(IlvStoreJob{src[p], dst, n[p], shift, 0});
+      u.max_store = std::max(u.max_store, n[p] + shift);
+      continue;
     }
+    if (form[p] == kFormPacked) {
+      pack.push_back(IlvPackJob{src[p], dst + kPackedHeadBytes, n[p]});
+      u.max_pack = std::max(u.max_pack, n[p]);
+    }
+    const uint64_t len = form[p] == kFormPacked ? kPackedHeadBytes : head_len[p];
+    heads.push_back(IlvStoreJob{0, dst, len, 0, 0});
+    head_of.push_back(p);
+    u.max_head = std::max(u.max_head, len);
   }
-  if (nj || ns) {
-    const size_t pack_bytes = nj * sizeof(IlvPackJob);
-    PTWM_HIP_TRY(ctx.enc_pack.ensure(pack_bytes + ns * sizeof(IlvStoreJob)));
-    if (ns) std::memmove(reinterpret_cast<uint8_t*>(jobs) + pack_bytes, sjobs, ns * sizeof(IlvStoreJob));
-    PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_pack.ptr, jobs, pack_bytes + ns * sizeof(IlvStoreJob), hipMemcpyHostToDevice,
-                                s));
-    uint8_t* d = static_cast<uint8_t*>(ctx.enc_pack.ptr);
-    PTWM_HIP_TRY(launch_ilv_pack(reinterpret_cast<const IlvPackJob*>(d), nj, max_n, s));
-    PTWM_HIP_TRY(launch_ilv_store(reinterpret_cast<const IlvStoreJob*>(d + pack_bytes), ns, max_s, s));
-  }
+  size_t at = 0;
+  auto place = [&at](size_t bytes) {
+    const size_t a = at;
+    at = align_up(at + bytes, 16);
+    return a;
+  };
+  u.pack_jobs = place(pack.size() * sizeof(IlvPackJob));
+  u.store_jobs = place(store.size() * sizeof(IlvStoreJob));
+  u.head_jobs = place(heads.size() * sizeof(IlvStoreJob));
+  const size_t first_head = at;
+  u.head.assign(np, 0);
+  for (size_t i = 0; i < heads.size(); ++i) u.head[head_of[i]] = place(heads[i].n);
+  u.blocks = place(block_bytes);
+  u.bytes = at;
+  u.n_pack = (uint32_t)pack.size();
+  u.n_store = (uint32_t)store.size();
+  u.n_head = (uint32_t)heads.size();
+  if (!u.bytes) return kOk;
+  PTWM_HIP_TRY(ctx.enc_pack.ensure(u.bytes));
+  PTWM_HIP_TRY(ctx.h_enc.ensure(u.bytes));
+  u.host = static_cast<uint8_t*>(ctx.h_enc.ptr);
+  u.dev = static_cast<uint8_t*>(ctx.enc_pack.ptr);
+  for (size_t i = 0; i < heads.size(); ++i)
+    heads[i].src = reinterpret_cast<uint64_t>(u.dev) + u.head[head_of[i]];
+  std::copy(pack.begin(), pack.end(), reinterpret_cast<IlvPackJob*>(u.host + u.pack_jobs));
+  std::copy(store.begin(), store.end(), reinterpret_cast<IlvStoreJob*>(u.host + u.store_jobs));
+  std::copy(heads.begin(), heads.end(), reinterpret_cast<IlvStoreJob*>(u.host + u.head_jobs));
+  std::memset(u.host + first_head, 0, u.blocks - first_head);
+  for (const uint32_t p : head_of)
+    if (form[p] == kFormPacked) {
+      uint8_t* const h = u.host + u.head[p];
+      h[0] = 2;
+      const uint32_t nn = (uint32_t)n[p];
+      std::memcpy(h + 1, &nn, 4);
+    }
+  return kOk;
+}
+
+int64_t ilv_upload_send(DevCtx& ctx, const IlvUpload& u) {
+  if (!u.bytes) return kOk;
+  hipStream_t s = ctx.stream;
+  PTWM_HIP_TRY(hipMemcpyAsync(u.dev, u.host, u.bytes, hipMemcpyHostToDevice, s));
+  PTWM_HIP_TRY(launch_ilv_store(reinterpret_cast<const IlvStoreJob*>(u.dev + u.head_jobs), u.n_head, u.max_head, s));
+  PTWM_HIP_TRY(launch_ilv_pack(reinterpret_cast<const IlvPackJob*>(u.dev + u.pack_jobs), u.n_pack, u.max_pack, s));
+  PTWM_HIP_TRY(launch_ilv_store(reinterpret_cast<const IlvStoreJob*>(u.dev + u.store_jobs), u.n_store, u.max_store, s));
   return kOk;
 }
 
@@ -160,7 +193,8 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
     for (uint32_t b = 0; b < nbs[p]; ++b) blocks.push_back(IlvEncBlock{0, p, b, 0, 0});
   }
   const uint32_t nblk = (uint32_t)blocks.size();
-  std::vector<uint32_t> bbytes(nblk);
+  PTWM_HIP_TRY(ctx.h_sizes.ensure(nblk * sizeof(uint32_t)));
+  uint32_t* const bbytes = static_cast<uint32_t*>(ctx.h_sizes.ptr);
   if (nblk) {
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(IlvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_lane_words.ensure((size_t)nblk * 64));
@@ -174,7 +208,7 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
                                  static_cast<const uint32_t*>(ctx.enc_codes.ptr),
                                  static_cast<uint8_t*>(ctx.enc_lane_words.ptr),
                                  static_cast<uint32_t*>(ctx.enc_block_bytes.ptr), s));
-    PTWM_HIP_TRY(hipMemcpyAsync(bbytes.data(), ctx.enc_block_bytes.ptr, nblk * 4, hipMemcpyDeviceToHost, s));
+    PTWM_HIP_TRY(hipMemcpyAsync(bbytes, ctx.enc_block_bytes.ptr, nblk * 4, hipMemcpyDeviceToHost, s));
     PTWM_HIP_TRY(hipStreamSynchronize(s));
   }
   // ---- layout: payloads at 256-byte aligned offsets ----
@@ -203,60 +237,49 @@ int64_t ilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, u
     if (needed) *needed = total;
     return kBufferTooSmall;
   }
-  // ---- headers, offset tables and block destinations ----
-  uint64_t host_bytes = 0;
+  // ---- headers, offset tables and block destinations: one upload ----
+  // (only blocks of coded planes are written; lw keeps the size-pass index)
+  size_t live = 0;
+  std::vector<uint64_t> head_len(np, 0);
   for (uint32_t p = 0; p < np; ++p)
-    if (res[p].coded) host_bytes += head[p] + 4ull * (nbs[p] + 1);
-  PTWM_HIP_TRY(ctx.h_enc.ensure(host_bytes + nblk * sizeof(IlvEncBlock) + 64));
-  uint8_t* hb = static_cast<uint8_t*>(ctx.h_enc.ptr);
-  IlvEncBlock* hblk = reinterpret_cast<IlvEncBlock*>(hb + host_bytes);
-  std::memcpy(hblk, blocks.data(), nblk * sizeof(IlvEncBlock));
-  std::vector<uint8_t> keep;
-  if (int64_t rc = ilv_store_planes(ctx, src, n, np, out_dev, res, form.data(), keep); rc != kOk) return rc;
-  uint64_t hoff = 0;
+    if (res[p].coded) {
+      head_len[p] = head[p] + 4ull * (nbs[p] + 1);
+      live += nbs[p];
+    }
+  IlvUpload u;
+  if (int64_t rc = ilv_upload_begin(ctx, src, n, np, out_dev, res, form.data(), head_len.data(),
+                                    live * sizeof(IlvEncBlock), u);
+      rc != kOk)
+    return rc;
+  IlvEncBlock* hblk = reinterpret_cast<IlvEncBlock*>(u.host + u.blocks);
+  uint32_t max_words = 0;
   for (uint32_t p = 0; p < np; ++p) {
-    const uint64_t dst = out_dev + res[p].offset;
     if (!res[p].coded) continue;
-    uint8_t* h = hb + hoff;
-    std::memset(h, 0, head[p]);
+    uint8_t* h = u.host + u.head[p];
     h[0] = 1;
     uint32_t nn = (uint32_t)n[p];
     std::memcpy(h + 1, &nn, 4);
     std::memcpy(h + 5, info[p].head, info[p].head_len);
     uint32_t* tab = reinterpret_cast<uint32_t*>(h + head[p]);
     uint64_t acc = 0;
-    const uint64_t data_dev = dst + head[p] + 4ull * (nbs[p] + 1);
+    const uint64_t data_dev = out_dev + res[p].offset + head_len[p];
     for (uint32_t b = 0; b < nbs[p]; ++b) {
+      const uint32_t i = first_block[p] + b;
       tab[b] = (uint32_t)acc;
-      hblk[first_block[p] + b].dst = data_dev + acc;
-      acc += bbytes[first_block[p] + b];
+      *hblk++ = IlvEncBlock{data_dev + acc, p, b, i, 0};
+      acc += bbytes[i];
+      max_words = std::max(max_words, bbytes[i] >= 64 ? (bbytes[i] - 64) / 4 : 0u);
     }
     tab[nbs[p]] = (uint32_t)acc;
-    const uint64_t hl = head[p] + 4ull * (nbs[p] + 1);
-    PTWM_HIP_TRY(hipMemcpyAsync(reinterpret_cast<void*>(dst), h, hl, hipMemcpyHostToDevice, s));
-    hoff += hl;
   }
-  if (nblk) {
-    // only blocks of coded planes are written; lw keeps the size-pass index
-    uint32_t live = 0, max_words = 0;
-    for (uint32_t i = 0; i < nblk; ++i)
-      if (res[hblk[i].plane].coded) {
-        IlvEncBlock bk = hblk[i];
-        bk.lw = i;
-        hblk[live++] = bk;
-        max_words = std::max(max_words, bbytes[i] >= 64 ? (bbytes[i] - 64) / 4 : 0u);
-      }
-    // LDS for the largest block's words, within the cap (larger blocks are
-    // written lane by lane)
-    const uint32_t stage_words = std::min<uint32_t>(kIlvEncStageMax, (max_words + 3) & ~3u);
-    if (live) {
-      PTWM_HIP_TRY(hipMemcpyAsync(ctx.enc_blocks.ptr, hblk, live * sizeof(IlvEncBlock), hipMemcpyHostToDevice, s));
-      PTWM_HIP_TRY(launch_ilv_encode(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
-                                     static_cast<const IlvEncBlock*>(ctx.enc_blocks.ptr), live,
-                                     static_cast<const uint32_t*>(ctx.enc_codes.ptr),
-                                     static_cast<const uint8_t*>(ctx.enc_lane_words.ptr), stage_words, s));
-    }
-  }
+  if (int64_t rc = ilv_upload_send(ctx, u); rc != kOk) return rc;
+  // LDS for the largest block's words, within the cap (larger blocks are
+  // written lane by lane)
+  const uint32_t stage_words = std::min<uint32_t>(kIlvEncStageMax, (max_words + 3) & ~3u);
+  PTWM_HIP_TRY(launch_ilv_encode(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
+                                 reinterpret_cast<const IlvEncBlock*>(u.dev + u.blocks), (uint32_t)live,
+                                 static_cast<const uint32_t*>(ctx.enc_codes.ptr),
+                                 static_cast<const uint8_t*>(ctx.enc_lane_words.ptr), stage_words, s));
   PTWM_HIP_TRY(hipStreamSynchronize(s));
   return (int64_t)total;
 }

@@ -77,7 +77,8 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     for (uint32_t b = 0; b < nbs[p]; ++b) blocks.push_back(RilvEncBlock{0, p, b, (uint32_t)blocks.size(), 0});
   }
   const uint32_t nblk = (uint32_t)blocks.size();
-  std::vector<uint32_t> bwords(nblk);
+  PTWM_HIP_TRY(ctx.h_sizes.ensure(nblk * sizeof(uint32_t)));
+  uint32_t* const bwords = static_cast<uint32_t*>(ctx.h_sizes.ptr);
   uint32_t kept = std::min(nblk, kRilvKeepBlocks);
   if (kept && ctx.enc_keep.ensure(kept * kRilvKeepBytes) != hipSuccess) {
     (void)hipGetLastError();
@@ -86,14 +87,16 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   if (nblk) {
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(RilvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_block_bytes.ensure(nblk * sizeof(uint32_t)));
+    PTWM_HIP_TRY(ctx.h_enc.ensure(nblk * sizeof(RilvEncBlock)));
+    std::memcpy(ctx.h_enc.ptr, blocks.data(), nblk * sizeof(RilvEncBlock));
     PTWM_HIP_TRY(
-        hipMemcpyAsync(ctx.enc_blocks.ptr, blocks.data(), nblk * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
+        hipMemcpyAsync(ctx.enc_blocks.ptr, ctx.h_enc.ptr, nblk * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
     PTWM_HIP_TRY(launch_rilv_size(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr),
                                   static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr), nblk, kept,
                                   static_cast<const uint32_t*>(ctx.enc_codes.ptr),
                                   static_cast<uint32_t*>(ctx.enc_block_bytes.ptr),
                                   static_cast<uint8_t*>(ctx.enc_keep.ptr), s));
-    PTWM_HIP_TRY(hipMemcpyAsync(bwords.data(), ctx.enc_block_bytes.ptr, nblk * 4, hipMemcpyDeviceToHost, s));
+    PTWM_HIP_TRY(hipMemcpyAsync(bwords, ctx.enc_block_bytes.ptr, nblk * 4, hipMemcpyDeviceToHost, s));
     PTWM_HIP_TRY(hipStreamSynchronize(s));
   }
   // ---- layout: payloads at 256-byte aligned offsets ----
@@ -122,46 +125,49 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
     if (needed) *needed = total;
     return kBufferTooSmall;
   }
-  // ---- headers, offset tables, stored / packed planes; block destinations ----
-  // (host buffers of the asynchronous uploads stay alive until the final
-  // stream synchronisation)
-  std::vector<uint8_t> keep;
-  if (int64_t rc = ilv_store_planes(ctx, src, n, np, out_dev, res, form.data(), keep); rc != kOk) return rc;
-  std::vector<std::vector<uint8_t>> hbufs(np);
-  std::vector<RilvEncBlock> live;
+  // ---- headers, offset tables, stored / packed planes, block destinations:
+  // one upload ----
+  size_t live = 0, n_kept = 0;  // blocks of coded planes, and those whose words are there
+  std::vector<uint64_t> head_len(np, 0);
+  for (uint32_t p = 0; p < np; ++p)
+    if (res[p].coded) {
+      head_len[p] = head[p] + 4ull * (nbs[p] + 1);
+      live += nbs[p];
+    }
+  IlvUpload u;
+  if (int64_t rc = ilv_upload_begin(ctx, src, n, np, out_dev, res, form.data(), head_len.data(),
+                                    live * sizeof(RilvEncBlock), u);
+      rc != kOk)
+    return rc;
+  RilvEncBlock* hblk = reinterpret_cast<RilvEncBlock*>(u.host + u.blocks);
   for (uint32_t p = 0; p < np; ++p) {
-    const uint64_t dst = out_dev + res[p].offset;
     if (!res[p].coded) continue;
-    std::vector<uint8_t>& hbuf = hbufs[p];
-    hbuf.assign(head[p] + 4ull * (nbs[p] + 1), 0);
-    hbuf[0] = 1;
+    uint8_t* const h = u.host + u.head[p];
+    h[0] = 1;
     const uint32_t nn = (uint32_t)n[p];
-    std::memcpy(hbuf.data() + 1, &nn, 4);
-    std::memcpy(hbuf.data() + 5, info[p].head, info[p].head_len);
-    uint32_t* tab = reinterpret_cast<uint32_t*>(hbuf.data() + head[p]);
+    std::memcpy(h + 1, &nn, 4);
+    std::memcpy(h + 5, info[p].head, info[p].head_len);
+    uint32_t* tab = reinterpret_cast<uint32_t*>(h + head[p]);
     uint64_t acc = 0;
-    const uint64_t data_dev = dst + hbuf.size();
+    const uint64_t data_dev = out_dev + res[p].offset + head_len[p];
     for (uint32_t b = 0; b < nbs[p]; ++b) {
+      const uint32_t i = first_block[p] + b;
       tab[b] = (uint32_t)acc;
-      RilvEncBlock bk = blocks[first_block[p] + b];
-      bk.dst = data_dev + acc;
-      live.push_back(bk);
-      acc += align_up(kRilvBlockHead + 2ull * bwords[first_block[p] + b], 4);
+      *hblk++ = RilvEncBlock{data_dev + acc, p, b, i, 0};
+      n_kept += i < kept;  // (i rises along the list)
+      acc += align_up(kRilvBlockHead + 2ull * bwords[i], 4);
     }
     tab[nbs[p]] = (uint32_t)acc;
-    PTWM_HIP_TRY(hipMemcpyAsync(reinterpret_cast<void*>(dst), hbuf.data(), hbuf.size(), hipMemcpyHostToDevice, s));
   }
-  if (!live.empty()) {
-    const RilvEncBlock* const bd = static_cast<const RilvEncBlock*>(ctx.enc_blocks.ptr);
+  if (int64_t rc = ilv_upload_send(ctx, u); rc != kOk) return rc;
+  if (live) {
+    const RilvEncBlock* const bd = reinterpret_cast<const RilvEncBlock*>(u.dev + u.blocks);
     const uint32_t* const words = static_cast<const uint32_t*>(ctx.enc_block_bytes.ptr);
-    uint32_t n_kept = 0;  // rows rise along `live`
-    while (n_kept < live.size() && live[n_kept].row < kept) ++n_kept;
     PTWM_HIP_TRY(
-        hipMemcpyAsync(ctx.enc_blocks.ptr, live.data(), live.size() * sizeof(RilvEncBlock), hipMemcpyHostToDevice, s));
-    PTWM_HIP_TRY(launch_rilv_place(bd, n_kept, words, static_cast<const uint8_t*>(ctx.enc_keep.ptr), s));
+        launch_rilv_place(bd, (uint32_t)n_kept, words, static_cast<const uint8_t*>(ctx.enc_keep.ptr), s));
     PTWM_HIP_TRY(launch_rilv_encode(static_cast<const IlvEncPlane*>(ctx.enc_planes.ptr), bd + n_kept,
-                                    (uint32_t)live.size() - n_kept, static_cast<const uint32_t*>(ctx.enc_codes.ptr),
-                                    words, s));
+                                    (uint32_t)(live - n_kept), static_cast<const uint32_t*>(ctx.enc_codes.ptr), words,
+                                    s));
   }
   PTWM_HIP_TRY(hipStreamSynchronize(s));
   return (int64_t)total;

@@ -94,7 +94,7 @@ struct DevCtx {
   PinnedBuffer h_ref;
   // what the encoders' table builds tell the host (TableInfo, host-coherent)
   PinnedBuffer h_tables;
-  PinnedBuffer h_enc, h_ilv;
+  PinnedBuffer h_enc, h_sizes, h_ilv;
   // fused-decode status words, written by the kernels (host-coherent)
   PinnedBuffer h_ilv_status;
   // parallel Huffman decode of reference streams
