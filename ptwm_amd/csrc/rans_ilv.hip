@@ -484,11 +484,12 @@ __device__ __forceinline__ uint64_t rilv_pos(uint32_t b, uint32_t lane, uint32_t
   return (uint64_t)b * kIlvBlock + (uint64_t)kIlvGroup * (64u * (s / kIlvGroup) + lane) + (s % kIlvGroup);
 }
 
-// 1 / f of each symbol's frequency (f = 0, a symbol the histogram did not
-// see, as 1), for the encoder's quotient estimate
-__device__ __forceinline__ float rilv_rcp(uint32_t fc) {
-  const uint32_t f0 = fc & 0xFFFFu;
-  return 1.0f / (float)(f0 ? f0 : 1u);
+// A symbol's entry: f | cum << 16, with f = 1 for a symbol that the histogram
+// did not see (source changed: a bad stream, no trap), and the bits of 1 / f for
+// the quotient estimate.
+__device__ __forceinline__ uint2 rilv_entry(uint32_t fc) {
+  if (!(fc & 0xFFFFu)) fc |= 1u;
+  return make_uint2(fc, __builtin_bit_cast(uint32_t, 1.0f / (float)(fc & 0xFFFFu)));
 }
 
 // The encoder's step for one lane: renormalise (emit) then encode.  After
@@ -496,14 +497,13 @@ __device__ __forceinline__ float rilv_rcp(uint32_t fc) {
 // x * (1 / f) is within one of it (x rounds by at most f / 8, the product
 // and the reciprocal add under 2^-22 relative); one correction step makes
 // q and r exact.
-__device__ __forceinline__ bool rilv_enc_step(uint32_t& x, uint32_t fc, float rf, uint32_t& word) {
-  const uint32_t f0 = fc & 0xFFFFu, c = fc >> 16;
-  const uint32_t f = f0 ? f0 : 1u;  // a symbol the histogram did not see (source changed): a bad stream, no trap
-  const bool emit = (uint64_t)x >= ((uint64_t)f << 21);
+__device__ __forceinline__ bool rilv_enc_step(uint32_t& x, uint2 e, uint32_t& word) {
+  const uint32_t f = e.x & 0xFFFFu, c = e.x >> 16;
+  const bool emit = x >> 21 >= f;
   word = x & 0xFFFFu;
   if (emit) x >>= 16;
-  uint32_t q = (uint32_t)((float)x * rf);
-  int32_t r = (int32_t)(x - q * f);  // true value in [-f, 2f): exact as int32
+  uint32_t q = (uint32_t)((float)x * __builtin_bit_cast(float, e.y));
+  int32_t r = (int32_t)(x - __umul24(q, f));  // true value in [-f, 2f): exact as int32
   if (r < 0) {
     --q;
     r += (int32_t)f;
@@ -529,6 +529,53 @@ __device__ __forceinline__ void rilv_load_group(const IlvEncPlane& P, uint64_t g
   }
 }
 
+// Block B of plane P, last symbol first: put(emit, word) for every step, all
+// lanes taking part.  The chain of a lane is a step's arithmetic alone where
+// the block is whole: the 16 entries of a group are read before its steps, its
+// bytes a group ahead.
+// Encode of e4m3 5001x3333: 167 to 145 us, of a 4096x4096 bf16 tensor 157 to
+// 133 us.
+template <typename F>
+__device__ __forceinline__ uint32_t rilv_encode_block(const IlvEncPlane& P, uint32_t block, uint32_t lane,
+                                                      const uint2* entry, F put) {
+  uint32_t x = kRilvL;
+  if (((uint64_t)block + 1) * kIlvBlock <= P.n) {  // uniform
+    uint32_t next[4];
+    rilv_load_group(P, rilv_pos(block, lane, 16u * (kIlvRounds - 1)), next);
+    for (int r = (int)kIlvRounds - 1; r >= 0; --r) {
+      const uint32_t sym[4] = {next[0], next[1], next[2], next[3]};
+      if (r > 0) rilv_load_group(P, rilv_pos(block, lane, 16u * (uint32_t)(r - 1)), next);
+      uint2 e[kIlvGroup];
+#pragma unroll
+      for (uint32_t k = 0; k < kIlvGroup; ++k) e[k] = entry[(sym[k >> 2] >> (8 * (k & 3))) & 0xFFu];
+#pragma unroll
+      for (int k = (int)kIlvGroup - 1; k >= 0; --k) {
+        uint32_t w;
+        const bool emit = rilv_enc_step(x, e[k], w);
+        put(emit, w);
+      }
+    }
+    return x;
+  }
+  for (int r = (int)kIlvRounds - 1; r >= 0; --r) {
+    const uint64_t g0 = rilv_pos(block, lane, 16u * (uint32_t)r);
+    uint32_t sym[4];
+    rilv_load_group(P, g0, sym);
+    for (int k = (int)kIlvGroup - 1; k >= 0; --k) {
+      bool emit = false;
+      uint32_t w = 0;
+      if (g0 + k < P.n) emit = rilv_enc_step(x, entry[(sym[k >> 2] >> (8 * (k & 3))) & 0xFFu], w);
+      put(emit, w);
+    }
+  }
+  return x;
+}
+
+// Lanes below this one among `bal`.
+__device__ __forceinline__ uint32_t rilv_rank(uint64_t bal) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+}
+
 // One wavefront per block: run the encoder and count the words.  The states
 // of a lane form one chain of 256 steps, which bounds this kernel and
 // rilv_encode_kernel alike, so the words and final states are kept where
@@ -540,38 +587,21 @@ __global__ void __launch_bounds__(64) rilv_size_kernel(const IlvEncPlane* __rest
                                                        const RilvEncBlock* __restrict__ blocks, uint32_t kept,
                                                        const uint32_t* __restrict__ syms,
                                                        uint32_t* __restrict__ block_words, uint8_t* keep) {
-  __shared__ uint32_t fc[256];
-  __shared__ float rf[256];
+  __shared__ uint2 entry[256];
   const RilvEncBlock B = blocks[blockIdx.x];
   const IlvEncPlane P = planes[B.plane];
   const uint32_t lane = threadIdx.x;
-  for (uint32_t i = lane; i < 256; i += 64) {
-    fc[i] = syms[256u * P.code_slot + i];
-    rf[i] = rilv_rcp(fc[i]);
-  }
+  for (uint32_t i = lane; i < 256; i += 64) entry[i] = rilv_entry(syms[256u * P.code_slot + i]);
   __syncthreads();
   const bool keeps = blockIdx.x < kept;  // uniform
   const uint64_t slot = reinterpret_cast<uint64_t>(keep) + kRilvKeepBytes * blockIdx.x;
-  uint32_t x = kRilvL, nw = 0;
-  for (int r = (int)kIlvRounds - 1; r >= 0; --r) {
-    const uint64_t g0 = rilv_pos(B.block, lane, 16u * (uint32_t)r);
-    uint32_t sym[4];
-    rilv_load_group(P, g0, sym);
-    for (int tt = (int)kIlvGroup - 1; tt >= 0; --tt) {
-      bool emit = false;
-      uint32_t w = 0;
-      if (g0 + tt < P.n) {
-        const uint32_t sy = (sym[tt >> 2] >> (8 * (tt & 3))) & 0xFFu;
-        emit = rilv_enc_step(x, fc[sy], rf[sy], w);
-      }
-      const uint64_t bal = __ballot(emit);
-      nw += (uint32_t)__builtin_popcountll(bal);
-      const uint32_t rank =
-          __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-      // (at most one word a symbol: nw <= kIlvBlock)
-      if (keeps && emit) g_st<uint16_t>(slot + 2ull * (kIlvBlock - nw + rank), (uint16_t)w);
-    }
-  }
+  uint32_t nw = 0;
+  const uint32_t x = rilv_encode_block(P, B.block, lane, entry, [&](bool emit, uint32_t w) {
+    const uint64_t bal = __ballot(emit);
+    nw += (uint32_t)__builtin_popcountll(bal);
+    // (at most one word a symbol: nw <= kIlvBlock)
+    if (keeps && emit) g_st<uint16_t>(slot + 2ull * (kIlvBlock - nw + rilv_rank(bal)), (uint16_t)w);
+  });
   if (lane == 0) block_words[blockIdx.x] = nw;
   if (keeps) g_st<uint32_t>(slot + 2ull * kIlvBlock + 4 * lane, x);
 }
@@ -601,39 +631,23 @@ __global__ void __launch_bounds__(64) rilv_encode_kernel(const IlvEncPlane* __re
                                                          const RilvEncBlock* __restrict__ blocks,
                                                          const uint32_t* __restrict__ syms,
                                                          const uint32_t* __restrict__ block_words) {
-  __shared__ uint32_t fc[256];
-  __shared__ float rf[256];
+  __shared__ uint2 entry[256];
   const RilvEncBlock B = blocks[blockIdx.x];
   const IlvEncPlane P = planes[B.plane];
   const uint32_t lane = threadIdx.x;
-  for (uint32_t i = lane; i < 256; i += 64) {
-    fc[i] = syms[256u * P.code_slot + i];
-    rf[i] = rilv_rcp(fc[i]);
-  }
+  for (uint32_t i = lane; i < 256; i += 64) entry[i] = rilv_entry(syms[256u * P.code_slot + i]);
   __syncthreads();
   const uint32_t nw = block_words[B.row];
   const uint64_t words = B.dst + kRilvBlockHead;
-  uint32_t x = kRilvL, tail = nw;
-  for (int r = (int)kIlvRounds - 1; r >= 0; --r) {
-    const uint64_t g0 = rilv_pos(B.block, lane, 16u * (uint32_t)r);
-    uint32_t sym[4];
-    rilv_load_group(P, g0, sym);
-    for (int tt = (int)kIlvGroup - 1; tt >= 0; --tt) {
-      bool emit = false;
-      uint32_t w = 0;
-      if (g0 + tt < P.n) {
-        const uint32_t sy = (sym[tt >> 2] >> (8 * (tt & 3))) & 0xFFu;
-        emit = rilv_enc_step(x, fc[sy], rf[sy], w);
-      }
-      const uint64_t bal = __ballot(emit);
-      tail -= (uint32_t)__builtin_popcountll(bal);
-      const uint32_t rank =
-          __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-      // (the size pass counted the same words; the bound only guards a
-      // source that changed between the passes)
-      if (emit && tail + rank < nw) g_st<uint16_t>(words + 2ull * (tail + rank), (uint16_t)w);
-    }
-  }
+  uint32_t tail = nw;
+  const uint32_t x = rilv_encode_block(P, B.block, lane, entry, [&](bool emit, uint32_t w) {
+    const uint64_t bal = __ballot(emit);
+    tail -= (uint32_t)__builtin_popcountll(bal);
+    const uint32_t rank = rilv_rank(bal);
+    // (the size pass counted the same words; the bound only guards a
+    // source that changed between the passes)
+    if (emit && tail + rank < nw) g_st<uint16_t>(words + 2ull * (tail + rank), (uint16_t)w);
+  });
   g_st<uint32_t>(B.dst + 4 + 4 * lane, x);
   if (lane == 0) {
     g_st<uint32_t>(B.dst, nw);
