@@ -17,19 +17,21 @@
 // steps instead of 255).  Depths by pointer jumping; the rest is a few ballots.
 #include "code_tables.h"
 
+#include "huffman_merge.h"
+
 namespace ptwm {
 
 namespace {
 
-constexpr uint32_t kNone = 0xFFFFFFFFu;
+constexpr uint32_t kNone = kMergeNone;
 constexpr uint32_t kScale = 2048;     // rANS frequencies sum to 2^11
 constexpr uint32_t kThreads = 256;
-constexpr uint32_t kRound = 16;       // items that make a round worth its barriers (0.14 us a step, 1 us a round)
+constexpr uint32_t kRound = kMergeRound;
 
 struct Scratch {
   u32x4 f4[64];                 // counts by symbol
   uint32_t leaf[256 + kRound];  // counts of the sorted leaves, then kNone
-  uint32_t node[256 + kRound];  // counts of the internal nodes, in creation order, then kNone
+  uint32_t node[256 + kRound];  // counts of the internal nodes, in creation order
   uint32_t order[256];          // a round's counts in order
   uint16_t up[512];             // parent: leaf i at i, internal node q at 256 + q
   uint16_t dist[512];           // edges to `up`
@@ -76,7 +78,7 @@ __device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t n, uint32_t 
   const uint32_t t = threadIdx.x;
   if (n == 1) return h ? 1u : 0u;
   reinterpret_cast<uint32_t*>(S.f4)[t] = h;
-  for (uint32_t i = t; i < 256 + kRound; i += kThreads) S.leaf[i] = S.node[i] = kNone;
+  for (uint32_t i = t; i < 256 + kRound; i += kThreads) S.leaf[i] = kNone;
   S.len[t] = 0;
   __syncthreads();
   // rank: symbols with (count, symbol) below this one's; a count of zero
@@ -93,19 +95,17 @@ __device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t n, uint32_t 
     S.sym[rank] = (uint8_t)t;
   }
   __syncthreads();
-  // Two FIFO queues: the sorted leaves and the internal nodes, whose counts
-  // never decrease in creation order; a leaf goes first on ties (its id is
-  // smaller).  Every thread takes every step: the writes are alike, and each
-  // reads what it wrote itself.  Counts of up to 2^32 - 1 bytes in all stay
-  // below kNone.
-  uint32_t li = 0, qi = 0, qe = 0;
-  while (n - li + (qe - qi) > 1) {
-    const uint32_t l0 = S.leaf[li], l1 = S.leaf[li + 1], i0 = S.node[qi], i1 = S.node[qi + 1];
-    const uint32_t l_far = S.leaf[li + kRound - 1], i_far = S.node[qi + kRound - 1];
-    const bool a_leaf = l0 <= i0;
-    const bool b_leaf = a_leaf ? l1 <= i0 : l0 <= i1;
-    const uint32_t both = (a_leaf ? l0 : i0) + (b_leaf ? (a_leaf ? l1 : l0) : (a_leaf ? i0 : i1));
-    if (min(l_far, i_far) <= both) {
+  // Two FIFO queues: the sorted leaves and the internal nodes; a leaf goes
+  // first on ties (its id is smaller).  Every thread takes every step: the
+  // writes are alike, each thread uses only what it wrote itself since the
+  // last barrier (merge_step), and so all wavefronts reach the same rounds and
+  // the same end.  Counts of up to 2^32 - 1 bytes in all stay below kNone
+  // until the last pair.
+  MergeQueues m{0, 0, 0};
+  while (n - m.li + (m.qe - m.qi) > 1) {
+    const MergeStep step = merge_step(S.leaf, S.node, m);
+    const uint32_t li = m.li, qi = m.qi, qe = m.qe, both = step.both;
+    if (step.round) {
       // a round: the items no larger than `both`, in order, in pairs; an odd
       // last one stays
       __syncthreads();  // (every wavefront has made its steps before)
@@ -125,20 +125,17 @@ __device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t n, uint32_t 
       const bool last_leaf = cl && (!ci || S.leaf[li + cl - 1] > S.node[qi + ci - 1]);
       __syncthreads();
       if (t < pairs) S.node[qe + t] = S.order[2 * t] + S.order[2 * t + 1];
-      li += cl - (odd && last_leaf ? 1u : 0u);
-      qi += ci - (odd && !last_leaf ? 1u : 0u);
-      qe += pairs;
+      m.li += cl - (odd && last_leaf ? 1u : 0u);
+      m.qi += ci - (odd && !last_leaf ? 1u : 0u);
+      m.qe += pairs;
       __syncthreads();
       continue;
     }
-    const uint32_t a = a_leaf ? li : 256u + qi;
-    const uint32_t b = b_leaf ? li + (a_leaf ? 1u : 0u) : 256u + qi + (a_leaf ? 0u : 1u);
+    const uint32_t a = step.a_leaf ? li : 256u + qi;
+    const uint32_t b = step.b_leaf ? li + (step.a_leaf ? 1u : 0u) : 256u + qi + (step.a_leaf ? 0u : 1u);
     S.node[qe] = both;
     S.up[a] = S.up[b] = (uint16_t)(256u + qe);
-    const uint32_t leaves = (a_leaf ? 1u : 0u) + (b_leaf ? 1u : 0u);
-    li += leaves;
-    qi += 2u - leaves;
-    ++qe;
+    m = merge_next(m, step);
   }
   const uint32_t root = 256u + n - 2u;
   __syncthreads();

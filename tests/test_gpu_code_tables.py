@@ -81,3 +81,17 @@ def test_many_tables_in_one_call():
         used, st = api.encode_tensor_ref_cuda(6, [codec], 777, src, out, 0)
         want, _ = O.encode_plane_chunked(codec, data.tobytes(), 777)
         assert out[:used].cpu().numpy().tobytes() == want
+
+
+@pytest.mark.parametrize("n", [16, 17, 22, 30, 31, 32, 33, 44, 57, 60, 61, 88, 113, 120, 121, 225, 240, 255])
+def test_flat_alphabets(n):
+    """Alphabets of n equal counts: all pairs of a level are alike, so that the merge goes through rounds and leaves
+    between 2 and 16 nodes of one queue to the serial steps."""
+    plane = spread([37] * n, n)
+    src = dev(plane)
+    out = torch.zeros(2 * len(plane) + 4096, dtype=torch.uint8, device="cuda:0")
+    for label, want in (("huffman", O.codec_encode(O.CODEC_HUFFMAN, plane.tobytes())),
+                        (ids.PLANE_CODEC_LABEL, O.ilv_encode(plane.tobytes()))):
+        print(n, label, flush=True)
+        used = api.plane_codec_encode_cuda(ids.PLANE_CODEC_LABEL, label, b"", src, out, 0)
+        assert out[:used].cpu().numpy().tobytes() == want
