@@ -502,7 +502,9 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
     JobInfo& I = info_[j];
     I.raw = true;
     const uint64_t n = jobs[j].n;
-    if (n == 0) continue;
+    // (past 32 bits no payload is coded, and the table build adds counts in 32
+    // bits: its merge may not end once its sums wrap several times)
+    if (n == 0 || n > 0xFFFFFFFFull) continue;
     const bool rans = jobs[j].codec == kCodecRans;
     tj[j] = TableJob{rans ? kTableRans : kTableHuffman, (uint32_t)jd.size(), 4, 0};
     uint64_t st[4], sn[4];
@@ -603,7 +605,7 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
     if (!I.raw) {
       uint64_t blob = I.header.size() + 16;
       for (int i = 0; i < 4; ++i) blob += seg_len_[I.seg0 + i];
-      bool coded = blob < n && n <= 0xFFFFFFFFull;  // NotBeneficial when blob >= len (compress.rs:72-75)
+      bool coded = blob < n;  // NotBeneficial when blob >= len (compress.rs:72-75)
       for (int i = 0; i < 4; ++i) coded = coded && seg_len_[I.seg0 + i] <= 0xFFFFFFFFull;
       // length_prefix::accepted (codecs/length_prefix.rs:15-56), rANS only
       if (coded && jobs[j].codec == kCodecRans) coded = n <= (1ull << 30) || n <= blob * 64;

@@ -181,3 +181,15 @@ def test_trial_encode_selection_matches_the_oracle(name, chain, make, codecs, ch
     n = api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, st,
                                                   out[:used], restored, 0)
     assert n == len(data) and host(restored) == data
+
+
+def test_plane_past_32_bits():
+    """A plane of 2^32 + 5 bytes is stored raw, as every plane longer than a payload's length field can say."""
+    n = (1 << 32) + 5
+    src = torch.randint(0, 7, (n,), dtype=torch.uint8, device="cuda:0")
+    out = torch.zeros(n + 4096, dtype=torch.uint8, device="cuda:0")
+    for codec in (O.CODEC_HUFFMAN, O.CODEC_RANS):
+        print("2^32 + 5 bytes, codec", codec, flush=True)
+        out.zero_()
+        used, st = api.encode_tensor_ref_cuda(plan.CHAIN_PASSTHROUGH, [codec], 0, src, out, 0)
+        assert used == n + 1 and int(out[0]) == 0 and torch.equal(out[1:used], src)
