@@ -18,6 +18,7 @@
 #include "code_tables.h"
 
 #include "huffman_merge.h"
+#include "ref_rans.h"
 
 namespace ptwm {
 
@@ -282,7 +283,7 @@ __global__ void __launch_bounds__(kThreads) code_tables_kernel(const TableJob* _
         if (t == 0) I.bits[0] = bits;
       } else {
         // EncSymbol (rans/compress.rs:35-68): {rcp, bias, cmpl | shift << 24},
-        // and the thresholds that ref_encode.hip's shed takes
+        // and the thresholds that shed takes (ref_rans.h)
         uint4 e;
         if (f < 2) {
           e = make_uint4(kNone, start + kScale - 1, kScale - f, 0u);
@@ -300,6 +301,10 @@ __global__ void __launch_bounds__(kThreads) code_tables_kernel(const TableJob* _
       }
       if (t == 0) head[0] = (uint8_t)(n_sym - 1);
       head_len = 1 + 2 * n_sym;
+    } else if (J.kind == kTableRans) {
+      // refused: the encoder, which runs before the host knows, goes over the
+      // plane with entries that leave its state alone
+      rans[256ull * j + t] = make_uint4(0u, 0u, 0u, kRansIdentityTh);
     }
   }
   __syncthreads();

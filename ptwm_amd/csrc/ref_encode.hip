@@ -16,9 +16,8 @@
 //      reciprocal parameters of rans/compress.rs:35-122);
 //   3. Huffman: bits per segment from the segment's histogram and the code
 //      lengths (the histograms are taken per split_four segment); rANS:
-//      each segment encoded by one lane into scratch (ref_rans_kernel; a
-//      segment's state chain is serial by construction, 64 segments run
-//      per wavefront);
+//      each segment encoded into scratch (ref_rans_kernel; a segment's
+//      state chain is serial by construction);
 //   4. host: payload sizes, coded-or-raw decisions, output layout;
 //   5. Huffman segments packed in parallel: every symbol's bit offset is a
 //      prefix sum of code lengths, so each segment is cut into slices of
@@ -34,6 +33,7 @@
 #include <cstring>
 
 #include "code_tables.h"
+#include "ref_rans.h"
 
 namespace ptwm {
 
@@ -266,18 +266,6 @@ constexpr uint32_t kRansEncJobs = kRansEncSegs / 4 + 1;  // job tables a workgro
 constexpr uint32_t kRansEncBatch = 32;                   // steps
 constexpr uint32_t kRansEncThreads = 192;
 
-// Bytes that state x sheds before the symbol of thresholds th: one if
-// x >= freq << 20 and another if x >= freq << 28.  x is below 2^31 and both
-// thresholds' low 16 bits are zero, so the upper half of x decides, below
-// 2^15: th holds (freq << 4) - 1 and (min(freq, 8) << 12) - 1, and the
-// signs of th - (x >> 16) are counted.
-__device__ __forceinline__ uint32_t shed(uint32_t x, uint32_t th) {
-  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-  const u16x2 v = __builtin_bit_cast(u16x2, x);
-  const u16x2 d = __builtin_bit_cast(u16x2, th) - v.yy;
-  return (uint32_t)__builtin_popcount(__builtin_bit_cast(uint32_t, d) & 0x80008000u);
-}
-
 __global__ void __launch_bounds__(kRansEncThreads) ref_rans_kernel(const RefSegDev* __restrict__ segs, uint32_t n_segs,
                                                                    const u32x4* __restrict__ tables,
                                                                    uint8_t* __restrict__ scratch,
@@ -302,8 +290,7 @@ __global__ void __launch_bounds__(kRansEncThreads) ref_rans_kernel(const RefSegD
     rest &= rest - 1;
     const uint32_t jr = (uint32_t)__builtin_amdgcn_readlane((int)S.table, at);
     for (uint32_t i = threadIdx.x; i < 256; i += kRansEncThreads) tab[r][i] = tables[256ull * jr + i];
-    // identity: rcp 0, bias 0, cmpl 0, no byte shed
-    if (threadIdx.x == 0) tab[r][256] = u32x4_make(0u, 0u, 0u, 0x7FFF7FFFu);
+    if (threadIdx.x == 0) tab[r][256] = u32x4_make(0u, 0u, 0u, kRansIdentityTh);
   }
   // Batch b of the segment: the symbols of the aligned block top - b B.
   const uint64_t n = g < n_here ? S.n : 0;
@@ -519,7 +506,7 @@ int64_t RefEncoder::plan(DevCtx& ctx, const std::vector<RefJob>& jobs, std::vect
       g.table = j;
       if (rans) {
         g.scratch_byte = rans_scratch;
-        rans_scratch = align_up(rans_scratch + 4 + 2 * sn[i], 16);
+        rans_scratch = align_up(rans_scratch + ref_rans_scratch(sn[i]), 16);
         ridx.push_back((uint32_t)segs_.size());
         rsegs.push_back(g);
       }

@@ -83,3 +83,22 @@ def test_first_states(kind, state):
             except O.OracleError:
                 want = None
             assert decode(payload, len(plane)) == want
+
+
+def test_refused_tables():
+    """Chunks whose frequencies cannot be normalised (stored raw) between coded ones, in two calls: the second finds
+    the first one's tables in the same rows."""
+    rng = np.random.default_rng(3)
+    refused = np.repeat(np.arange(256, dtype=np.uint8), [353] * 56 + [1] * 200)
+    n = len(refused)
+    rng.shuffle(refused)
+    assert O.codec_encode(O.CODEC_RANS, refused.tobytes())[0] == 0
+    coded = [symbols(k, n, 5) for k in ("rare", "geometric", "one")]
+    assert all(O.codec_encode(O.CODEC_RANS, c.tobytes())[0] == 1 for c in coded)
+    for order in (coded + [refused], [refused, coded[0], refused, coded[1]], [refused] * 4):
+        plane = np.concatenate(order)[:-5]
+        out = torch.zeros(2 * len(plane) + (1 << 16), dtype=torch.uint8, device="cuda:0")
+        print([len(o) for o in order], flush=True)
+        used, _ = api.encode_tensor_ref_cuda(6, [O.CODEC_RANS], n, device(plane), out, 0)
+        want, _ = O.encode_plane_chunked(O.CODEC_RANS, plane.tobytes(), n)
+        assert out[:used].cpu().numpy().tobytes() == want
