@@ -40,9 +40,8 @@ constexpr uint32_t kRansL = 1u << 23;
 // kRansStageGranules 16-byte granules per chain (global loads issued before
 // the round's decode and written to the rings after it) and every chain
 // decodes up to kRansRound symbols from what is staged.
-constexpr uint32_t kRansRing = 2048;
+constexpr uint32_t kRansRing = 1024;
 constexpr uint32_t kRansRingPad = 528;        // a round's 512 bytes and a word read at their end
-constexpr uint32_t kAtMask = 8 * (2 * kRansScale - 1);  // an entry's byte address
 constexpr uint32_t kRansStageGranules = 32;   // 2 per lane: 512 bytes per chain per round
 constexpr uint32_t kRansRound = 256;          // <= 2 bytes per symbol: 512 bytes per chain
 constexpr uint32_t kTansStageWords = 1024;    // tANS stream words staged at a time (4 KiB)
@@ -251,9 +250,9 @@ __device__ void parse_job(const DecodeJob& job, SharedHeader& h) {
 }
 
 // kRans: the rANS jobs (their own launch: its table entries and stream rings
-// take three times the LDS of the other codecs), else every other job of
-// this kernel.
-template <bool kRans>
+// take several times the LDS of the other codecs), else every other job of
+// this kernel.  kFew: the form for few of them (launch_rans_exact).
+template <bool kRans, bool kFew>
 __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __restrict__ jobs,
                                                           uint32_t* __restrict__ status,
                                                           SyncStream* __restrict__ sync_streams,
@@ -262,9 +261,10 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
   __shared__ SharedHeader h;
   __shared__ uint16_t rev[256];
   __shared__ uint8_t sorted_sym[256];              // Huffman: symbols by (length, symbol)
-  // rANS: {2 freq | sym << 24, 2 (slot - start) + bit} per slot and lookahead
-  // bit; Huffman: (len << 8) | sym per window
-  __shared__ __align__(16) uint32_t table_mem[(kRans ? 4 : 1) * kRansScale];
+  // rANS: {freq | sym << 24, slot - start} per slot, with kFew {2 freq |
+  // sym << 24, 2 (slot - start) + bit} per slot and lookahead bit; Huffman:
+  // (len << 8) | sym per window
+  __shared__ __align__(16) uint32_t table_mem[(kRans ? kFew ? 4 : 2 : 1) * kRansScale];
   __shared__ uint8_t hdr_stage[kHdrStage];   // Huffman: weights header and jump table
   uint2* table64 = reinterpret_cast<uint2*>(table_mem);
   uint16_t* table16 = reinterpret_cast<uint16_t*>(table_mem);
@@ -565,18 +565,21 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
     cum[256] = (uint16_t)run;
   }
   __syncthreads();
-  // Slot i of symbol s, as entries 2 i and 2 i + 1 for the state y = 2 x + (a
-  // lookahead bit): {2 freq | s << 24, 2 (i - start) + bit}, so that one
-  // 24-bit multiply-add, 2 freq * (y >> 12) + entry.y, is the state update
-  // and keeps the bit.
+  // Slot i of symbol s: {freq | s << 24, i - start}, so that one 24-bit
+  // multiply-add, freq * (x >> 11) + (i - start), is the state update.  kFew:
+  // entries 2 i and 2 i + 1 for the state y = 2 x + (a lookahead bit), all
+  // doubled and the bit added, so that the same update keeps the bit.
+  constexpr uint32_t kPer = kFew ? 2 : 1;
   for (uint32_t s = lane; s < 256; s += 64) {
-    const uint32_t f = rev[s], st = 2 * cum[s];
-    for (uint32_t j = 0; j < 2 * f; ++j) table64[st + j] = make_uint2(2 * f | (s << 24), j);
+    const uint32_t f = kPer * rev[s], st = kPer * cum[s];
+    for (uint32_t j = 0; j < f; ++j) table64[st + j] = make_uint2(f | (s << 24), j);
   }
-  // The four serial state chains (decompress.rs:80-111).  Chain c runs in
-  // every lane with (lane & 3) == c, the sixteen of them alike and storing
-  // the same bytes: the instructions of a step issue faster with all lanes
-  // active (52 cycles against 63 for eight of them with 16 active).
+  // The four serial state chains (decompress.rs:80-111), chain c in lane c;
+  // with kFew in every lane with (lane & 3) == c, the sixteen of them alike
+  // and storing the same bytes: the instructions of a step issue faster with
+  // all lanes active (52 cycles against 63 for eight of them with 16 active;
+  // past four wavefronts per CU it is the other way round).
+  const bool runs = kFew || lane < 4;
   __shared__ __align__(16) uint8_t ring[4][kRansRing + kRansRingPad];
   uint64_t s4[4], e4[4];
   split_four(job.dst_len, s4, e4);
@@ -587,7 +590,7 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
   const uint64_t out = reinterpret_cast<uint64_t>(dst);
   uint32_t x = 0, q = 4;  // state; next stream byte to read
   bool good = true, done = true, pending = false;
-  if (k != end) {
+  if (runs && k != end) {
     if (sl < 4) good = false;
     else {
       const uint8_t* st = enc + h.seg_src[c];
@@ -647,8 +650,36 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
         // hand the state stays normalised through the stretch and needs no
         // checks.  The bytes it takes are clz(x1) - 1 (1..18) bits rounded
         // down to whole bytes.
-        //
-        // A step's time is its serial chain, so that is kept short.  The
+        // Past four wavefronts per CU the shorter program is the faster one.
+        if (!kFew && x >= kRansL && (int32_t)x >= 0) {
+          uint32_t m = min(end - k, kRansRound - n);
+          m = min(m, (avail - min(q, avail)) / 2);
+          n += m;
+          const uint32_t q0 = 8 * ((q + my_off) & (kRansRing - 1));
+          uint32_t qb = q0;  // ring read position in bits
+          auto step = [&]() -> uint32_t {
+            const uint2 e = table64[x & (kRansScale - 1)];
+            uint16_t b01;
+            __builtin_memcpy(&b01, my_ring + (qb >> 3), 2);
+            const uint32_t x1 = __umul24(e.x, x >> kRansProbBits) + e.y;
+            const uint32_t sh = ((uint32_t)__builtin_clz(x1) - 1u) & ~7u;
+            // [b0 b1 0 0] from the top byte down
+            const uint32_t w = __builtin_amdgcn_perm(0u, (uint32_t)b01, 0x00010C0Cu);
+            x = (uint32_t)(((((uint64_t)x1 << 32) | w) << sh) >> 32);
+            qb += sh;
+            return e.x;
+          };
+          for (; m && ((out + k) & 3u); --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step() >> 24));
+          for (; m >= 4; m -= 4, k += 4) {
+            // the symbols are the entries' top bytes: [a3 b3 d3 f3], low byte first
+            const uint32_t a = step(), b = step(), d = step(), f = step();
+            const uint32_t w = __builtin_amdgcn_perm(b, a, 0x0C0C0703u) | __builtin_amdgcn_perm(f, d, 0x07030C0Cu);
+            g_st<uint32_t>(out + k, w);
+          }
+          for (; m; --m, ++k) g_st<uint8_t>(out + k, (uint8_t)(step() >> 24));
+          q += (qb - q0) / 8;
+        }
+        // Else a step's time is its serial chain, so that is kept short.  The
         // state is held as y = 2 x + b, b the top bit of the next stream
         // byte: clz(y1) is clz(x1) - 1 without the subtraction, and b stays
         // in place through the update because the table is indexed with it.
@@ -659,11 +690,12 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
         // is issued while the read is under way.  A 16 MiB plane in 256 KiB
         // chunks, 65536 steps a chain, takes 3.5 ms (4.5 with the state as x
         // and the other work in the chain).
-        if (x >= kRansL && (int32_t)x >= 0) {
+        if (kFew && x >= kRansL && (int32_t)x >= 0) {
           uint32_t m = min(end - k, kRansRound - n);
           m = min(m, (avail - min(q, avail)) / 2);
           if (m) {
             n += m;
+            constexpr uint32_t kAtMask = 8 * (2 * kRansScale - 1);  // an entry's byte address
             const uint32_t p0 = (q + my_off) & (kRansRing - 1);
             uint32_t qb = 8 * (c * (kRansRing + kRansRingPad) + p0);  // read position in ring[0], in bits
             const uint32_t q0 = qb;
@@ -746,9 +778,9 @@ __global__ void __launch_bounds__(64) decode_exact_kernel(const DecodeJob* __res
         if (k == end) { done = true; break; }
         if (n >= kRansRound) break;
         // one careful symbol (unnormalised start, or the staged bytes' end)
-        const uint2 e = table64[2 * (x & (kRansScale - 1))];
+        const uint2 e = table64[kPer * (x & (kRansScale - 1))];
         g_st<uint8_t>(out + k, (uint8_t)(e.x >> 24));
-        x = __umul24((e.x & 0xFFFFFFu) >> 1, x >> kRansProbBits) + (e.y >> 1);
+        x = __umul24((e.x & 0xFFFFFFu) / kPer, x >> kRansProbBits) + e.y / kPer;
         ++k;
         ++n;
         pending = true;
@@ -1010,8 +1042,8 @@ hipError_t launch_decode_exact(const DecodeJob* jobs_dev, uint32_t* status_dev, 
                                SyncStream* sync_streams, uint16_t* sync_tables, uint64_t* copy_src,
                                hipStream_t stream) {
   if (n_jobs == 0) return hipSuccess;
-  hipLaunchKernelGGL(decode_exact_kernel<false>, dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev, sync_streams,
-                     sync_tables, copy_src);
+  hipLaunchKernelGGL((decode_exact_kernel<false, false>), dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev,
+                     sync_streams, sync_tables, copy_src);
   return hipGetLastError();
 }
 
@@ -1021,11 +1053,22 @@ hipError_t launch_tans_decode(const DecodeJob* jobs_dev, uint32_t* status_dev, u
   return hipGetLastError();
 }
 
-hipError_t launch_rans_exact(const DecodeJob* jobs_dev, uint32_t* status_dev, uint32_t n_jobs, uint64_t* copy_src,
-                             hipStream_t stream) {
+// The kernel has two forms.  kFew takes 40 KB of LDS, four workgroups per CU,
+// and a chunk is the faster for it while all of them run at once; the other
+// takes 24 KB, six per CU, and is not slowed by the two wavefronts that then
+// share a SIMD.  So the line lies where the first would need a second round.  A
+// plane in 256 KiB chunks, ms in the first and in the second form: 256 chunks
+// 3.5 and 4.5, 1024 chunks 5.4 and 7.0, 1536 chunks 10.6 and 4.5, 6144 chunks
+// 32 and 17.5 (256 CUs).
+hipError_t launch_rans_exact(const DecodeJob* jobs_dev, uint32_t* status_dev, uint32_t n_jobs, uint32_t n_rans,
+                             uint32_t cu_count, uint64_t* copy_src, hipStream_t stream) {
   if (n_jobs == 0) return hipSuccess;
-  hipLaunchKernelGGL(decode_exact_kernel<true>, dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev, nullptr,
-                     nullptr, copy_src);
+  if (n_rans <= 4 * cu_count)
+    hipLaunchKernelGGL((decode_exact_kernel<true, true>), dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev,
+                       nullptr, nullptr, copy_src);
+  else
+    hipLaunchKernelGGL((decode_exact_kernel<true, false>), dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev,
+                       nullptr, nullptr, copy_src);
   return hipGetLastError();
 }
 

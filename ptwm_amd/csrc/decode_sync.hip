@@ -883,15 +883,16 @@ int64_t decode_jobs_launch(DevCtx& ctx, DecodeJob* hj, size_t n_jobs, ExactRun& 
   if (any_tans) PTWM_HIP_TRY(launch_tans_decode(d_jobs, status, (uint32_t)n_jobs, s));
   // reference rANS payloads are a few long serial chains: they run on the
   // side stream while this stream decodes everything else
-  bool any_rans = false;
-  for (size_t j = 0; j < n_jobs; ++j) any_rans |= hj[j].codec == kCodecRans;
-  if (any_rans) {
+  uint32_t n_rans = 0;
+  for (size_t j = 0; j < n_jobs; ++j) n_rans += hj[j].codec == kCodecRans;
+  if (n_rans) {
     PTWM_HIP_TRY(ctx.ensure_side());
     PTWM_HIP_TRY(hipEventRecord(ctx.side_fork, s));
     PTWM_HIP_TRY(hipStreamWaitEvent(ctx.side_stream, ctx.side_fork, 0));
     // (stored-bytes payloads of rANS jobs are copied by that kernel itself:
     // raw_copy_kernel on this stream does not wait for the side stream)
-    PTWM_HIP_TRY(launch_rans_exact(d_jobs, status, (uint32_t)n_jobs, nullptr, ctx.side_stream));
+    PTWM_HIP_TRY(launch_rans_exact(d_jobs, status, (uint32_t)n_jobs, n_rans,
+                                   ctx.cu_count > 0 ? (uint32_t)ctx.cu_count : 256u, nullptr, ctx.side_stream));
     PTWM_HIP_TRY(hipEventRecord(ctx.side_join, ctx.side_stream));
   }
   bool any_o1sac = false;
@@ -917,7 +918,7 @@ int64_t decode_jobs_launch(DevCtx& ctx, DecodeJob* hj, size_t n_jobs, ExactRun& 
     }
     PTWM_HIP_TRY(sync_finish(s, streams, d_wave_job, d_job_wave0, tables, A, nw, n_def, status, run.out_stage));
   }
-  if (any_rans) PTWM_HIP_TRY(hipStreamWaitEvent(s, ctx.side_join, 0));
+  if (n_rans) PTWM_HIP_TRY(hipStreamWaitEvent(s, ctx.side_join, 0));
   run.jobs = d_jobs;
   run.status = status;
   run.streams = streams;

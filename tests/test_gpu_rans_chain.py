@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from ptwm_amd import api, ids
+from ptwm_amd import api, ids, plan
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -102,3 +102,60 @@ def test_refused_tables():
         used, _ = api.encode_tensor_ref_cuda(6, [O.CODEC_RANS], n, device(plane), out, 0)
         want, _ = O.encode_plane_chunked(O.CODEC_RANS, plane.tobytes(), n)
         assert out[:used].cpu().numpy().tobytes() == want
+
+
+def cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("extra", [0, 1, 700])
+def test_decode_chunk_counts(extra):
+    """Chunks around the line between the decoder's two forms (four per CU), of any alphabet and alignment."""
+    chunks, size = 4 * cus() + extra, 2061
+    kinds = ["one", "rare", "flat", "geometric"]
+    plane = np.concatenate([symbols(kinds[c % 4], size, c) for c in range(chunks)])[:-9]
+    payload, entries = O.encode_plane_chunked(O.CODEC_RANS, plane.tobytes(), size)
+    n = len(plane)
+    st = plan.encode_plan([plan.TensorPlan(plan.CHAIN_PASSTHROUGH, 0, n, [
+        plan.PlanePlan(O.CODEC_RANS, 0, len(payload), n, [tuple(map(int, e)) for e in entries])])])
+    out = torch.zeros(n, dtype=torch.uint8, device="cuda:0")
+    print(chunks, flush=True)
+    api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, st,
+                                              device(np.frombuffer(payload, np.uint8)), out, 0)
+    assert out.cpu().numpy().tobytes() == plane.tobytes()
+
+
+@pytest.mark.parametrize("state", [0, (1 << 23) - 1, 1 << 23, (1 << 31) - 1, 1 << 31, (1 << 32) - 1])
+@pytest.mark.parametrize("kind", ["one", "rare", "geometric"])
+def test_first_states_of_one_among_many(kind, state):
+    """As test_first_states, in the form for many chunks: the last of a call's payloads is the altered one."""
+    src = symbols(kind, 5000, 11)
+    good = O.codec_encode(O.CODEC_RANS, src.tobytes())
+    at = 5 + 1 + 2 * (good[5] + 1)
+    lens = np.frombuffer(good[at:at + 16], "<u4")
+    count, room = 4 * cus() + 1, 5008
+    for seg in (0, 3):
+        bad = bytearray(good)
+        first = at + 16 + int(lens[:seg].sum())
+        bad[first:first + 4] = int(state).to_bytes(4, "little")
+        for payload in (bytes(bad), bytes(bad[:-1]), bytes(bad) + b"\x5a"):
+            tensors = [plan.TensorPlan(plan.CHAIN_PASSTHROUGH, room * k, len(src), [
+                plan.PlanePlan(O.CODEC_RANS, 0, len(good), len(src))]) for k in range(count)]
+            tensors[-1].planes[0].payload_offset = len(good)
+            tensors[-1].planes[0].payload_len = len(payload)
+            out = torch.zeros(room * count, dtype=torch.uint8, device="cuda:0")
+            print(kind, state, seg, len(payload), flush=True)
+            try:
+                want = O.codec_decode(O.CODEC_RANS, payload, len(src))
+            except O.OracleError:
+                want = None
+            try:
+                api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL,
+                                                          plan.encode_plan(tensors),
+                                                          device(np.frombuffer(good + payload, np.uint8)), out, 0)
+                got = out.view(count, room)[:, :len(src)].cpu().numpy()
+            except Exception:  # noqa: BLE001
+                got = None
+            assert (got is None) == (want is None)
+            if want is not None:
+                assert (got[:-1] == src).all() and got[-1].tobytes() == want
