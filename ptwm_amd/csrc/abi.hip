@@ -99,8 +99,10 @@ struct DeviceScope {
     ctx->stream = t_stream.set && t_stream.dev == ord ? reinterpret_cast<hipStream_t>(t_stream.stream) : ctx->own_stream;
     (void)hipGetDevice(&prev);
     ok = hipSetDevice(ctx->dev) == hipSuccess;
+    DeviceBuffer::spare = &ctx->enc_keep;
   }
   ~DeviceScope() {
+    DeviceBuffer::spare = nullptr;
     if (ctx && prev >= 0) (void)hipSetDevice(prev);
   }
 };

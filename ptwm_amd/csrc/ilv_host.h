@@ -60,6 +60,9 @@ int64_t ilv_upload_begin(DevCtx& ctx, const uint64_t* src, const uint64_t* n, ui
                          const IlvEncResult* res, const uint32_t* form, const uint64_t* head_len, size_t block_bytes,
                          IlvUpload& u);
 int64_t ilv_upload_send(DevCtx& ctx, const IlvUpload& u);
+// The most bytes that it takes for np planes and block_bytes of block list,
+// the coded planes' heads apart.
+size_t ilv_upload_bound(uint32_t np, size_t block_bytes);
 
 // np rows of 256 zeros in ctx.enc_hist, for counts that the encoders take with
 // `counted`; nullptr on an error.

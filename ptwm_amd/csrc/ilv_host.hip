@@ -110,6 +110,13 @@ int64_t ilv_upload_begin(DevCtx& ctx, const uint64_t* src, const uint64_t* n, ui
   return kOk;
 }
 
+size_t ilv_upload_bound(uint32_t np, size_t block_bytes) {
+  // per plane a pack and a head job or a store job, and a head; each piece
+  // rounded up to 16
+  return np * (sizeof(IlvPackJob) + 2 * sizeof(IlvStoreJob) + align_up(kPackedHeadBytes, 16) + 16) + 4 * 16 +
+         align_up(block_bytes, 16);
+}
+
 int64_t ilv_upload_send(DevCtx& ctx, const IlvUpload& u) {
   if (!u.bytes) return kOk;
   hipStream_t s = ctx.stream;

@@ -19,7 +19,7 @@
 
 namespace ptwm {
 
-// Blocks whose words the size pass keeps: 1 GiB of scratch at most, which is
+// Blocks whose words the size pass keeps: 1032 MiB of scratch at most, for
 // 512 MiB of planes.  Blocks past them, and all where the scratch cannot be
 // had, are encoded twice.
 constexpr uint32_t kRilvKeepBlocks = 32 << 10;
@@ -80,13 +80,19 @@ int64_t rilv_encode_planes(DevCtx& ctx, const uint64_t* src, const uint64_t* n, 
   PTWM_HIP_TRY(ctx.h_sizes.ensure(nblk * sizeof(uint32_t)));
   uint32_t* const bwords = static_cast<uint32_t*>(ctx.h_sizes.ptr);
   uint32_t kept = std::min(nblk, kRilvKeepBlocks);
-  if (kept && ctx.enc_keep.ensure(kept * kRilvKeepBytes) != hipSuccess) {
-    (void)hipGetLastError();
-    kept = 0;
-  }
   if (nblk) {
+    // all that the encode cannot do without, the last pass's upload at its
+    // largest included, before the blocks' words (DeviceBuffer::spare)
     PTWM_HIP_TRY(ctx.enc_blocks.ensure(nblk * sizeof(RilvEncBlock)));
     PTWM_HIP_TRY(ctx.enc_block_bytes.ensure(nblk * sizeof(uint32_t)));
+    size_t pack = ilv_upload_bound(np, nblk * sizeof(RilvEncBlock));
+    for (uint32_t p = 0; p < np; ++p)
+      if (codable[p]) pack += align_up(5 + (uint64_t)info[p].head_len, 4) + 4 * ((uint64_t)nbs[p] + 1);
+    PTWM_HIP_TRY(ctx.enc_pack.ensure(pack));
+    if (kept && ctx.enc_keep.ensure(kept * kRilvKeepBytes) != hipSuccess) {
+      (void)hipGetLastError();
+      kept = 0;
+    }
     PTWM_HIP_TRY(ctx.h_enc.ensure(nblk * sizeof(RilvEncBlock)));
     std::memcpy(ctx.h_enc.ptr, blocks.data(), nblk * sizeof(RilvEncBlock));
     PTWM_HIP_TRY(

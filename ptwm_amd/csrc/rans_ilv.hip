@@ -26,9 +26,10 @@
 // plus the lane's rank among the lanes that renormalise (mbcnt).  Rounds
 // end in the same merge and dwordx4 stores as huff_ilv.
 //
-// Encode: histogram (shared with huff_ilv), host normalisation, a size pass
-// (one wavefront per block runs the encoder and counts words), host layout,
-// and a write pass that runs the encoder again and writes each step's words
+// Encode: histogram and frequency tables (code_tables.hip), a size pass (one
+// wavefront per block runs the encoder, counts its words and keeps them where
+// there is room), host layout, and a write pass that copies the kept blocks to
+// their places and runs the encoder again for the others, each step's words
 // below the previous step's (the decoder reads the stream forward).
 #include "rans_ilv.h"
 

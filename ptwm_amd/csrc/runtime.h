@@ -18,6 +18,10 @@ namespace ptwm {
 // decode's fixed scratch): ensure() never allocates for it and fails when
 // the view is too small.
 struct DeviceBuffer {
+  // The calling thread's context's buffer that calls can do without
+  // (DevCtx::enc_keep; set by its DeviceScope): ensure() frees it where memory
+  // is short, so whoever uses it allocates nothing else until it is done.
+  static thread_local DeviceBuffer* spare;
   void* ptr = nullptr;
   size_t cap = 0;
   bool borrowed = false;

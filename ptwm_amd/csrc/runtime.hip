@@ -28,6 +28,8 @@ std::atomic<uint64_t> g_alloc_calls{0};
 void note_alloc() { g_alloc_calls.fetch_add(1, std::memory_order_relaxed); }
 uint64_t alloc_calls() { return g_alloc_calls.load(std::memory_order_relaxed); }
 
+thread_local DeviceBuffer* DeviceBuffer::spare = nullptr;
+
 hipError_t DeviceBuffer::ensure(size_t bytes) {
   if (bytes <= cap && ptr) return hipSuccess;
   if (borrowed) return hipErrorOutOfMemory;
@@ -39,7 +41,15 @@ hipError_t DeviceBuffer::ensure(size_t bytes) {
   size_t want = bytes < 4096 ? 4096 : bytes;
   note_alloc();
   hipError_t e = hipMalloc(&ptr, want);
+  if (e != hipSuccess && spare && spare != this && spare->ptr) {
+    (void)hipGetLastError();
+    (void)hipFree(spare->ptr);
+    spare->ptr = nullptr;
+    spare->cap = 0;
+    e = hipMalloc(&ptr, want);
+  }
   if (e == hipSuccess) cap = want;
+  else ptr = nullptr;
   return e;
 }
 DeviceBuffer::~DeviceBuffer() {}

@@ -81,3 +81,29 @@ def test_blocks_past_the_kept_ones():
     part = bytes(h) + (table[lo:hi + 1] - table[lo]).astype(np.uint32).tobytes() + \
         out[data + int(table[lo]):data + int(table[hi])].cpu().numpy().tobytes()
     assert O.rans_ilv_decode(part, (hi - lo) * BLOCK) == d[lo * BLOCK:hi * BLOCK].cpu().numpy().tobytes()
+
+
+def test_kept_words_are_given_back():
+    """A call that needs more scratch than the card has left gets what the kept words of an earlier call hold, and
+    encodes its blocks twice.  Both tensors are larger than any that another test encodes, so that their planes'
+    scratch is allocated here; some 300 MiB stay free throughout."""
+    mib = 1 << 20
+    n, before = 6 << 30, 9 << 29
+    a = (torch.randn(32 * mib, device="cuda:0") * 0.02).to(torch.bfloat16).view(torch.uint8).repeat(n // (64 * mib))
+    out = torch.zeros(n, dtype=torch.uint8, device="cuda:0")
+    back = torch.zeros(n, dtype=torch.uint8, device="cuda:0")
+    torch.cuda.empty_cache()
+    api.encode_tensor_cuda(plan.CHAIN_IEEE16_SPLIT2, a[:before], out, 0, codec="rans_ilv")  # keeps all it may
+    free = torch.cuda.mem_get_info()[0]
+    filler = torch.empty(free - (n - before - 700 * mib), dtype=torch.uint8, device="cuda:0")
+    print("free", torch.cuda.mem_get_info()[0] // mib, "MiB, needed", (n - before) // mib, flush=True)
+    try:
+        used, state = api.encode_tensor_cuda(plan.CHAIN_IEEE16_SPLIT2, a, out, 0, codec="rans_ilv")
+    finally:
+        del filler
+        torch.cuda.empty_cache()
+    p = plan.decode_plan(state)[0].planes[1]
+    assert p.codec == ids.CODEC_RANS_ILV and p.payload_len < n // 4
+    api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, state, out[:used],
+                                              back, 0)
+    assert torch.equal(back, a)
