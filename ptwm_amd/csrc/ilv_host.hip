@@ -551,10 +551,11 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
   if (!any_retry) return kOk;
   if (all_slots) return kInternal;
   // a tensor without its sums again, and with it the chunks that share them
+  std::vector<char> sums_lost(n_acc, 0);
   for (size_t i = 0; i < nt; ++i)
-    if (retry[i] && tensors[i].crc_ix != kIlvNoCrc)
-      for (size_t k = 0; k < nt; ++k)
-        if (tensors[k].crc_ix == tensors[i].crc_ix) retry[k] = 1;
+    if (retry[i] && tensors[i].crc_ix != kIlvNoCrc) sums_lost[tensors[i].crc_ix] = 1;
+  for (size_t i = 0; i < nt; ++i)
+    if (tensors[i].crc_ix != kIlvNoCrc && sums_lost[tensors[i].crc_ix]) retry[i] = 1;
   std::vector<IlvTensor> again;
   std::vector<uint32_t> again_ix;
   for (size_t i = 0; i < nt; ++i)

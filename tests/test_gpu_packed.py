@@ -182,3 +182,52 @@ def test_coded_payload_with_stored_or_packed_length(name, label, enc, wire, targ
     got = api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, st,
                                                     dev(bytes(blob)), restored, 0)
     assert got == len(data) and host(restored) == data
+
+
+@pytest.mark.parametrize("name,label,enc,wire,target,ns,gen", COLLISIONS[::2], ids=[c[0] for c in COLLISIONS[::2]])
+def test_retries_keep_every_sum(name, label, enc, wire, target, ns, gen):
+    """Plane CRCs of a call where some tensors are decoded again: tensors of one plane, chunked ones (all chunks of a
+    retried chunk's tensor go again) and ones that are not retried, each checked and each refused for a wrong CRC."""
+    x, payload = _collision(enc, target, ns, gen)
+    n = len(x)
+    other = np.minimum(np.random.default_rng(99).geometric(0.3, 16384), 255).astype(np.uint8).tobytes()
+    p1 = enc(other)
+    assert p1[0] == 1 and len(p1) not in (16385, 8 + 8192)
+    frame = b"\0\0\0\0\0"
+    blob = bytearray(payload)
+    offs = {"retried": 0}
+    for k, b in (("plain", p1), ("chunks", b"\0\0\0" + frame + p1 + frame + payload)):
+        blob += b"\0" * (-len(blob) % 256)
+        offs[k] = len(blob)
+        blob += b
+    second = 5 + len(p1)
+    tensors, want = [], []
+    for k in range(90):
+        o = sum((len(w) + 255) // 256 * 256 for w in want)
+        if k % 3 == 0:
+            data, p = x, plan.PlanePlan(wire, 0, len(payload), n)
+        elif k % 3 == 1:
+            data, p = other, plan.PlanePlan(wire, offs["plain"], len(p1), 16384)
+        else:
+            data = other + x
+            p = plan.PlanePlan(wire, offs["chunks"] + 3, second + 5 + len(payload), 16384 + n, [(0, 16384), (second, n)])
+        p.crc32 = O.crc32(data)
+        tensors.append(plan.TensorPlan(plan.CHAIN_PASSTHROUGH, o, len(data), [p]))
+        want.append(data)
+    restored = torch.zeros(tensors[-1].out_offset + tensors[-1].out_len, dtype=torch.uint8, device="cuda:0")
+    src = dev(bytes(blob))
+
+    def decode():
+        api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL,
+                                                  plan.encode_plan(tensors), src, restored, 0)
+        return host(restored)
+
+    got = decode()
+    for t, w in zip(tensors, want):
+        assert got[t.out_offset:t.out_offset + t.out_len] == w
+    for t in tensors[-3:]:
+        t.planes[0].crc32 ^= 1
+        with pytest.raises(Exception) as e:
+            decode()
+        assert getattr(e.value, "rc", None) == -1
+        t.planes[0].crc32 ^= 1
