@@ -9,135 +9,175 @@
 // tensor.  Here all tables of a call are built at once.
 //
 // The tree: leaves sorted by (count, symbol) by counting the smaller ones,
-// then the two-queue merge, the only serial part: a step per symbol, four LDS
-// reads that depend on the step before, 0.14 us each, run by all threads
-// alike.  Where many items are no larger than the two smallest together, none
-// of the nodes made of them can come before any of them, so they are paired
-// all at once (a flat 256-symbol alphabet takes 5 such rounds and some 20
-// steps instead of 255).  Depths by pointer jumping; the rest is a few ballots.
+// then the two-queue merge, the only serial part.  Its steps depend on each
+// other, but none of the nodes made of the items that are no larger than the
+// two smallest together can come before any of these items, so they are
+// paired all at once: rounds of 0.3 us, by one wavefront, which needs no
+// barriers for them.  (A step a pair, by four wavefronts with barriers around
+// rounds of 16 items or more, took 0.22 us a pair: 29 of the 43 us of a
+// 142-symbol table.)  Depths by pointer jumping; the rest is a few ballots.
 #include "code_tables.h"
 
-#include "huffman_merge.h"
 #include "ref_rans.h"
 
 namespace ptwm {
 
 namespace {
 
-constexpr uint32_t kNone = kMergeNone;
+constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr uint32_t kScale = 2048;     // rANS frequencies sum to 2^11
 constexpr uint32_t kThreads = 256;
-constexpr uint32_t kRound = kMergeRound;
 
 struct Scratch {
-  u32x4 f4[64];                 // counts by symbol
-  uint32_t leaf[256 + kRound];  // counts of the sorted leaves, then kNone
-  uint32_t node[256 + kRound];  // counts of the internal nodes, in creation order
-  uint32_t order[256];          // a round's counts in order
-  uint16_t up[512];             // parent: leaf i at i, internal node q at 256 + q
-  uint16_t dist[512];           // edges to `up`
-  uint8_t sym[256];             // symbol of leaf i
-  uint8_t len[256];             // code length by symbol
-  uint32_t head[132];           // header bytes, 4-byte aligned
-  uint32_t count[4][12];        // per wavefront: symbols of each length
+  u32x4 f4[64];             // nonzero counts by symbol, then kNone
+  uint32_t leaf[256 + 64];  // counts of the sorted leaves, then kNone
+  uint32_t node[256 + 64];  // counts of the internal nodes, in creation order
+  uint32_t order[128];      // a round's counts in order
+  uint16_t up[512];         // parent: leaf i at i, internal node q at 256 + q
+  uint16_t dist[512];       // edges to `up`
+  uint8_t sym[256];         // symbol of leaf i
+  uint8_t len[256];         // code length by symbol
+  uint32_t head[132];       // header bytes, 4-byte aligned
+  uint32_t count[4][16];    // per wavefront: symbols of each length
+  uint64_t used[4];         // per wavefront: the symbols with nonzero counts
   uint64_t part[4];
 };
 
-// Sum, minimum and maximum over the workgroup (every thread calls).
+// Over the wavefront, in lane 63 (all lanes active): rows of 16 by row shifts,
+// then broadcasts of rows 0, 2 (to 1, 3) and of row 1 (to 2, 3).
+template <uint32_t kCtrl, uint32_t kRows>
+__device__ __forceinline__ uint32_t dpp(uint32_t old, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRows, 0xF, false);
+}
+__device__ __forceinline__ uint32_t wave_sum63(uint32_t v) {
+  v += dpp<0x111, 0xF>(0, v);
+  v += dpp<0x112, 0xF>(0, v);
+  v += dpp<0x114, 0xF>(0, v);
+  v += dpp<0x118, 0xF>(0, v);
+  v += dpp<0x142, 0xA>(0, v);
+  return v + dpp<0x143, 0xC>(0, v);
+}
+__device__ __forceinline__ uint32_t wave_min63(uint32_t v) {
+  v = min(v, dpp<0x111, 0xF>(kNone, v));
+  v = min(v, dpp<0x112, 0xF>(kNone, v));
+  v = min(v, dpp<0x114, 0xF>(kNone, v));
+  v = min(v, dpp<0x118, 0xF>(kNone, v));
+  v = min(v, dpp<0x142, 0xA>(kNone, v));
+  return min(v, dpp<0x143, 0xC>(kNone, v));
+}
+
+// Sum (of values below 2^48) and minimum over the workgroup (every thread
+// calls).
 __device__ __forceinline__ uint64_t sum_all(Scratch& S, uint64_t v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor((unsigned long long)v, d, 64);
+  const uint32_t lo = wave_sum63((uint32_t)v & 0xFFFFFFu), hi = wave_sum63((uint32_t)(v >> 24));
   __syncthreads();
-  if ((threadIdx.x & 63u) == 0) S.part[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63u) == 63u) S.part[threadIdx.x >> 6] = lo + ((uint64_t)hi << 24);
   __syncthreads();
   return S.part[0] + S.part[1] + S.part[2] + S.part[3];
 }
 __device__ __forceinline__ uint32_t min_all(Scratch& S, uint32_t v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v = min(v, (uint32_t)__shfl_xor(v, d, 64));
+  v = wave_min63(v);
   __syncthreads();
-  if ((threadIdx.x & 63u) == 0) S.part[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63u) == 63u) S.part[threadIdx.x >> 6] = v;
   __syncthreads();
   return (uint32_t)min(min(S.part[0], S.part[1]), min(S.part[2], S.part[3]));
 }
 
-// Items of the ascending list a[lo .. hi) below v (kEqual: or equal to it).
-template <bool kEqual>
-__device__ __forceinline__ uint32_t below(const uint32_t* a, uint32_t lo, uint32_t hi, uint32_t v) {
-  const uint32_t lo0 = lo;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (kEqual ? a[mid] <= v : a[mid] < v) lo = mid + 1;
-    else hi = mid;
+__device__ __forceinline__ uint32_t lane_of(uint32_t v, uint32_t lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
+}
+
+// What lanes of this wavefront wrote to LDS is there for its other lanes.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The two-queue merge of n >= 2 leaves, by one wavefront: S.up of all but the
+// root.  Two FIFO queues: the sorted leaves [li, n) and the internal nodes
+// [qi, qe), whose counts never decrease in creation order; a leaf goes first on
+// ties (its id is smaller).  Each round takes up to 64 items of either queue.
+// Counts of up to 2^32 - 1 bytes in all stay below kNone until the last pair.
+__device__ __forceinline__ void merge_leaves(Scratch& S, uint32_t n) {
+  const uint32_t lane = threadIdx.x;
+  n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
+  uint32_t li = 0, qi = 0, qe = 0;
+  while (n - li + (qe - qi) > 1) {
+    const uint32_t nl = n - li, nq = qe - qi;
+    const uint32_t a = S.leaf[li + lane], b = lane < nq ? S.node[qi + lane] : kNone;
+    // the two smallest together, and the items no larger than that: the first
+    // cl leaves and ci nodes
+    const uint32_t l0 = lane_of(a, 0), l1 = lane_of(a, 1), i0 = lane_of(b, 0), i1 = lane_of(b, 1);
+    const uint32_t both = min(min(__builtin_elementwise_add_sat(l0, l1), __builtin_elementwise_add_sat(l0, i0)),
+                              __builtin_elementwise_add_sat(i0, i1));
+    uint32_t cl = min((uint32_t)__popcll(__ballot(a <= both)), nl);
+    uint32_t ci = min((uint32_t)__popcll(__ballot(b <= both)), nq);
+    if (max(cl, ci) == 64) {  // more may follow: up to the last that surely goes before those
+      const uint32_t al = cl == 64 ? lane_of(a, 63) : kNone, bl = ci == 64 ? lane_of(b, 63) : kNone;
+      if (al <= bl) ci = (uint32_t)__popcll(__ballot(b < al));
+      else cl = (uint32_t)__popcll(__ballot(a <= bl));
+    }
+    // their ranks among each other
+    uint32_t ra = lane, rb = lane;
+    const uint32_t both_kinds = cl ? ci : 0;
+    for (uint32_t j0 = 0; j0 < both_kinds; j0 += 4)  // (past ci: larger than any of the leaves)
+#pragma unroll
+      for (uint32_t j = j0; j < j0 + 4; ++j) {
+        const uint32_t v = lane_of(b, j);
+        ra += a > v ? 1u : 0u;
+        const uint32_t at = j + (uint32_t)__popcll(__ballot(a <= v));
+        rb = lane == j ? at : rb;
+      }
+    // in pairs, in order; an odd last one stays, and gets its parent later
+    const uint32_t items = cl + ci, pairs = items / 2, odd = items & 1u;
+    if (lane < cl) {
+      S.order[ra] = a;
+      S.up[li + lane] = (uint16_t)(256u + qe + ra / 2);
+    }
+    if (lane < ci) {
+      S.order[rb] = b;
+      S.up[256u + qi + lane] = (uint16_t)(256u + qe + rb / 2);
+    }
+    wave_sync();
+    const uint32_t sum = S.order[2 * lane] + S.order[2 * lane + 1];
+    S.node[qe + lane] = sum;  // (what is past the pairs is not in the queue)
+    wave_sync();
+    const uint32_t odd_leaf = odd && lane_of(ra, (cl - 1) & 63u) == items - 1 ? 1u : 0u;
+    li += cl - odd_leaf;
+    qi += ci - (odd - odd_leaf);
+    qe += pairs;
   }
-  return lo - lo0;
 }
 
 // Code length of symbol t (tree.rs:19-85, 212-242), its count h; n symbols
-// have nonzero counts.
-__device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t n, uint32_t max_len) {
+// have nonzero counts, `below` of them come before t.
+__device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t below, uint32_t n, uint32_t max_len) {
   const uint32_t t = threadIdx.x;
   if (n == 1) return h ? 1u : 0u;
-  reinterpret_cast<uint32_t*>(S.f4)[t] = h;
-  for (uint32_t i = t; i < 256 + kRound; i += kThreads) S.leaf[i] = kNone;
+  uint32_t* const counts = reinterpret_cast<uint32_t*>(S.f4);
+  if (h) counts[below] = h;
+  if (t >= n) counts[t] = kNone;
+  for (uint32_t i = t; i < 256 + 64; i += kThreads) S.leaf[i] = kNone;
   S.len[t] = 0;
   __syncthreads();
-  // rank: symbols with (count, symbol) below this one's; a count of zero
-  // wraps to the largest value
+  // rank: symbols with (count, symbol) below this one's
   uint32_t rank = 0;
-#pragma unroll 4
-  for (uint32_t j = 0; j < 64; ++j) {
+#pragma unroll 8
+  for (uint32_t j = 0; 4 * j < n; ++j) {
     const u32x4 f = S.f4[j];
+    const uint32_t limit = h + (j < below / 4 ? 1u : 0u);
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) rank += f[i] - 1u < h - 1u + (4 * j + i < t ? 1u : 0u) ? 1u : 0u;
+    for (uint32_t i = 0; i < 4; ++i) rank += f[i] < limit ? 1u : 0u;
   }
+#pragma unroll
+  for (uint32_t i = 0; i < 3; ++i) rank += i < below % 4 && S.f4[below / 4 & 63u][i] == h ? 1u : 0u;
   if (h) {
     S.leaf[rank] = h;
     S.sym[rank] = (uint8_t)t;
   }
   __syncthreads();
-  // Two FIFO queues: the sorted leaves and the internal nodes; a leaf goes
-  // first on ties (its id is smaller).  Every thread takes every step: the
-  // writes are alike, each thread uses only what it wrote itself since the
-  // last barrier (merge_step), and so all wavefronts reach the same rounds and
-  // the same end.  Counts of up to 2^32 - 1 bytes in all stay below kNone
-  // until the last pair.
-  MergeQueues m{0, 0, 0};
-  while (n - m.li + (m.qe - m.qi) > 1) {
-    const MergeStep step = merge_step(S.leaf, S.node, m);
-    const uint32_t li = m.li, qi = m.qi, qe = m.qe, both = step.both;
-    if (step.round) {
-      // a round: the items no larger than `both`, in order, in pairs; an odd
-      // last one stays
-      __syncthreads();  // (every wavefront has made its steps before)
-      const uint32_t cl = below<true>(S.leaf, li, n, both), ci = below<true>(S.node, qi, qe, both);
-      const uint32_t pairs = (cl + ci) / 2;
-      if (t < cl) {
-        const uint32_t f = S.leaf[li + t], r = t + below<false>(S.node, qi, qi + ci, f);
-        S.order[r & 255u] = f;
-        if (r < 2 * pairs) S.up[li + t] = (uint16_t)(256u + qe + r / 2);
-      }
-      if (t < ci) {
-        const uint32_t f = S.node[qi + t], r = t + below<true>(S.leaf, li, li + cl, f);
-        S.order[r & 255u] = f;
-        if (r < 2 * pairs) S.up[256u + qi + t] = (uint16_t)(256u + qe + r / 2);
-      }
-      const bool odd = (cl + ci) & 1u;
-      const bool last_leaf = cl && (!ci || S.leaf[li + cl - 1] > S.node[qi + ci - 1]);
-      __syncthreads();
-      if (t < pairs) S.node[qe + t] = S.order[2 * t] + S.order[2 * t + 1];
-      m.li += cl - (odd && last_leaf ? 1u : 0u);
-      m.qi += ci - (odd && !last_leaf ? 1u : 0u);
-      m.qe += pairs;
-      __syncthreads();
-      continue;
-    }
-    const uint32_t a = step.a_leaf ? li : 256u + qi;
-    const uint32_t b = step.b_leaf ? li + (step.a_leaf ? 1u : 0u) : 256u + qi + (step.a_leaf ? 0u : 1u);
-    S.node[qe] = both;
-    S.up[a] = S.up[b] = (uint16_t)(256u + qe);
-    m = merge_next(m, step);
-  }
+  if (t < 64) merge_leaves(S, n);
   const uint32_t root = 256u + n - 2u;
   __syncthreads();
   // depths: every node's pointer jumps to its pointer's, distances add
@@ -172,42 +212,52 @@ __device__ uint32_t huffman_length(Scratch& S, uint32_t h, uint32_t n, uint32_t 
   const bool clamped = __syncthreads_or(over);
   uint32_t l = S.len[t];
   if (!clamped) return l;
-  for (;;) {
-    const uint32_t kraft = (uint32_t)sum_all(S, l ? 1u << (max_len - l) : 0u);
+  uint32_t kraft = (uint32_t)sum_all(S, l ? 1u << (max_len - l) : 0u);
+  while (kraft > 1u << max_len) {
     const uint32_t best = min_all(S, l && l < max_len ? l << 8 | t : kNone);
-    if (kraft <= 1u << max_len || best == kNone) return l;
+    if (best == kNone) break;
     if ((best & 255u) == t) ++l;
+    kraft -= 1u << (max_len - 1u - (best >> 8));
   }
+  return l;
 }
 
 // Canonical bit-reversed code of symbol t (tree.rs:102-177); false if the
 // lengths form no code.
 __device__ bool canonical(Scratch& S, uint32_t l, uint32_t& rev) {
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  uint32_t rank = 0;
-#pragma unroll
+  // lane b: this wavefront's symbols of length b
+  uint32_t rank = 0, mine = 0;
+#pragma unroll 1
   for (uint32_t b = 1; b <= 11; ++b) {
     const uint64_t m = __ballot(l == b);
     if (l == b) rank = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) S.count[wave][b] = (uint32_t)__popcll(m);
+    if (lane == b) mine = (uint32_t)__popcll(m);
   }
+  if (lane < 16) S.count[wave][lane] = mine;
   __syncthreads();
+  // lane b: the first code of length b, and the symbols of it in the
+  // wavefronts before this one
+  uint32_t count = 0, before = 0, first = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    const uint32_t c = S.count[w][lane & 15u];
+    count += c;
+    before += w < wave ? c : 0u;
+  }
   uint32_t code = 0, prev = 0;
   bool ok = true;
-  rev = 0;
-#pragma unroll
+#pragma unroll 1
   for (uint32_t b = 1; b <= 11; ++b) {
-    const uint32_t count = S.count[0][b] + S.count[1][b] + S.count[2][b] + S.count[3][b];
-    code = (code + prev) << 1;  // first code of length b
+    const uint32_t c = lane_of(count, b);
+    code = (code + prev) << 1;
+    if (lane == b) first = code;
     // (past the longest length the reference does not look)
-    if (count && code + count > (1u << b)) ok = false;
-    if (l == b) {
-      uint32_t c = code + rank;
-      for (uint32_t w = 0; w < wave; ++w) c += S.count[w][b];
-      rev = __builtin_bitreverse32(c) >> (32u - b);
-    }
-    prev = count;
+    if (c && code + c > (1u << b)) ok = false;
+    prev = c;
   }
+  const uint32_t at = (uint32_t)__shfl((int)(first + before), (int)l, 64) + rank;
+  rev = l ? __builtin_bitreverse32(at) >> (32u - l) : 0u;
   return ok;
 }
 
@@ -227,14 +277,23 @@ __global__ void __launch_bounds__(kThreads) code_tables_kernel(const TableJob* _
     h += row[r];
   }
   for (uint32_t i = t; i < 132; i += kThreads) S.head[i] = 0;
-  const uint32_t n = (uint32_t)__syncthreads_count(h != 0);
-  const uint32_t n_sym = 256u - min_all(S, h ? 255u - t : 256u);
+  const uint64_t used = __ballot(h != 0);
+  if ((t & 63u) == 0) S.used[t >> 6] = used;
+  __syncthreads();
+  uint32_t n = 0, n_sym = 0, below = (uint32_t)__popcll(used & ((1ull << (t & 63u)) - 1ull));
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    const uint64_t m = S.used[w];
+    if (w < t >> 6) below += (uint32_t)__popcll(m);
+    n += (uint32_t)__popcll(m);
+    if (m) n_sym = 64 * w + 64 - (uint32_t)__builtin_clzll(m);
+  }
   uint8_t* const head = reinterpret_cast<uint8_t*>(S.head);
   bool ok = n != 0;
   uint32_t head_len = 0;
   if (ok && J.kind <= kTableIlv) {
     uint32_t rev;
-    const uint32_t l = huffman_length(S, h, n, J.kind == kTableIlv && n_sym <= 16 ? 6u : 11u);
+    const uint32_t l = huffman_length(S, h, below, n, J.kind == kTableIlv && n_sym <= 16 ? 6u : 11u);
     ok = canonical(S, l, rev);
     g_st<uint32_t>(reinterpret_cast<uint64_t>(codes + 256ull * j + t), l << 16 | rev);
     // weights header: 0x80 | count, or 0x80 and count (256 as 0), then the
