@@ -159,3 +159,24 @@ def test_first_states_of_one_among_many(kind, state):
             assert (got is None) == (want is None)
             if want is not None:
                 assert (got[:-1] == src).all() and got[-1].tobytes() == want
+
+
+@pytest.mark.parametrize("share", [31, 32, 33, 64, 65, 1000, 2047])
+def test_slots_of_frequent_symbols(share):
+    """Frequencies around the line (64 table entries) from which all lanes fill a symbol's slots, in both forms."""
+    counts = np.zeros(256, int)
+    counts[7] = counts[70] = share if 2 * share < 2048 else 1
+    counts[200] = 2048 - counts.sum()
+    src = np.repeat(np.arange(256, dtype=np.uint8), counts)
+    np.random.default_rng(share).shuffle(src)
+    pay = O.codec_encode(O.CODEC_RANS, src.tobytes())
+    assert pay[0] == 1
+    print(share, flush=True)
+    assert decode(pay, len(src)) == src.tobytes()
+    count = 4 * cus() + 1
+    tensors = [plan.TensorPlan(plan.CHAIN_PASSTHROUGH, 2048 * k, len(src), [
+        plan.PlanePlan(O.CODEC_RANS, 0, len(pay), len(src))]) for k in range(count)]
+    out = torch.zeros(2048 * count, dtype=torch.uint8, device="cuda:0")
+    api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL,
+                                              plan.encode_plan(tensors), device(np.frombuffer(pay, np.uint8)), out, 0)
+    assert (out.view(count, 2048).cpu().numpy() == src).all()
