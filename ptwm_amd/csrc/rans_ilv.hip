@@ -369,7 +369,7 @@ __global__ void __launch_bounds__(256) rilv_decode_kernel(const IlvTensor* __res
                                    ChainInfo<kChain>::xf[p]);
         __syncthreads();
       }
-      if (t == 0 && ctl.bad) status_or(&status[ti], ctl.bad);
+      if (t == 0 && ctl.bad && tile == tpre[j]) status_or(&status[ti], ctl.bad);  // as in ilv_decode_kernel
     }
     if (ctl.bad) continue;  // uniform: the tensor is rejected
     const uint32_t bi = kIlvBlocksPerTile * (tile - tpre[j]) + wave;
