@@ -114,6 +114,42 @@ def test_past_65536_blocks():
     assert getattr(e.value, "rc", None) == -1
 
 
+@pytest.mark.parametrize("codec", list(CODECS))
+@pytest.mark.parametrize("blocks", [8191, 8193])
+def test_many_blocks_without_sums(codec, blocks):
+    """Tensors with plane CRCs beside one without: in its launch up to 8192 of its blocks, else in one of their own."""
+    n = blocks * 16384 - 77
+    g = torch.Generator(device="cuda:0").manual_seed(blocks)
+    plain = torch.randint(100, 104, (n,), generator=g, device="cuda:0", dtype=torch.uint8)
+    items = [(6, data(6, 20_001, 1)), (6, data(6, 33_000, 2))]
+    src = [(6, dev(items[0][1])), (6, plain), (6, dev(items[1][1]))]
+    out = torch.zeros(n // 2, dtype=torch.uint8, device="cuda:0")
+    used, st = api.encode_tensors_cuda(src, out, 0, codec=codec)
+    tensors = plan.decode_plan(st)
+    for k in (0, 2):
+        tensors[k].planes[0].crc32 = O.crc32(items[k // 2][1])
+    plain_plan = plan.encode_plan([tensors[1]])
+    total = tensors[2].out_offset + tensors[2].out_len
+    for wrong in (False, True):
+        back = torch.zeros(total, dtype=torch.uint8, device="cuda:0")
+        if wrong:
+            tensors[2].planes[0].crc32 ^= 4
+        # has_crc is a tensor's own flag: each tensor encoded by itself, then joined
+        parts = [plan.encode_plan([tensors[0]]), plain_plan, plan.encode_plan([tensors[2]])]
+        joined = parts[0][:8] + (3).to_bytes(4, "little") + b"".join(p[12:] for p in parts)
+        print(codec, blocks, wrong, flush=True)
+        if wrong:
+            with pytest.raises(Exception) as e:
+                api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, joined,
+                                                          out[:used], back, 0)
+            assert getattr(e.value, "rc", None) == -1
+            continue
+        api.hardware_backend_dispatch_decode_cuda(ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL, joined,
+                                                  out[:used], back, 0)
+        for (_, s), t in zip(src, tensors):
+            assert torch.equal(back[t.out_offset:t.out_offset + t.out_len], s)
+
+
 @pytest.mark.parametrize("stored", [False, True])
 @pytest.mark.parametrize("codec", list(CODECS))
 @pytest.mark.parametrize("chain", [3, 4, 5])
