@@ -115,9 +115,10 @@ int64_t ptwm_hardware_backend_v1_dispatch_decode_cuda(uint8_t state_format_versi
  * stream or event creation (ptwm_mi355x_alloc_calls does not move across
  * it).  Returns -3 (MissingCapability) when the device's context does not
  * exist yet or its scratch could not be resolved.  Plans outside these
- * limits (more than PTWM_MI355X_NOALLOC_MAX_TENSORS tensors, or more than
- * PTWM_MI355X_NOALLOC_MAX_CRC_BLOCKS CRC-checked 16384-byte plane blocks in
- * all) return -5 (Unsupported).  Calls on one device are serialised by the
+ * limits (more than PTWM_MI355X_NOALLOC_MAX_TENSORS tensors, or huff_ilv
+ * tensors of more than PTWM_MI355X_NOALLOC_MAX_CRC_BLOCKS CRC-checked blocks of
+ * 16384 bytes a plane in all: a limit of this entry point, not of its scratch)
+ * return -5 (Unsupported).  Calls on one device are serialised by the
  * library; the array keeps the last call's contents (every call rewrites
  * what it reads), so calls that overlap on one device from outside the
  * library (another process) would race. */

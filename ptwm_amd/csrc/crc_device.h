@@ -1,6 +1,6 @@
 // crc_device.h -- CRC-32/ISO-HDLC building blocks shared by the CRC kernels
-// (integrity.hip) and the fused decode's CRC of the planes it restores
-// (huff_ilv.hip).  Reflected representation: bit 31 - i holds the x^i
+// (integrity.hip) and the fused decodes' CRCs of the planes they restore
+// (huff_ilv.hip, rans_ilv.hip).  Reflected representation: bit 31 - i holds the x^i
 // coefficient; a zero-initialised CRC register is linear in the data, and
 // advancing it over m zero bytes multiplies it by x^(8m) mod P.
 #pragma once
@@ -124,7 +124,7 @@ __device__ __forceinline__ uint32_t crc_piece(const uint32_t* T, uint32_t c, u32
 // bank conflicts, 20 VALU instructions and 4 MFMAs, and 4 reads and 20
 // instructions more that all planes share.  Measured on whole calls: four
 // bf16 layers (1.74 GB) 878 -> 750 us; the nibble and rans_ilv tensors, whose
-// CRCs were passes of their own before, e4m3 8192 x 8192 187 -> 67 us and
+// CRCs were passes of their own before, e4m3 8192 x 8192 186 -> 87 us and
 // fp32 4096 x 4096 153 -> 96 us.  The call waits for the device once (before:
 // again for each of the range and combine kernels and their uploads): one
 // norm weight 98 -> 43 us.

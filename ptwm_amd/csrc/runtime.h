@@ -42,7 +42,7 @@ struct PinnedBuffer {
 // all its device scratch lives in one fixed array per device (runtime.hip),
 // laid out as [CRC accumulators][tensor descriptors, launch indexes][CRC
 // tables][exact-route stubs], and its host staging in a fixed per-device host
-// area.
+// area.  The layout takes 1.3 MiB; the array's 16 MiB are the published size.
 constexpr uint64_t kNoAllocScratchBytes = 16ull << 20;
 constexpr uint64_t kNoAllocAccOff = 0, kNoAllocAccBytes = 128ull << 10;
 constexpr uint64_t kNoAllocArgsOff = kNoAllocAccOff + kNoAllocAccBytes, kNoAllocArgsBytes = 1ull << 20;
@@ -55,7 +55,9 @@ constexpr uint64_t kNoAllocHostBytes = 1ull << 20;
 constexpr uint64_t kNoAllocStatusBytes = 16ull << 10;
 constexpr uint64_t kNoAllocCrcOutBytes = (64ull << 10) + 256;
 static_assert(kNoAllocStatusBytes >= 4ull * 4096, "a status word for every tensor the allocation-free decode takes");
-// limits of a plan the allocation-free decode accepts
+// limits of a plan the allocation-free decode accepts: tensors by the areas
+// above; CRC-checked blocks of huff_ilv tensors by the entry point's published
+// contract only (a sum takes one word a plane, whatever its length)
 constexpr uint32_t kNoAllocMaxTensors = 4096;
 constexpr uint64_t kNoAllocMaxCrcBlocks = 883456;
 
@@ -172,8 +174,8 @@ int64_t execute_plan(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t ou
 
 // The same without allocating device or pinned memory: every tensor must
 // take the fused route (fused_eligible), carry no XXH64, have 4-byte aligned
-// coded payloads and fit the fixed scratch (kNoAllocMaxTensors,
-// kNoAllocMaxCrcBlocks); kUnsupported otherwise, kMissingCapability when the
+// coded payloads and keep to kNoAllocMaxTensors and kNoAllocMaxCrcBlocks;
+// kUnsupported otherwise, kMissingCapability when the
 // device's scratch address could not be resolved.
 int64_t execute_plan_noalloc(DevCtx& ctx, const Plan& plan, uint64_t in_dev, uint64_t out_dev);
 

@@ -134,8 +134,8 @@ __global__ void __launch_bounds__(256) merge_nibble_kernel(const uint8_t* __rest
 // and workgroup, copy lane % 16, symbols 17 words apart.  The split is bound by
 // HBM and the counting by LDS atomics, so most of the counting hides here (two
 // bf16 layers of 436 MB: 356 us for the split alone and 220 us for a pass of
-// its own over the planes).  One workgroup of 1024 threads per CU: each ends with
-// 512 atomics on the same words, which cost about 12 ns a workgroup (a 4096 x
+// its own over the planes).  One workgroup of 1024 threads per CU (256 of them,
+// the whole card): each ends with 512 atomics on the same words, which cost about 12 ns a workgroup (a 4096 x
 // 4096 tensor: 16.8 us with 256 workgroups, 20.0 with 512 of 512 threads, 26.5
 // with 1024 of them).
 constexpr uint32_t kSplitCopies = 16, kSplitStride = 17;
