@@ -390,15 +390,19 @@ int64_t ilv_decode_tensors(DevCtx& ctx, const std::vector<IlvTensor>& tensors_in
   // own, which the device starts some 25 us later (512 MiB of bf16 planes
   // beside one tensor with CRCs: huff_ilv 284 to 252 us, rans_ilv 434 to 334).
   constexpr uint64_t kPlainBlocks = 8192;
+  uint64_t chain_blocks[2][8][2] = {};  // by family, chain and whether without CRCs
+  for (const IlvTensor& T : tensors)
+    if (T.family <= kFamilyRans && T.chain < 8)
+      chain_blocks[T.family][T.chain][T.crc_ix == kIlvNoCrc] += (T.n + kIlvBlock - 1) / kIlvBlock;
   for (uint32_t fam = kFamilyHuff; fam <= kFamilyRans; ++fam)
   for (uint32_t chain : launch_codes(fam))
   for (const bool plain : {false, true}) {
-    uint64_t crc_blocks = 0, plain_blocks = 0;
-    for (const IlvTensor& T : tensors)
-      if (T.family == fam && ilv_code_has(chain, T.chain))
-        (T.crc_ix != kIlvNoCrc ? crc_blocks : plain_blocks) += (T.n + kIlvBlock - 1) / kIlvBlock;
-    const bool apart = crc_blocks && plain_blocks >= kPlainBlocks;
-    if (plain && !apart) continue;
+    uint64_t blocks[2] = {};
+    for (uint32_t c = 0; c < 8; ++c)
+      if (ilv_code_has(chain, c))
+        for (uint32_t k = 0; k < 2; ++k) blocks[k] += chain_blocks[fam][c][k];
+    const bool apart = blocks[0] && blocks[1] >= kPlainBlocks;
+    if (plain ? !apart : !(blocks[0] + blocks[1])) continue;
     std::vector<uint32_t> tix, tpre{0};
     uint32_t slots = 0;
     uint64_t est = 0, pool = 0, pool_skew = 0;
