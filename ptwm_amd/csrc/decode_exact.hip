@@ -1068,11 +1068,15 @@ hipError_t launch_tans_decode(const DecodeJob* jobs_dev, uint32_t* status_dev, u
 // share a SIMD.  So the line lies where the first would need a second round.  A
 // plane in 256 KiB chunks, ms in the first and in the second form: 256 chunks
 // 3.5 and 4.5, 1024 chunks 5.4 and 7.0, 1536 chunks 10.6 and 4.5, 6144 chunks
-// 32 and 17.5 (256 CUs).
+// 32 and 17.5 (256 CUs).  Beside jobs of other codecs, whose kernels run on
+// the other stream and take LDS too, the second round comes earlier: an fp32
+// tensor with three Huffman planes and one rANS plane of 512 chunks 5.7 and
+// 6.4, 640 chunks 6.7 and 6.6, 768 chunks 10.0 and 6.2, 1024 chunks 11.7 and
+// 5.5.
 hipError_t launch_rans_exact(const DecodeJob* jobs_dev, uint32_t* status_dev, uint32_t n_jobs, uint32_t n_rans,
                              uint32_t cu_count, uint64_t* copy_src, hipStream_t stream) {
   if (n_jobs == 0) return hipSuccess;
-  if (n_rans <= 4 * cu_count)
+  if (n_rans <= (n_rans == n_jobs ? 4 : 2) * cu_count)
     hipLaunchKernelGGL((decode_exact_kernel<true, true>), dim3(n_jobs), dim3(64), 0, stream, jobs_dev, status_dev,
                        nullptr, nullptr, copy_src);
   else

@@ -125,6 +125,27 @@ def test_decode_chunk_counts(extra):
     assert out.cpu().numpy().tobytes() == plane.tobytes()
 
 
+@pytest.mark.parametrize("extra", [0, 1])
+def test_decode_chunk_counts_beside_huffman(extra):
+    """The line for calls that hold other jobs too: two chunks per CU."""
+    chunks, size = 2 * cus() + extra, 1283
+    planes = [np.concatenate([symbols(k, size, 3 * c) for c in range(chunks)])[:-9] for k in ("geometric", "rare")]
+    n, blob, pp = len(planes[0]), b"", []
+    for codec, plane in zip((O.CODEC_HUFFMAN, O.CODEC_RANS), planes):
+        blob += b"\0" * (-len(blob) % 16)
+        payload, entries = O.encode_plane_chunked(codec, plane.tobytes(), size)
+        pp.append(plan.PlanePlan(codec, len(blob), len(payload), n, [tuple(map(int, e)) for e in entries]))
+        blob += payload
+    want = O.chain_inverse(O.CHAIN_IEEE16_SPLIT2, [p.tobytes() for p in planes])
+    out = torch.zeros(2 * n, dtype=torch.uint8, device="cuda:0")
+    print(chunks, flush=True)
+    api.hardware_backend_dispatch_decode_cuda(
+        ids.HARDWARE_BACKEND_LABEL, ids.DECODE_PLAN_LABEL,
+        plan.encode_plan([plan.TensorPlan(plan.CHAIN_IEEE16_SPLIT2, 0, 2 * n, pp)]),
+        device(np.frombuffer(blob, np.uint8)), out, 0)
+    assert out.cpu().numpy().tobytes() == want
+
+
 @pytest.mark.parametrize("state", [0, (1 << 23) - 1, 1 << 23, (1 << 31) - 1, 1 << 31, (1 << 32) - 1])
 @pytest.mark.parametrize("kind", ["one", "rare", "geometric"])
 def test_first_states_of_one_among_many(kind, state):
