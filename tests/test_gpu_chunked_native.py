@@ -6,9 +6,9 @@ with the plane's chunk table of (offset, decoded size)); the container reads
 them per chunk (container.rs:1975-2050).  Each chunk payload here is this
 library's own encoder output for that chunk's bytes; the plan decodes the
 tensor bit-exactly through the fused route (chunk boundaries on 16384-symbol
-blocks, same across planes: one sub-tensor per chunk, CRC partials
-contiguous) or through plane scratch (other boundaries), and rejects a
-native chunk that carries state.
+blocks, same across planes: one sub-tensor per chunk, each block's CRC
+weighted by its place in the plane) or through plane scratch (other
+boundaries), and rejects a native chunk that carries state.
 """
 import sys
 import time

@@ -43,6 +43,7 @@ def planes():
         "nibble ties": spread([100, 100, 100, 1, 1, 1, 1, 1, 1], 10),
         "long tail": spread([60000] + [1] * 255, 11),
         "rounding": spread([1000 // (k + 1) for k in range(200)], 12),
+        "refused": spread([353] * 56 + [1] * 200, 14),
     }
     rng = np.random.default_rng(13)
     for k in range(20):

@@ -1,13 +1,13 @@
-"""Plane CRC-32 computed inside the fused huff_ilv decode (whole 16 KiB
-blocks of each plane folded while the planes are merged, the partial last
-block from the restored tensor, then combined), checked the way the
+"""Plane CRC-32 computed inside the fused decodes (16 KiB blocks of each
+plane while the planes are merged, the last one padded with zeros, each
+block's sum weighted by its place), checked the way the
 reference checks a decoded plane (container.rs:2154-2159: crc32fast of the
 plane bytes, a mismatch is InvalidContainer):
 
 - one plan mixing chains (bf16 split2, fp32 split4, passthrough), plane
   lengths that are exact multiples of the block, under one block, one
-  element, and ragged; tensors with and without CRCs; rans_ilv tensors
-  (standalone CRC kernel) in the same plan;
+  element, and ragged; tensors with and without CRCs; rans_ilv tensors in
+  the same plan;
 - every plane's expected CRC is the oracle's CRC-32 of the oracle's plane
   bytes, so a dropped block, a wrong advance or a wrong byte rotation of
   the exponent plane fails the decode;
@@ -111,13 +111,13 @@ def test_fused_crc_plan_verifies_and_detects_each_plane():
                 _decode(plan.encode_plan(tensors), blob_dev, out)
             assert getattr(ei.value, "rc", None) == -1, (ti, pi)
             p.crc32 ^= 1 << (pi + ti) % 32
-    # and the restored plan still verifies afterwards (partials rewritten)
+    # and the restored plan still verifies afterwards (the sums start from zero)
     assert _decode(plan.encode_plan(tensors), blob_dev, out) == written
 
 
 def test_fused_crc_llama_like_tensor_repeated():
     """A 16 Mi-element bf16 tensor (1024 blocks per plane), decoded twice in
-    a row with CRCs: the second call's partials overwrite the first's."""
+    a row with CRCs: the second call's sums start from zero."""
     g = torch.Generator(device="cuda:0").manual_seed(5)
     x = (torch.randn(1 << 24, generator=g, device="cuda:0") * 0.02).to(torch.bfloat16).view(torch.uint8)
     blob, tp = _encode([(plan.CHAIN_IEEE16_SPLIT2, x)], "huff_ilv")
